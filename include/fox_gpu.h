@@ -343,6 +343,48 @@ fox_gpu_status fox_gpu_argmax(fox_gpu_ctx *ctx, const float *logits, size_t n,
                               uint32_t *idx, uint32_t *pos, uint32_t advance,
                               uint32_t *history);
 
+/* ---------------------------------------------------- batched passes */
+
+/* The stages of a layer over many tokens at once (a prompt: src/forward.c
+ * takes n_batch tokens per pass): up to FOX_GPU_BATCH_TOKENS tokens, results
+ * bit-identical to the calls above in passes of FOX_GPU_MAX_TOKENS.  Weights
+ * are read once per pass and multiplied on the matrix cores; scratch comes
+ * from the context's workspace.  Strides are always used (also for one
+ * token).
+ *
+ * fox_gpu_batch_gemv: y_i = W_i x for n matrices of one type and width.
+ * fox_gpu_batch_gemv_rmsnorm / _gate_up_silu: as fox_gpu_gemv_rmsnorm and
+ * fox_gpu_gate_up_silu; block types up to 32768 columns with 16-byte aligned
+ * inputs, other cases return FOX_GPU_ERR_UNSUPPORTED (use fox_gpu_rmsnorm,
+ * fox_gpu_batch_gemv and fox_gpu_silu_mul).
+ * fox_gpu_batch_attention: exact mode only (the reference's order). */
+#define FOX_GPU_BATCH_TOKENS 1024
+fox_gpu_status fox_gpu_batch_gemv(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor *const *ws,
+                                  const float *x, size_t x_stride, size_t M,
+                                  float *const *outs, const size_t *out_strides,
+                                  unsigned flags);
+fox_gpu_status fox_gpu_batch_gemv_rmsnorm(fox_gpu_ctx *ctx, size_t n,
+                                          const fox_gpu_tensor *const *ws, const float *x,
+                                          size_t x_stride, size_t M, const float *norm_w,
+                                          float eps, float *const *outs,
+                                          const size_t *out_strides, unsigned flags);
+fox_gpu_status fox_gpu_batch_gate_up_silu(fox_gpu_ctx *ctx, const fox_gpu_tensor *w_gate,
+                                          const fox_gpu_tensor *w_up, const float *x,
+                                          size_t x_stride, size_t M, const float *norm_w,
+                                          float eps, float *h_out, size_t h_stride);
+fox_gpu_status fox_gpu_batch_rope_store(fox_gpu_ctx *ctx, float *q, size_t q_stride,
+                                        float *k, size_t k_stride,
+                                        const float *v, size_t v_stride,
+                                        size_t n_head, size_t n_head_kv, size_t head_dim,
+                                        size_t M, const float *cos_t, const float *sin_t,
+                                        const uint32_t *pos, size_t n_ctx,
+                                        float *k_cache, float *v_cache);
+fox_gpu_status fox_gpu_batch_attention(fox_gpu_ctx *ctx, float *out, size_t out_stride,
+                                       const float *q, size_t q_stride, const float *k_cache,
+                                       const float *v_cache, size_t n_head, size_t n_head_kv,
+                                       size_t head_dim, size_t M, const uint32_t *pos,
+                                       size_t n_ctx);
+
 /* ------------------------------------------------------------- graphs */
 
 /* Record the work queued on the context's stream between begin and end into

@@ -26,6 +26,7 @@ ACT_PER_VECTOR, ACT_PER_BLOCK = 0, 1
 GEMV_ACCUMULATE = 1
 ATTN_SPLIT, ATTN_EXACT = 0, 1
 MAX_TOKENS = 8
+BATCH_TOKENS = 1024
 
 STATUS = ["OK", "ERR_ARG", "ERR_IO", "ERR_NOMEM", "ERR_FORMAT", "ERR_UNSUPPORTED",
           "ERR_NOTFOUND", "ERR_INTERNAL"]
@@ -109,6 +110,14 @@ def gpu_lib() -> C.CDLL:
         "fox_gpu_qkv_rope": [vp, vp, vp, vp, vp, sz, sz, vp, C.c_float, vp, sz, vp, vp, vp, sz,
                              vp, vp, sz],
         "fox_gpu_gate_up_silu": [vp, vp, vp, vp, sz, sz, vp, C.c_float, vp, sz],
+        "fox_gpu_batch_gemv": [vp, sz, C.POINTER(vp), vp, sz, sz, C.POINTER(vp), C.POINTER(sz),
+                               C.c_uint],
+        "fox_gpu_batch_gemv_rmsnorm": [vp, sz, C.POINTER(vp), vp, sz, sz, vp, C.c_float,
+                                       C.POINTER(vp), C.POINTER(sz), C.c_uint],
+        "fox_gpu_batch_gate_up_silu": [vp, vp, vp, vp, sz, sz, vp, C.c_float, vp, sz],
+        "fox_gpu_batch_rope_store": [vp, vp, sz, vp, sz, vp, sz, sz, sz, sz, sz, vp, vp, vp, sz,
+                                     vp, vp],
+        "fox_gpu_batch_attention": [vp, vp, sz, vp, sz, vp, vp, sz, sz, sz, sz, vp, sz],
         "fox_gpu_silu_mul": [vp, vp, vp, sz, sz, sz],
         "fox_gpu_add": [vp, vp, vp, sz, sz, sz],
         "fox_gpu_argmax": [vp, vp, sz, vp, vp, C.c_uint32, vp],
@@ -372,6 +381,28 @@ class Gpu:
         _check(self.lib.fox_gpu_attention(self.ctx, out.ptr, out_stride or w, q.ptr,
                                           q_stride or w, kc.ptr, vc.ptr, n_head, n_head_kv,
                                           head_dim, M, pos.ptr, n_ctx, mode))
+
+    # -- batched passes (up to BATCH_TOKENS tokens)
+    def batch_gemv(self, ws, x: DeviceArray, M, outs, norm: DeviceArray = None, eps=0.0, flags=0):
+        n = len(ws)
+        hs = (C.c_void_p * n)(*[w.h for w in ws])
+        os_ = (C.c_void_p * n)(*[o.ptr for o in outs])
+        st = (C.c_size_t * n)(*[w.ne1 for w in ws])
+        if norm is None:
+            _check(self.lib.fox_gpu_batch_gemv(self.ctx, n, hs, x.ptr, ws[0].ne0, M, os_, st, flags))
+        else:
+            _check(self.lib.fox_gpu_batch_gemv_rmsnorm(self.ctx, n, hs, x.ptr, ws[0].ne0, M,
+                                                       norm.ptr, eps, os_, st, flags))
+
+    def batch_gate_up_silu(self, wg, wu, x: DeviceArray, M, norm: DeviceArray, eps, h: DeviceArray):
+        _check(self.lib.fox_gpu_batch_gate_up_silu(self.ctx, wg.h, wu.h, x.ptr, wg.ne0, M, norm.ptr,
+                                                   eps, h.ptr, wg.ne1))
+
+    def batch_attention(self, out: DeviceArray, q: DeviceArray, kc: DeviceArray, vc: DeviceArray,
+                        n_head, n_head_kv, hd, M, pos: DeviceArray, n_ctx):
+        _check(self.lib.fox_gpu_batch_attention(self.ctx, out.ptr, n_head * hd, q.ptr, n_head * hd,
+                                                kc.ptr, vc.ptr, n_head, n_head_kv, hd, M, pos.ptr,
+                                                n_ctx))
 
     def event(self):
         e = C.c_void_p()

@@ -1,0 +1,867 @@
+// fox_batch.hip -- projections of a batched pass (a prompt's tokens, more
+// than the FOX_GPU_MAX_TOKENS of the decode kernels), bit-identical to them.
+//
+// batch_prep quantises the tokens once (optionally RMS-normalised first), a
+// workgroup per token, and batch_gemm is an int8 MFMA matrix product over
+// the 256-element weight blocks:
+//   * the activations are the MFMA's A operand (16 tokens), the weight rows
+//     its B operand (16 rows), so lane (j, g) holds row j's sums of tokens
+//     4g .. 4g + 3: a lane needs the scales of one row only;
+//   * a wave owns its rows' whole K range and adds each block's float term
+//     as the block is done, in block order from 0.0f, which is the
+//     reference's row loop (src/ternary.c:226-246, src/kernels.c:571-661):
+//     no terms go through memory;
+//   * the integer sums start from the bits of 1.5 * 2^23 (MAGIC), so an
+//     accumulator's bits are the float 12582912 + S exactly (|S| < 2^22), and
+//     fma(d, that, -12582912 d) is d * S rounded once (12582912 d is exact:
+//     d has at most 17 significant bits), the reference's d * (float)S, one
+//     instruction in place of a conversion and a product.  A row whose d is
+//     infinite or NaN takes the conversion (wave-uniform test).
+//
+// The pass over a 1024-token prompt is bound by the matrix cores and the
+// vector unit about equally on ternary weights (four MFMAs, 64 clocks,
+// against 8 vector instructions per 16 x 16 x 256 tile and the split of the
+// codes, 28 shared by the wave's token tiles) and by the vector unit on the
+// K-quants (5 instructions per 32-element sub-block and output for Q4_K).
+// Measured: two 4B-class layers over a 1024-token prompt 22.0 ms in passes of
+// eight, 1.32 ms batched; two 8B-class layers over 77 tokens on 1024 cached
+// rows 7.24 -> 1.02 ms.  A 1024-token gate/up (2 x 9728 x 2560, ternary) takes
+// 100 us, a 77-token one of the 8B class (Q4_K, 2 x 14336 x 4096) 77 us.
+#include "fox_gemv_dev.h"
+#include "fox_math.h"
+
+#include <cstring>
+#include <type_traits>
+
+#define BT_THREADS 256
+#define MAGIC_BITS 0x4B400000           // 12582912.0f = 1.5 * 2^23
+#define MAGIC_F 12582912.0f
+#define B_ROW 272                       // LDS bytes of one token's block (256 and a 16-byte pad)
+
+// 16-byte quads of per-token values per (16-token tile, block): TQ2_0 the
+// negated block sums (plus MAGIC_BITS), Q4_K eight sub-block sums and the
+// block scale as floats, Q6_K the block scale
+__host__ __device__ constexpr int aux_quads(int fmt)
+{
+    return fmt == FMT_Q4K ? 36 : 4;
+}
+
+// ------------------------------------------------------------------ prep
+
+// where lane dl's dword (elements 4 dl .. 4 dl + 3 of a block) goes in the
+// token's 256 bytes: 16-byte piece (step, g) is what lane group g feeds to
+// MFMA step `step` (mirroring the weight decodes below)
+template <int FMT>
+__device__ __forceinline__ int piece_off(int dl)
+{
+    const int e0 = 4 * dl;
+    if (FMT == FMT_TQ2) {
+        const int half = e0 >> 7, l = (e0 >> 5) & 3, o = e0 & 31;
+        const int g = 2 * half + (o >> 4), u = (o & 15) >> 2;
+        return (u * 4 + g) * 16 + l * 4;
+    } else if (FMT == FMT_Q4K) {
+        // sub-blocks 2p and 2p + 1 side by side, eight elements of each
+        const int s = e0 >> 5, o = e0 & 31;
+        return ((s >> 1) * 4 + (o >> 3)) * 16 + (s & 1) * 8 + (o & 4);
+    } else {
+        // quarter v = 2 half + s, sub-group c: elements 128 half + 32 c + 16 s
+        const int h = e0 >> 7, c = (e0 >> 5) & 3, s = (e0 >> 4) & 1;
+        return ((2 * h + s) * 4 + c) * 16 + (e0 & 15);
+    }
+}
+
+// one dword of four quantised values, and the scale: the reference's
+// per-element rule for an amax whose bits are am (the largest |x| bit
+// pattern: NaN above inf) and m, the largest |x| that is not NaN
+struct Quant {
+    float inv, act;
+    int mode;                  // 0 zeros, 1 quant_fast, 2 quant_one
+};
+__device__ __forceinline__ Quant quant_of(uint32_t am, float m)
+{
+    Quant q;
+    if (am >= 0x03800000u && am < 0x7f800000u) {
+        const float amax = __uint_as_float(am);
+        q.inv = fox_div(127.0f, amax);
+        q.act = fox_div(amax, 127.0f);
+        q.mode = 1;
+    } else if (m > 0.0f) {
+        q.inv = fox_div(127.0f, m);
+        q.act = fox_div(m, 127.0f);
+        q.mode = 2;
+    } else {
+        q.inv = q.act = 0.0f;
+        q.mode = 0;
+    }
+    return q;
+}
+
+__device__ __forceinline__ uint32_t quant4(const Quant &q, const float4 &x)
+{
+    if (q.mode == 1)
+        return pack_lo_bytes(quant_fast(x.x, q.inv), quant_fast(x.y, q.inv),
+                             quant_fast(x.z, q.inv), quant_fast(x.w, q.inv));
+    if (q.mode == 2)
+        return pack_lo_bytes(quant_one(x.x, q.inv), quant_one(x.y, q.inv), quant_one(x.z, q.inv),
+                             quant_one(x.w, q.inv));
+    return 0u;
+}
+
+__device__ __forceinline__ uint32_t abs_bits4(const float4 &x)
+{
+    const uint32_t a = max(__float_as_uint(x.x) & 0x7fffffffu, __float_as_uint(x.y) & 0x7fffffffu);
+    const uint32_t b = max(__float_as_uint(x.z) & 0x7fffffffu, __float_as_uint(x.w) & 0x7fffffffu);
+    return max(a, b);
+}
+
+// the largest |x| that is not NaN (src/gemv.c:20-23: `a > amax` from 0)
+__device__ __forceinline__ float abs_max4(const float4 &x)
+{
+    const float v[4] = {fabsf(x.x), fabsf(x.y), fabsf(x.z), fabsf(x.w)};
+    float m = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; e++) m = v[e] > m ? v[e] : m;
+    return m;
+}
+
+__device__ __forceinline__ uint32_t wave_max_u(uint32_t v)
+{
+    return wave_reduce(v, 0u, [](uint32_t x, uint32_t y) { return x > y ? x : y; });
+}
+
+// Token blockIdx.x: RMSNorm (NORM; src/ops.c:7-22), int8 quantisation and the
+// block sums.  512 threads; thread tid holds dwords tid + 512 r, so a wave
+// holds whole blocks (block wave + 8 r).  q: [token][K] bytes, each block's
+// 256 in piece_off order; aux: [token / 16][block][aux_quads][token % 16].
+template <int FMT, bool NORM, int R>
+__global__ __launch_bounds__(512) void batch_prep(const float *__restrict__ x,
+                                                  const float *__restrict__ norm_w, int K,
+                                                  size_t x_stride, float eps,
+                                                  uint8_t *__restrict__ q,
+                                                  uint32_t *__restrict__ aux,
+                                                  float *__restrict__ scale)
+{
+    __shared__ double dred[8];
+    __shared__ uint32_t ured[8];
+    const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nb = K >> 8, nd = K >> 2;
+    const float *xt = x + (size_t)t * x_stride;
+    const float4 *x4 = (const float4 *)xt, *w4 = (const float4 *)norm_w;
+    float4 xv[R], wv[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int m = min(tid + 512 * r, nd - 1);
+        xv[r] = x4[m];
+        if (NORM) wv[r] = w4[m];
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++)
+        if (tid + 512 * r >= nd) xv[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (NORM) {
+        double ss = 0.0;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const double x0 = xv[r].x, x1 = xv[r].y, x2 = xv[r].z, x3 = xv[r].w;
+            ss = __builtin_fma(x0, x0, ss);
+            ss = __builtin_fma(x1, x1, ss);
+            ss = __builtin_fma(x2, x2, ss);
+            ss = __builtin_fma(x3, x3, ss);
+        }
+        ss = wave_reduce(ss, 0.0, [](double a, double b) { return a + b; });
+        if (lane == 0) dred[wave] = ss;
+        __syncthreads();
+        double tot = 0.0;
+        for (int w = 0; w < 8; w++) tot += dred[w];
+        // the scale from both ends of the interval that holds the
+        // index-order sum (fox_fused.hip, rms_apply); undecided: that sum
+        const double rel = (double)(K + 64) * 0x1p-52;
+        const double sgn = (lane & 1) ? 1.0 : -1.0;
+        const double y = 1.0 / __builtin_sqrt(tot * (1.0 + sgn * rel) / (double)K + (double)eps) *
+                         (1.0 - sgn * 0x1p-50);
+        const float f = (float)y;
+        float rs = read_lane(f, 0);
+        if (rs != read_lane(f, 1)) {
+            double seq = 0.0;
+            for (int i = 0; i < K; i++) seq += (double)xt[i] * (double)xt[i];
+            rs = (float)(1.0 / __builtin_sqrt(seq / (double)K + (double)eps));
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            xv[r].x = xv[r].x * rs * wv[r].x;
+            xv[r].y = xv[r].y * rs * wv[r].y;
+            xv[r].z = xv[r].z * rs * wv[r].z;
+            xv[r].w = xv[r].w * rs * wv[r].w;
+            // (dwords past the end: 0 * rs * w may be NaN)
+            if (tid + 512 * r >= nd) xv[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
+    }
+    Quant qv;
+    if (FMT == FMT_TQ2) {
+        uint32_t am = 0;
+#pragma unroll
+        for (int r = 0; r < R; r++) am = max(am, abs_bits4(xv[r]));
+        am = wave_max_u(am);
+        if (lane == 0) ured[wave] = am;
+        __syncthreads();
+        am = 0;
+        for (int w = 0; w < 8; w++) am = max(am, ured[w]);
+        float m = 0.0f;
+        if (am >= 0x7f800000u || am < 0x03800000u) {        // (uniform over the workgroup)
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const float v = abs_max4(xv[r]);
+                m = v > m ? v : m;
+            }
+            m = wave_max(m);
+            __syncthreads();
+            if (lane == 0) ured[wave] = __float_as_uint(m);
+            __syncthreads();
+            m = 0.0f;
+            for (int w = 0; w < 8; w++) m = fmaxf(m, __uint_as_float(ured[w]));
+        }
+        qv = quant_of(am, m);
+        if (tid == 0) scale[t] = qv.act;
+    }
+    const int po = piece_off<FMT>(lane);
+    uint8_t *qt = q + (size_t)t * K;
+    uint32_t *at = aux + ((size_t)(t >> 4) * nb) * (aux_quads(FMT) * 4) + (t & 15);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int b = wave + 8 * r;
+        if (b >= nb) break;                                 // (uniform)
+        if (FMT != FMT_TQ2) {
+            // one scale per block (src/kernels.c:722-754)
+            const uint32_t am = wave_max_u(abs_bits4(xv[r]));
+            const float m = am >= 0x7f800000u || am < 0x03800000u ? wave_max(abs_max4(xv[r])) : 0.0f;
+            qv = quant_of(am, m);
+        }
+        const uint32_t qd = quant4(qv, xv[r]);
+        *(uint32_t *)(qt + (size_t)b * 256 + po) = qd;
+        uint32_t *ab = at + (size_t)b * (aux_quads(FMT) * 4);
+        if (FMT == FMT_TQ2) {
+            const int s = wave_sum_i(__builtin_amdgcn_sdot4((int)qd, 0x01010101, 0, false));
+            if (lane == 0) ab[0] = (uint32_t)(MAGIC_BITS - s);
+        } else {
+            if (FMT == FMT_Q4K) {
+                int s = __builtin_amdgcn_sdot4((int)qd, 0x01010101, 0, false);
+                s += dpp_t<0xB1, 0xF>(0, s);
+                s += dpp_t<0x4E, 0xF>(0, s);
+                s += dpp_t<0x141, 0xF>(0, s);               // sums of 8 lanes: 32 elements
+                if ((lane & 7) == 0) ab[(lane >> 3) * 16] = __float_as_uint((float)s);
+            }
+            if (lane == 0) ab[(aux_quads(FMT) * 4) - 16] = __float_as_uint(qv.act);
+        }
+    }
+}
+
+// ------------------------------------------------------------------ GEMM
+
+struct BatchArgs {
+    const uint8_t *w[MAX_SEGS];
+    float *out[MAX_SEGS];
+    size_t out_stride[MAX_SEGS];
+    int n_rows[MAX_SEGS];
+    int tile_start[MAX_SEGS + 1];
+    int nseg, nb, M, n_tg, n_wg;
+    unsigned flags;
+    const uint8_t *q;
+    const uint32_t *aux;
+    const float *scale;
+};
+
+enum { BE_STORE = 0, BE_SILU = 1 };
+
+// blocks per stage: as many as keep a stage's loads at four 16-byte pieces
+// per thread (few tokens), fewer for the K-quants, whose raw blocks take
+// more registers
+__host__ __device__ constexpr int stage_blocks(int fmt, int C)
+{
+    return C >= 3 ? 1 : fmt == FMT_TQ2 ? 4 / C : fmt == FMT_Q4K ? 2 / C : 1;
+}
+
+__host__ __device__ constexpr int batch_chunk(int fmt)
+{
+    return fmt == FMT_TQ2 ? TQ2_CHUNK : fmt == FMT_Q4K ? Q4K_CHUNK : Q6K_CHUNK;
+}
+
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+
+// a lane's bytes of one weight block (row j of a 16-row tile, group g)
+template <int FMT>
+struct RawBlock;
+template <>
+struct RawBlock<FMT_TQ2> {
+    u4v qs;
+    uint32_t d;
+    __device__ __forceinline__ void load(const uint8_t *ch, int lane)
+    {
+        qs = *(const u4v *)(ch + 16 * lane);
+        d = *(const unsigned short *)(ch + 1024 + 2 * (lane & 15));
+    }
+};
+template <>
+struct RawBlock<FMT_Q4K> {
+    u4v q0, q1, h;
+    __device__ __forceinline__ void load(const uint8_t *ch, int lane)
+    {
+        q0 = *(const u4v *)(ch + 32 * lane);
+        q1 = *(const u4v *)(ch + 32 * lane + 16);
+        h = *(const u4v *)(ch + 2048 + 16 * (lane & 15));
+    }
+};
+template <>
+struct RawBlock<FMT_Q6K> {
+    u4v l[4], hq[4], sc;
+    uint32_t d;
+    __device__ __forceinline__ void load(const uint8_t *ch, int lane)
+    {
+        const int i = lane & 15, g = lane >> 4;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int h = v >> 1, s = v & 1;
+            l[v] = *(const u4v *)(ch + 128 * i + 64 * h + 32 * (g & 1) + 16 * s);
+            hq[v] = *(const u4v *)(ch + 2048 + 64 * i + 32 * h + 16 * s);
+        }
+        sc = *(const u4v *)(ch + 3072 + 16 * i);
+        d = *(const unsigned short *)(ch + 3328 + 2 * i);
+    }
+};
+
+__device__ __forceinline__ v4i mfma64(v4i a, v4i b, v4i c)
+{
+    return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
+}
+
+// any lane's value infinite or NaN (wave-uniform)
+__device__ __forceinline__ bool any_nonfinite(float d)
+{
+    return __builtin_amdgcn_ballot_w64(!(fabsf(d) < INFINITY)) != 0;
+}
+
+// One block of R row tiles against C token tiles, its float terms added to
+// acc.  bl: the block's token rows in LDS (tile c at bl + c * 16 * B_ROW),
+// ax: its aux (tile c at ax + c * aux_quads quads).
+template <int FMT, int R, int C>
+__device__ __forceinline__ void block_terms(const RawBlock<FMT> (&raw)[R], const uint8_t *bl,
+                                            const u4v *ax, int lane, f4v (&acc)[R][C])
+{
+    const int j = lane & 15, g = lane >> 4;
+    const uint8_t *bt = bl + j * B_ROW + g * 16;
+    if constexpr (FMT == FMT_TQ2) {
+        v4i D[R][C], corr[C];
+#pragma unroll
+        for (int c = 0; c < C; c++) corr[c] = ((const v4i *)ax)[c * 4 + g];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            v4i w[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const uint32_t d = raw[r].qs[u];
+                w[r] = v4i{(int)(d & 0x03030303u), (int)((d >> 2) & 0x03030303u),
+                           (int)((d >> 4) & 0x03030303u), (int)((d >> 6) & 0x03030303u)};
+            }
+#pragma unroll
+            for (int c = 0; c < C; c++) {
+                const v4i a = *(const v4i *)(bt + c * 16 * B_ROW + u * 64);
+#pragma unroll
+                for (int r = 0; r < R; r++) D[r][c] = mfma64(a, w[r], u == 0 ? corr[c] : D[r][c]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const float d = half_bits_to_float(raw[r].d);
+            if (!any_nonfinite(d)) {
+                const float nd = -MAGIC_F * d;
+#pragma unroll
+                for (int c = 0; c < C; c++)
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        acc[r][c][k] = acc[r][c][k] + __builtin_fmaf(d, __int_as_float(D[r][c][k]), nd);
+            } else {
+#pragma unroll
+                for (int c = 0; c < C; c++)
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        acc[r][c][k] = acc[r][c][k] + d * (float)(D[r][c][k] - MAGIC_BITS);
+            }
+        }
+    } else if constexpr (FMT == FMT_Q4K) {
+        // d * sc and dmin * mn of the row's eight sub-blocks (exact: 11 + 6
+        // bits), src/kernels.c:246-255, 585-599
+        float A[R][8], B[R][8];
+        bool odd = false;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const uint32_t s0 = raw[r].h[1], s1 = raw[r].h[2], s2 = raw[r].h[3];
+            const uint32_t sc[2] = {s0 & 0x3f3f3f3fu,
+                                    (s2 & 0x0f0f0f0fu) | (((s0 >> 6) & 0x03030303u) << 4)};
+            const uint32_t mn[2] = {s1 & 0x3f3f3f3fu,
+                                    ((s2 >> 4) & 0x0f0f0f0fu) | (((s1 >> 6) & 0x03030303u) << 4)};
+            const float d = half_bits_to_float(raw[r].h[0] & 0xffffu);
+            const float dmin = half_bits_to_float(raw[r].h[0] >> 16);
+            odd = odd || any_nonfinite(d);
+#pragma unroll
+            for (int s = 0; s < 8; s++) {
+                A[r][s] = d * (float)((sc[s >> 2] >> (8 * (s & 3))) & 0xffu);
+                B[r][s] = dmin * (float)((mn[s >> 2] >> (8 * (s & 3))) & 0xffu);
+            }
+        }
+        const v4i magic = {MAGIC_BITS, MAGIC_BITS, MAGIC_BITS, MAGIC_BITS};
+        auto run = [&](auto finite) __attribute__((always_inline)) {
+#pragma unroll
+            for (int p = 0; p < 4; p++) {
+                long wl[R], wh[R];
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const uint32_t a0 = p < 2 ? raw[r].q0[2 * p] : raw[r].q1[2 * p - 4];
+                    const uint32_t a1 = p < 2 ? raw[r].q0[2 * p + 1] : raw[r].q1[2 * p - 3];
+                    wl[r] = (long)((uint64_t)(a0 & 0x0f0f0f0fu) | (uint64_t)(a1 & 0x0f0f0f0fu) << 32);
+                    wh[r] = (long)((uint64_t)((a0 >> 4) & 0x0f0f0f0fu) |
+                                   (uint64_t)((a1 >> 4) & 0x0f0f0f0fu) << 32);
+                }
+#pragma unroll
+                for (int c = 0; c < C; c++) {
+                    typedef long l2v __attribute__((ext_vector_type(2)));
+                    const l2v a = *(const l2v *)(bt + c * 16 * B_ROW + p * 64);
+                    const f4v as = ((const f4v *)ax)[c * 36 + 32 + g];
+#pragma unroll
+                    for (int hh = 0; hh < 2; hh++) {
+                        const int s = 2 * p + hh;
+                        const f4v sq = ((const f4v *)ax)[c * 36 + 4 * s + g];
+#pragma unroll
+                        for (int r = 0; r < R; r++) {
+                            const v4i D = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+                                a[hh], hh ? wh[r] : wl[r], magic, 0, 0, 0);
+                            const float na = -MAGIC_F * A[r][s];
+#pragma unroll
+                            for (int k = 0; k < 4; k++) {
+                                const float pr =
+                                    decltype(finite)::value
+                                        ? __builtin_fmaf(A[r][s], __int_as_float(D[k]), na)
+                                        : A[r][s] * (float)(D[k] - MAGIC_BITS);
+                                const float tv = pr - B[r][s] * sq[k];
+                                acc[r][c][k] = acc[r][c][k] + as[k] * tv;
+                            }
+                        }
+                    }
+                }
+            }
+        };
+        if (!odd) run(std::true_type{});
+        else run(std::false_type{});
+    } else {
+        // Q6_K: quarter v's four 16-element sub-groups are the four lane
+        // groups' bytes; sub-group c alone is the product with the other
+        // lane groups' weights zeroed.  Values q - 32 as signed bytes, times
+        // four (the 6-bit value with its top bit flipped, shifted up), the
+        // factor taken out of the integer sum.
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int h = v >> 1, s = v & 1;
+            v4i w[R][4];
+            int sc[R][4];
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                v4i a;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const uint32_t L = raw[r].l[v][i], H = raw[r].hq[v][i];
+                    const uint32_t lo = ((g < 2 ? L : L >> 4) & 0x0f0f0f0fu) << 2;
+                    const uint32_t hi = ((H >> (2 * g)) & 0x03030303u) << 6;
+                    a[i] = (int)((lo | hi) ^ 0x80808080u);
+                }
+#pragma unroll
+                for (int c4 = 0; c4 < 4; c4++) {
+                    const int m = g == c4 ? -1 : 0;
+                    w[r][c4] = v4i{a[0] & m, a[1] & m, a[2] & m, a[3] & m};
+                    // scale 8h + s + 2 c4 (signed byte)
+                    const int byte = 8 * h + s + 2 * c4;
+                    sc[r][c4] = (int)(raw[r].sc[byte >> 2] << (24 - 8 * (byte & 3))) >> 24;
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < C; c++) {
+                v4i a = *(const v4i *)(bt + c * 16 * B_ROW + v * 64);
+                const f4v as = ((const f4v *)ax)[c * 4 + g];
+                asm volatile("" : "+v"(a));                // (see below)
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const v4i zero = {0, 0, 0, 0};
+                    v4i part = zero;
+#pragma unroll
+                    for (int c4 = 0; c4 < 4; c4++) {
+                        const v4i D = mfma64(a, w[r][c4], zero);
+#pragma unroll
+                        for (int k = 0; k < 4; k++) part[k] += __mul24(sc[r][c4], D[k]);
+                    }
+                    const float d = half_bits_to_float(raw[r].d);
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        acc[r][c][k] = acc[r][c][k] + as[k] * d * (float)(part[k] >> 2);
+                }
+                // (left to itself the compiler issues every matrix product of
+                // the block first and needs 256 more registers for them: the
+                // two empty statements order this tile's before the next's)
+#pragma unroll
+                for (int r = 0; r < R; r++) asm volatile("" : "+v"(acc[r][c]));
+            }
+        }
+    }
+}
+
+// Workgroup: 4 waves, each R 16-row tiles, all of them against the same C
+// 16-token tiles.  Work item = (row group, token group); items run token
+// groups first within contiguous ranges per XCD (blockIdx % 8), so that one
+// XCD's L2 serves a row group's weights to all its token groups.
+// BE_SILU: segment 0 is gate, segment 1 up; a wave's tiles are R / 2 gate
+// tiles and the same up tiles, out = silu(gate) * up.
+template <int FMT, int R, int C, int EPI>
+__global__ __launch_bounds__(BT_THREADS, 2) void batch_gemm(BatchArgs a)
+{
+    constexpr int KB = stage_blocks(FMT, C), CH = batch_chunk(FMT), AQ = aux_quads(FMT);
+    constexpr int BB = KB * C * 16 * B_ROW, NAX = KB * C * AQ;
+    static_assert(NAX <= BT_THREADS, "one aux quad per thread and stage");
+    static_assert(EPI != BE_SILU || R % 2 == 0, "gate and up tiles in pairs");
+    __shared__ __align__(16) uint8_t Bs[2][BB];
+    __shared__ u4v As[2][NAX];
+    const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int per = (a.n_wg + 7) >> 3;
+    const int item = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (item >= a.n_wg || (int)(blockIdx.x >> 3) >= per) return;    // (uniform)
+    const int rg = item / a.n_tg, tg = item - rg * a.n_tg;
+    const int nb = a.nb, K = nb * 256, ntt = (a.M + 15) >> 4;
+
+    // this wave's tiles: weights, segment and tile within it (tiles past the
+    // end repeat the last one and are not written)
+    const uint8_t *wp[R];
+    int seg[R], tl[R];
+    bool live[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if (EPI == BE_SILU) {
+            const int p = (rg * 4 + wave) * (R / 2) + (r >> 1);
+            seg[r] = r & 1;
+            live[r] = p < a.tile_start[1];
+            tl[r] = live[r] ? p : a.tile_start[1] - 1;
+        } else {
+            int t = (rg * 4 + wave) * R + r;
+            live[r] = t < a.tile_start[a.nseg];
+            t = live[r] ? t : a.tile_start[a.nseg] - 1;
+            int s = 0;
+            while (s + 1 < a.nseg && t >= a.tile_start[s + 1]) s++;
+            seg[r] = s;
+            tl[r] = t - a.tile_start[s];
+        }
+        wp[r] = a.w[seg[r]] + (size_t)tl[r] * nb * CH;
+    }
+
+    // staging: piece i = (block kb, tile c) of a stage, thread tid its token
+    // row tid / 16, 16-byte piece tid % 16
+    const int st = tid >> 4, sp = tid & 15;
+    const uint8_t *qrow[C];
+#pragma unroll
+    for (int c = 0; c < C; c++)
+        qrow[c] = a.q + (size_t)min((tg * C + c) * 16 + st, a.M - 1) * K + sp * 16;
+    u4v br[KB * C], ar = {0, 0, 0, 0};
+    auto fetch = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+            for (int c = 0; c < C; c++)
+                br[kb * C + c] = *(const u4v *)(qrow[c] + (size_t)min(s * KB + kb, nb - 1) * 256);
+        const int ai = min(tid, NAX - 1), i = ai / AQ, kb = i / C, c = i - kb * C;
+        ar = ((const u4v *)a.aux)[((size_t)min(tg * C + c, ntt - 1) * nb + min(s * KB + kb, nb - 1)) * AQ +
+                                  (ai - i * AQ)];
+    };
+    auto stash = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < KB * C; i++)
+            *(u4v *)(Bs[buf] + (i * 16 + st) * B_ROW + sp * 16) = br[i];
+        if (tid < NAX) As[buf][tid] = ar;
+    };
+    RawBlock<FMT> cur[KB][R], nxt[KB][R];
+    auto weights = [&](int s, RawBlock<FMT> (&dst)[KB][R]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                dst[kb][r].load(wp[r] + (size_t)min(s * KB + kb, nb - 1) * CH, lane);
+    };
+    f4v acc[R][C];
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int c = 0; c < C; c++) acc[r][c] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+
+    const int ns = (nb + KB - 1) / KB;
+    fetch(0);
+    weights(0, cur);
+    stash(0);
+    __syncthreads();
+    for (int s = 0; s < ns; s++) {
+        const int buf = s & 1, sn = min(s + 1, ns - 1);
+        fetch(sn);
+        weights(sn, nxt);
+#pragma unroll
+        for (int kb = 0; kb < KB; kb++)
+            if (s * KB + kb < nb)                            // (uniform)
+                block_terms<FMT, R, C>(cur[kb], Bs[buf] + kb * C * 16 * B_ROW,
+                                       &As[buf][kb * C * AQ], lane, acc);
+        // the other buffer was last read before the previous barrier
+        stash(buf ^ 1);
+#pragma unroll
+        for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+            for (int r = 0; r < R; r++) cur[kb][r] = nxt[kb][r];
+        __syncthreads();
+    }
+
+    // lane (j, g): row j of each tile, tokens 4g .. 4g + 3 of each token tile
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int t0 = (tg * C + c) * 16 + 4 * g;
+        float sc[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) sc[k] = FMT == FMT_TQ2 ? a.scale[min(t0 + k, a.M - 1)] : 1.0f;
+        if (EPI == BE_SILU) {
+#pragma unroll
+            for (int r = 0; r < R; r += 2) {
+                const int row = tl[r] * 16 + j;
+                if (!live[r] || row >= a.n_rows[0]) continue;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    if (t0 + k >= a.M) continue;
+                    const float gt = FMT == FMT_TQ2 ? acc[r][c][k] * sc[k] : acc[r][c][k];
+                    const float up = FMT == FMT_TQ2 ? acc[r + 1][c][k] * sc[k] : acc[r + 1][c][k];
+                    const float sg = fox_div(gt, 1.0f + fox_expf(-gt));
+                    a.out[0][(size_t)(t0 + k) * a.out_stride[0] + row] = sg * up;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const int row = tl[r] * 16 + j;
+                if (!live[r] || row >= a.n_rows[seg[r]]) continue;
+                float *o = a.out[seg[r]] + row;
+                const size_t os = a.out_stride[seg[r]];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    if (t0 + k >= a.M) continue;
+                    const float y = FMT == FMT_TQ2 ? acc[r][c][k] * sc[k] : acc[r][c][k];
+                    float *p = o + (size_t)(t0 + k) * os;
+                    *p = (a.flags & FOX_GPU_GEMV_ACCUMULATE) ? *p + y : y;
+                }
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------ host
+
+static size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+#define PREP_MAX_R 16                   // batch_prep: K <= 2048 * PREP_MAX_R
+
+struct BatchWs {
+    uint8_t *q;
+    uint32_t *aux;
+    float *scale;
+};
+
+// the prepared operand of M tokens of width K in the context's workspace
+static fox_gpu_status batch_carve(fox_gpu_ctx *ctx, int fmt, size_t K, size_t M, BatchWs *w)
+{
+    const size_t nq = up256(M * K);
+    const size_t na = up256((M + 15) / 16 * (K / 256) * (size_t)aux_quads(fmt) * 16);
+    const size_t ns = up256(M * 4);
+    fox_gpu_status st = fox_ws_reserve(ctx, nq + na + ns);
+    if (st) return st;
+    w->q = ctx->ws;
+    w->aux = (uint32_t *)(ctx->ws + nq);
+    w->scale = (float *)(ctx->ws + nq + na);
+    return FOX_GPU_OK;
+}
+
+template <int FMT, bool NORM>
+static const void *prep_kernel(int r)
+{
+    return r <= 1 ? (const void *)batch_prep<FMT, NORM, 1> : r <= 2 ? (const void *)batch_prep<FMT, NORM, 2>
+         : r <= 3 ? (const void *)batch_prep<FMT, NORM, 3> : r <= 4 ? (const void *)batch_prep<FMT, NORM, 4>
+         : r <= 6 ? (const void *)batch_prep<FMT, NORM, 6> : r <= 8 ? (const void *)batch_prep<FMT, NORM, 8>
+         : r <= 12 ? (const void *)batch_prep<FMT, NORM, 12> : (const void *)batch_prep<FMT, NORM, 16>;
+}
+
+template <int FMT>
+static const void *prep_fmt(bool norm, int r)
+{
+    return norm ? prep_kernel<FMT, true>(r) : prep_kernel<FMT, false>(r);
+}
+
+template <int FMT, int R, int EPI>
+static const void *gemm_c(int C)
+{
+    return C == 1 ? (const void *)batch_gemm<FMT, R, 1, EPI> : C == 2 ? (const void *)batch_gemm<FMT, R, 2, EPI>
+         : C == 3 ? (const void *)batch_gemm<FMT, R, 3, EPI> : (const void *)batch_gemm<FMT, R, 4, EPI>;
+}
+
+static const void *gemm_kernel(int fmt, int R, int C, int epi)
+{
+    if (fmt == FMT_TQ2) {
+        if (epi == BE_SILU) return R == 4 ? gemm_c<FMT_TQ2, 4, BE_SILU>(C) : gemm_c<FMT_TQ2, 2, BE_SILU>(C);
+        return R == 4 ? gemm_c<FMT_TQ2, 4, BE_STORE>(C) : R == 2 ? gemm_c<FMT_TQ2, 2, BE_STORE>(C)
+                                                                 : gemm_c<FMT_TQ2, 1, BE_STORE>(C);
+    }
+    if (fmt == FMT_Q4K)
+        return epi == BE_SILU ? gemm_c<FMT_Q4K, 2, BE_SILU>(C) : gemm_c<FMT_Q4K, 1, BE_STORE>(C);
+    return gemm_c<FMT_Q6K, 1, BE_STORE>(C);
+}
+
+static fox_gpu_status batch_check(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor *const *ws,
+                                  const float *x, size_t x_stride, size_t M, float *const *outs,
+                                  const size_t *out_strides)
+{
+    if (!ctx || !ws || !x || !outs || !out_strides || n == 0 || n > MAX_SEGS)
+        return fox_fail(FOX_GPU_ERR_ARG, "batch: bad argument");
+    if (M == 0 || M > FOX_GPU_BATCH_TOKENS)
+        return fox_fail(FOX_GPU_ERR_ARG, "batch: %zu tokens; 1 to %d per call", M,
+                        FOX_GPU_BATCH_TOKENS);
+    for (size_t i = 0; i < n; i++) {
+        if (!ws[i] || !outs[i]) return fox_fail(FOX_GPU_ERR_ARG, "batch: null matrix or output");
+        if (ws[i]->type != ws[0]->type || ws[i]->ne0 != ws[0]->ne0)
+            return fox_fail(FOX_GPU_ERR_ARG,
+                            "batch: matrices of one call must share type and width");
+        if (out_strides[i] < ws[i]->ne1)
+            return fox_fail(FOX_GPU_ERR_ARG, "batch: output stride < rows");
+        if (ws[i]->ne0 > (1u << 20) || ws[i]->ne1 > (1u << 30))
+            return fox_fail(FOX_GPU_ERR_UNSUPPORTED, "batch: matrix too large");
+    }
+    if (x_stride < ws[0]->ne0) return fox_fail(FOX_GPU_ERR_ARG, "batch: input stride < K");
+    return FOX_GPU_OK;
+}
+
+// prepare + GEMM; FOX_GPU_ERR_UNSUPPORTED (no error recorded) where the
+// caller takes the calls of FOX_GPU_MAX_TOKENS tokens
+static fox_gpu_status batch_run(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor *const *ws,
+                                const float *x, size_t x_stride, size_t M, const float *norm_w,
+                                float eps, float *const *outs, const size_t *out_strides,
+                                unsigned flags, int epi)
+{
+    const int fmt = fmt_of(ws[0]->type);
+    const size_t K = (size_t)ws[0]->ne0;
+    // (Q6_K gate/up pairs: two such tiles per wave do not fit its registers)
+    if (fmt < 0 || (fmt == FMT_Q6K && epi == BE_SILU) || K == 0 || K % 256 || K > 2048 * PREP_MAX_R || x_stride % 4 ||
+        ((uintptr_t)x | (uintptr_t)norm_w) % 16)
+        return FOX_GPU_ERR_UNSUPPORTED;
+    BatchWs w;
+    fox_gpu_status st = batch_carve(ctx, fmt, K, M, &w);
+    if (st) return st;
+    {
+        const int r = (int)((K / 4 + 511) / 512);
+        const void *k = fmt == FMT_TQ2 ? prep_fmt<FMT_TQ2>(norm_w != nullptr, r)
+                      : fmt == FMT_Q4K ? prep_fmt<FMT_Q4K>(norm_w != nullptr, r)
+                                       : prep_fmt<FMT_Q6K>(norm_w != nullptr, r);
+        int iK = (int)K;
+        void *args[] = {(void *)&x, (void *)&norm_w, (void *)&iK, (void *)&x_stride, (void *)&eps,
+                        (void *)&w.q, (void *)&w.aux, (void *)&w.scale};
+        hipError_t e = hipLaunchKernel(k, dim3((unsigned)M), dim3(512), args, 0, ctx->stream);
+        if (e != hipSuccess) return fox_hip_fail(e, "batch: prepare");
+        FOX_LAUNCHED("batch: prepare");
+    }
+    BatchArgs a;
+    memset(&a, 0, sizeof(a));
+    a.nseg = (int)n;
+    a.nb = (int)(K / 256);
+    a.M = (int)M;
+    a.flags = flags;
+    a.q = w.q;
+    a.aux = w.aux;
+    a.scale = w.scale;
+    int tiles = 0;
+    for (size_t i = 0; i < n; i++) {
+        a.w[i] = ws[i]->d;
+        a.out[i] = outs[i];
+        a.out_stride[i] = out_strides[i];
+        a.n_rows[i] = (int)ws[i]->ne1;
+        a.tile_start[i] = tiles;
+        tiles += (int)ws[i]->n_tiles;
+    }
+    a.tile_start[n] = tiles;
+    // token groups of C 16-token tiles, as even as they come at C <= 4
+    const int mt = (int)((M + 15) / 16), n_tg = (mt + 3) / 4, C = (mt + n_tg - 1) / n_tg;
+    a.n_tg = (mt + C - 1) / C;
+    // row tiles per wave: more share each token operand read from LDS (the
+    // ternary kernel's LDS reads take as long as its MFMAs below four), as
+    // long as every compute unit still gets two workgroups
+    int R = epi == BE_SILU ? 2 : 1;
+    if (fmt == FMT_TQ2) {
+        const int want = 2 * ctx->n_cu;
+        while (R < 4 && (tiles + 8 * R - 1) / (8 * R) * a.n_tg >= want) R *= 2;
+    }
+    a.n_wg = (tiles + 4 * R - 1) / (4 * R) * a.n_tg;
+    const void *k = gemm_kernel(fmt, R, C, epi);
+    void *args[] = {(void *)&a};
+    hipError_t e = hipLaunchKernel(k, dim3((unsigned)((a.n_wg + 7) / 8 * 8)), dim3(BT_THREADS), args, 0,
+                                   ctx->stream);
+    if (e != hipSuccess) return fox_hip_fail(e, "batch: product");
+    FOX_LAUNCHED("batch: product");
+    return FOX_GPU_OK;
+}
+
+extern "C" fox_gpu_status fox_gpu_batch_gemv(fox_gpu_ctx *ctx, size_t n,
+                                             const fox_gpu_tensor *const *ws, const float *x,
+                                             size_t x_stride, size_t M, float *const *outs,
+                                             const size_t *out_strides, unsigned flags)
+{
+    fox_gpu_status st = batch_check(ctx, n, ws, x, x_stride, M, outs, out_strides);
+    if (st) return st;
+    if (fmt_of(ws[0]->type) < 0) {
+        for (size_t i = 0; i < n && !st; i++)
+            st = fox_float_gemv(ctx, ws[i], x, x_stride, M, outs[i], out_strides[i], flags);
+        return st;
+    }
+    st = batch_run(ctx, n, ws, x, x_stride, M, nullptr, 0.0f, outs, out_strides, flags, BE_STORE);
+    if (st != FOX_GPU_ERR_UNSUPPORTED) return st;
+    for (size_t t = 0; t < M; t += FOX_GPU_MAX_TOKENS) {
+        const size_t m = M - t < FOX_GPU_MAX_TOKENS ? M - t : FOX_GPU_MAX_TOKENS;
+        float *o[MAX_SEGS];
+        for (size_t i = 0; i < n; i++) o[i] = outs[i] + t * out_strides[i];
+        st = fox_gemv_launch(ctx, n, ws, x + t * x_stride, x_stride, nullptr, nullptr, m, o,
+                             out_strides, flags, nullptr);
+        if (st) return st;
+    }
+    return FOX_GPU_OK;
+}
+
+extern "C" fox_gpu_status fox_gpu_batch_gemv_rmsnorm(fox_gpu_ctx *ctx, size_t n,
+                                                     const fox_gpu_tensor *const *ws,
+                                                     const float *x, size_t x_stride, size_t M,
+                                                     const float *norm_w, float eps,
+                                                     float *const *outs, const size_t *out_strides,
+                                                     unsigned flags)
+{
+    fox_gpu_status st = batch_check(ctx, n, ws, x, x_stride, M, outs, out_strides);
+    if (st) return st;
+    if (!norm_w) return fox_fail(FOX_GPU_ERR_ARG, "batch: null norm weights");
+    return batch_run(ctx, n, ws, x, x_stride, M, norm_w, eps, outs, out_strides, flags, BE_STORE);
+}
+
+extern "C" fox_gpu_status fox_gpu_batch_gate_up_silu(fox_gpu_ctx *ctx, const fox_gpu_tensor *w_gate,
+                                                     const fox_gpu_tensor *w_up, const float *x,
+                                                     size_t x_stride, size_t M,
+                                                     const float *norm_w, float eps, float *h_out,
+                                                     size_t h_stride)
+{
+    const fox_gpu_tensor *ws[2] = {w_gate, w_up};
+    float *outs[2] = {h_out, h_out};
+    size_t strides[2] = {h_stride, h_stride};
+    if (w_gate && w_up && w_gate->type != w_up->type) return FOX_GPU_ERR_UNSUPPORTED;
+    fox_gpu_status st = batch_check(ctx, 2, ws, x, x_stride, M, outs, strides);
+    if (st) return st;
+    if (!norm_w) return fox_fail(FOX_GPU_ERR_ARG, "batch: null norm weights");
+    if (w_gate->ne1 != w_up->ne1)
+        return fox_fail(FOX_GPU_ERR_ARG, "batch: gate and up must have the same rows");
+    return batch_run(ctx, 2, ws, x, x_stride, M, norm_w, eps, outs, strides, 0, BE_SILU);
+}

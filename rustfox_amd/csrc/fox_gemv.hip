@@ -452,7 +452,15 @@ __global__ __launch_bounds__(RW) void gemv_float(const WT *__restrict__ W, int K
     constexpr int NP = PPR;                             // pieces per thread
     __shared__ uint32_t wl[2][RW * RSTR];
     __shared__ float xs[2][MT * FK];
-    if (MT == 1) M = 1;
+    if (MT == 1) {
+        M = 1;
+    } else {
+        // (a batched pass: token groups of MT on the grid's second axis)
+        const int t0 = (int)blockIdx.y * MT;
+        x += (size_t)t0 * x_stride;
+        out += (size_t)t0 * out_stride;
+        M = min(MT, M - t0);
+    }
     const int tid = threadIdx.x;
     const int r0 = blockIdx.x * RW;
     const int nchunk = (K + FK - 1) / FK;               // steps
@@ -558,6 +566,38 @@ __global__ __launch_bounds__(RW) void gemv_float(const WT *__restrict__ W, int K
 }
 
 // ----------------------------------------------------------------- host
+
+// F16 / F32 weights, any number of tokens (groups of FOX_GPU_MAX_TOKENS)
+fox_gpu_status fox_float_gemv(fox_gpu_ctx *ctx, const fox_gpu_tensor *w, const float *x,
+                              size_t x_stride, size_t M, float *out, size_t out_stride,
+                              unsigned flags)
+{
+    const int N = (int)w->ne1, K = (int)w->ne0;
+    // one token: half-tile workgroups (a 151936-row head is 1187 of
+    // them: 4.6 per compute unit, against 2.3 whole tiles)
+    constexpr int RH = FR / 2;
+    dim3 grid((unsigned)((N + FR - 1) / FR),
+              (unsigned)((M + FOX_GPU_MAX_TOKENS - 1) / FOX_GPU_MAX_TOKENS)), block(FR);
+    dim3 grid1((unsigned)((N + RH - 1) / RH)), block1(RH);
+    const _Float16 *wh = (const _Float16 *)w->d;
+    const float *wf = (const float *)w->d;
+    if (w->type == FOX_GPU_F16 && M == 1)
+        hipLaunchKernelGGL((gemv_float<_Float16, 1, RH>), grid1, block1, 0, ctx->stream, wh, K, N, x,
+                           (int)x_stride, (int)M, out, (int)out_stride, flags);
+    else if (w->type == FOX_GPU_F16)
+        hipLaunchKernelGGL((gemv_float<_Float16, FOX_GPU_MAX_TOKENS, FR>), grid, block, 0,
+                           ctx->stream, wh, K, N, x, (int)x_stride, (int)M, out, (int)out_stride,
+                           flags);
+    else if (M == 1)
+        hipLaunchKernelGGL((gemv_float<float, 1, RH>), grid1, block1, 0, ctx->stream, wf, K, N, x,
+                           (int)x_stride, (int)M, out, (int)out_stride, flags);
+    else
+        hipLaunchKernelGGL((gemv_float<float, FOX_GPU_MAX_TOKENS, FR>), grid, block, 0,
+                           ctx->stream, wf, K, N, x, (int)x_stride, (int)M, out, (int)out_stride,
+                           flags);
+    FOX_LAUNCHED("gemv_float");
+    return FOX_GPU_OK;
+}
 
 static size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
@@ -702,33 +742,9 @@ static fox_gpu_status gemv_launch_ws(fox_gpu_ctx *ctx, size_t n, const fox_gpu_t
         if (!x || sums)
             return fox_fail(FOX_GPU_ERR_UNSUPPORTED,
                             "gemv: %s weights take float activations", fox_type_name(type));
-        for (size_t i = 0; i < n; i++) {
-            const int N = (int)ws[i]->ne1;
-            // one token: half-tile workgroups (a 151936-row head is 1187 of
-            // them: 4.6 per compute unit, against 2.3 whole tiles)
-            constexpr int RH = FR / 2;
-            dim3 grid((unsigned)((N + FR - 1) / FR)), block(FR);
-            dim3 grid1((unsigned)((N + RH - 1) / RH)), block1(RH);
-            const _Float16 *wh = (const _Float16 *)ws[i]->d;
-            const float *wf = (const float *)ws[i]->d;
-            if (type == FOX_GPU_F16 && M == 1)
-                hipLaunchKernelGGL((gemv_float<_Float16, 1, RH>), grid1, block1, 0, ctx->stream, wh,
-                                   (int)K, N, x, (int)x_stride, (int)M, outs[i],
-                                   (int)out_strides[i], flags);
-            else if (type == FOX_GPU_F16)
-                hipLaunchKernelGGL((gemv_float<_Float16, FOX_GPU_MAX_TOKENS, FR>), grid, block, 0,
-                                   ctx->stream, wh, (int)K, N, x, (int)x_stride, (int)M, outs[i],
-                                   (int)out_strides[i], flags);
-            else if (M == 1)
-                hipLaunchKernelGGL((gemv_float<float, 1, RH>), grid1, block1, 0, ctx->stream, wf,
-                                   (int)K, N, x, (int)x_stride, (int)M, outs[i],
-                                   (int)out_strides[i], flags);
-            else
-                hipLaunchKernelGGL((gemv_float<float, FOX_GPU_MAX_TOKENS, FR>), grid, block, 0,
-                                   ctx->stream, wf, (int)K, N, x, (int)x_stride, (int)M, outs[i],
-                                   (int)out_strides[i], flags);
-            FOX_LAUNCHED("gemv_float");
-        }
+        for (size_t i = 0; i < n; i++)
+            if ((st = fox_float_gemv(ctx, ws[i], x, x_stride, M, outs[i], out_strides[i], flags)))
+                return st;
         return FOX_GPU_OK;
     }
 

@@ -338,6 +338,23 @@ __global__ void rope_store_k(float *__restrict__ q, size_t q_stride, float *__re
     }
 }
 
+static fox_gpu_status rope_store_any(fox_gpu_ctx *ctx, float *q, size_t q_stride, float *k,
+                                     size_t k_stride, const float *v, size_t v_stride,
+                                     size_t n_head, size_t n_head_kv, size_t head_dim, size_t M,
+                                     const float *cos_t, const float *sin_t, const uint32_t *pos,
+                                     size_t n_ctx, float *k_cache, float *v_cache)
+{
+    if (!ctx || !q || !k || !v || !cos_t || !sin_t || !pos || !k_cache || !v_cache ||
+        n_head == 0 || n_head_kv == 0 || head_dim == 0 || M == 0 || n_ctx == 0)
+        return fox_fail(FOX_GPU_ERR_ARG, "rope_store: bad argument");
+    if (head_dim % 2) return fox_fail(FOX_GPU_ERR_UNSUPPORTED, "rope_store: odd head dimension");
+    hipLaunchKernelGGL(rope_store_k, dim3((unsigned)M), dim3(256), 0, ctx->stream, q, q_stride, k,
+                       k_stride, v, v_stride, (int)n_head, (int)n_head_kv, (int)head_dim, cos_t,
+                       sin_t, pos, n_ctx, k_cache, v_cache);
+    FOX_LAUNCHED("rope_store");
+    return FOX_GPU_OK;
+}
+
 extern "C" fox_gpu_status fox_gpu_rope_store(fox_gpu_ctx *ctx, float *q, size_t q_stride,
                                              float *k, size_t k_stride, const float *v,
                                              size_t v_stride, size_t n_head, size_t n_head_kv,
@@ -345,16 +362,22 @@ extern "C" fox_gpu_status fox_gpu_rope_store(fox_gpu_ctx *ctx, float *q, size_t 
                                              const float *sin_t, const uint32_t *pos,
                                              size_t n_ctx, float *k_cache, float *v_cache)
 {
-    if (!ctx || !q || !k || !v || !cos_t || !sin_t || !pos || !k_cache || !v_cache ||
-        n_head == 0 || n_head_kv == 0 || head_dim == 0 || M == 0 || n_ctx == 0)
-        return fox_fail(FOX_GPU_ERR_ARG, "rope_store: bad argument");
-    if (head_dim % 2) return fox_fail(FOX_GPU_ERR_UNSUPPORTED, "rope_store: odd head dimension");
     if (M > FOX_GPU_MAX_TOKENS) return fox_fail(FOX_GPU_ERR_ARG, "rope_store: too many tokens");
-    hipLaunchKernelGGL(rope_store_k, dim3((unsigned)M), dim3(256), 0, ctx->stream, q, q_stride, k,
-                       k_stride, v, v_stride, (int)n_head, (int)n_head_kv, (int)head_dim, cos_t,
-                       sin_t, pos, n_ctx, k_cache, v_cache);
-    FOX_LAUNCHED("rope_store");
-    return FOX_GPU_OK;
+    return rope_store_any(ctx, q, q_stride, k, k_stride, v, v_stride, n_head, n_head_kv, head_dim,
+                          M, cos_t, sin_t, pos, n_ctx, k_cache, v_cache);
+}
+
+// the same for a batched pass (up to FOX_GPU_BATCH_TOKENS tokens)
+extern "C" fox_gpu_status fox_gpu_batch_rope_store(fox_gpu_ctx *ctx, float *q, size_t q_stride, float *k,
+                                     size_t k_stride, const float *v, size_t v_stride,
+                                     size_t n_head, size_t n_head_kv, size_t head_dim, size_t M,
+                                     const float *cos_t, const float *sin_t, const uint32_t *pos,
+                                     size_t n_ctx, float *k_cache, float *v_cache)
+{
+    if (M > FOX_GPU_BATCH_TOKENS)
+        return fox_fail(FOX_GPU_ERR_ARG, "rope_store: too many tokens");
+    return rope_store_any(ctx, q, q_stride, k, k_stride, v, v_stride, n_head, n_head_kv, head_dim,
+                          M, cos_t, sin_t, pos, n_ctx, k_cache, v_cache);
 }
 
 // rows p0 .. p0+n-1 of both caches from row-major [n][kv_dim] k and v
@@ -1214,7 +1237,7 @@ __global__ __launch_bounds__(256) void attn_hv(const float *__restrict__ att, si
 __global__ __launch_bounds__(256) void attn_sm(float *__restrict__ att, size_t att_stride,
                                                const float *__restrict__ tmax, int n_tiles,
                                                int n_head, const uint32_t *__restrict__ pos,
-                                               int n_ctx)
+                                               int n_ctx, int t_base)
 {
     extern __shared__ float4 sm_lds[];
     float *e = (float *)sm_lds;                    // [ceil4(upto)]
@@ -1222,7 +1245,7 @@ __global__ __launch_bounds__(256) void attn_sm(float *__restrict__ att, size_t a
     __shared__ uint64_t tab[32];
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
     const int h = blockIdx.x, t = blockIdx.y;
-    const int upto = (int)min((size_t)pos[0] + (size_t)t + 1, (size_t)n_ctx);
+    const int upto = (int)min((size_t)pos[0] + (size_t)(t_base + t) + 1, (size_t)n_ctx);
     float *row = att + ((size_t)t * n_head + h) * att_stride;
     const bool producer = wave > 0;
     const int L = tid - 64;
@@ -1443,6 +1466,25 @@ __global__ __launch_bounds__(256) void attn_avm(const float *__restrict__ att, s
     }
 }
 
+fox_gpu_status fox_attn_softmax(fox_gpu_ctx *ctx, float *att, size_t att_stride, const float *tmax,
+                                int n_tiles, int n_head, const uint32_t *pos, int t_base, int n_ctx,
+                                int M)
+{
+    // (SUM_CHUNK floats past the weights: softmax_sum_block reads whole
+    // chunks of SUM_CHUNK)
+    const size_t sm_lds = (att_stride + SUM_CHUNK) * sizeof(float);
+    if (sm_lds > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute((const void *)attn_sm,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)sm_lds);
+        if (e != hipSuccess) return fox_hip_fail(e, "attention: LDS size");
+    }
+    hipLaunchKernelGGL(attn_sm, dim3((unsigned)n_head, (unsigned)M), dim3(256), sm_lds,
+                       ctx->stream, att, att_stride, tmax, n_tiles, n_head, pos, n_ctx, t_base);
+    FOX_LAUNCHED("attention softmax");
+    return FOX_GPU_OK;
+}
+
 extern "C" fox_gpu_status fox_gpu_attention(fox_gpu_ctx *ctx, float *out, size_t out_stride,
                                             const float *q, size_t q_stride, const float *k_cache,
                                             const float *v_cache, size_t n_head, size_t n_head_kv,
@@ -1542,21 +1584,9 @@ extern "C" fox_gpu_status fox_gpu_attention(fox_gpu_ctx *ctx, float *out, size_t
         // workgroup
         const int gp = gqa == 1 ? 1 : gqa == 2 ? 2 : gqa <= 4 ? 4 : 8;
         const size_t dcm = AV_CH / gp;
-        {
-            // (SUM_CHUNK floats past the weights: softmax_sum_block reads
-            // whole chunks of SUM_CHUNK)
-            const size_t sm_lds = (att_stride + SUM_CHUNK) * sizeof(float);
-            if (sm_lds > 64 * 1024) {
-                hipError_t e = hipFuncSetAttribute((const void *)attn_sm,
-                                                   hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                   (int)sm_lds);
-                if (e != hipSuccess) return fox_hip_fail(e, "attention: LDS size");
-            }
-            hipLaunchKernelGGL(attn_sm, dim3((unsigned)n_head, (unsigned)M), dim3(256), sm_lds,
-                               ctx->stream, att, att_stride, tmax, n_tiles, (int)n_head, pos,
-                               (int)n_ctx);
-            FOX_LAUNCHED("attention softmax");
-        }
+        if ((st = fox_attn_softmax(ctx, att, att_stride, tmax, n_tiles, (int)n_head, pos, 0,
+                                   (int)n_ctx, (int)M)))
+            return st;
         const void *avm = gp == 1 ? (const void *)attn_avm<1> : gp == 2 ? (const void *)attn_avm<2>
                         : gp == 4 ? (const void *)attn_avm<4> : (const void *)attn_avm<8>;
         const size_t avm_lds = 2 * 64 * MV_PS * 16;

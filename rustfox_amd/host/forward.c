@@ -11,11 +11,13 @@
  * The K cache is f32 [n_layer][n_ctx][n_head_kv * head_dim] as in the
  * reference, the V cache the device's position-quad interleaved layout
  * (fox_gpu.h) per layer; the RoPE tables are built on the host in double exactly as
- * src/forward.c:104-118 and uploaded.  A pass takes at most
- * FOX_GPU_MAX_TOKENS tokens; fox_eval cuts its input into such passes, which
- * gives the same result as the reference's n_batch chunks because a token
- * depends only on the cache rows before it (batched == stepped,
- * tests/test_forward.c:258-272).
+ * src/forward.c:104-118 and uploaded.  fox_eval cuts its input into passes:
+ * of at most FOX_GPU_MAX_TOKENS tokens (the decode kernels), or, where
+ * n_batch is larger than that and as many tokens are left, of up to
+ * FOX_GPU_BATCH_TOKENS (the batched kernels; a 1024-token prompt of the
+ * 4B-class layers in passes of 8 read the weights 128 times).  The result is
+ * that of the reference's n_batch chunks because a token depends only on the
+ * cache rows before it (batched == stepped, tests/test_forward.c:258-272).
  */
 #include "fox_host_internal.h"
 
@@ -28,6 +30,15 @@ typedef struct {
     const fox_gpu_tensor *attn_q, *attn_k, *attn_v, *attn_out, *ffn_gate, *ffn_up, *ffn_down;
     float *attn_norm, *ffn_norm;   /* device f32 [n_embd] */
 } dev_layer;
+
+/* device activations of a pass of up to `cap` tokens */
+typedef struct {
+    float *x, *xb, *q, *k, *v, *hb, *hb2;
+    uint32_t *tok, *pos;           /* pos[i]: the position of token 8 i */
+    size_t cap;
+} pass_buffers;
+
+#define HEAD_ROWS 64               /* logits rows of one product of a batched fox_eval_all */
 
 struct fox_context {
     fox_model          *m;
@@ -46,6 +57,11 @@ struct fox_context {
     float *logits;                 /* host */
     double last_seconds;
     uint64_t reads_at_start;
+    /* batched passes: allocated at the first one (cap 0 before, and where
+     * the memory is not there: passes of FOX_GPU_MAX_TOKENS then) */
+    pass_buffers B;
+    float *blogits;                /* HEAD_ROWS rows, at the first batched fox_eval_all */
+    int no_batch;
     fox_gpu_graph *greedy;
     int attn_mode;                 /* FOX_GPU_ATTN_EXACT or FOX_GPU_ATTN_SPLIT */
     void *allocs[32];
@@ -314,6 +330,51 @@ static fox_status project_group(fox_context *c, size_t n, const fox_gpu_tensor *
     return FOX_OK;
 }
 
+/* layer l's matrices: resident, or from the layer's slot (*SD; loaded now if
+ * the prefetch did not reach it; the compute stream waits for its upload) */
+static fox_status layer_of(fox_context *c, uint32_t l, dev_layer *SD, const dev_layer **D)
+{
+    const fox_gpu_tensor *lt[FOX_LAYER_ROLES];
+    fox_status st;
+    *D = &c->L[l];
+    if (!streaming(c)) return FOX_OK;
+    if ((st = fox_weights_use_layer(c->m->weights, l, lt)) != FOX_OK) return st;
+    *SD = c->L[l];
+    SD->attn_q = lt[FOX_ROLE_ATTN_Q];
+    SD->attn_k = lt[FOX_ROLE_ATTN_K];
+    SD->attn_v = lt[FOX_ROLE_ATTN_V];
+    SD->attn_out = lt[FOX_ROLE_ATTN_OUT];
+    SD->ffn_gate = lt[FOX_ROLE_FFN_GATE];
+    SD->ffn_up = lt[FOX_ROLE_FFN_UP];
+    SD->ffn_down = lt[FOX_ROLE_FFN_DOWN];
+    *D = SD;
+    return FOX_OK;
+}
+
+/* the layer-ahead load (src/forward.c:333-337): the next layer, or the first
+ * one of the next pass, goes up on the copy stream while this one computes */
+static fox_status layer_done(fox_context *c, uint32_t l)
+{
+    if (!streaming(c)) return FOX_OK;
+    fox_weights_done_layer(c->m->weights, l);
+    return fox_weights_prefetch_layer(c->m->weights, (l + 1) % c->m->info.n_layer);
+}
+
+/* output norm and head (src/forward.c:401-408) over rows of a pass: each
+ * row's are independent of the others */
+static fox_status head(fox_context *c, const float *x, float *xb, size_t rows, float *logits)
+{
+    GPU(fox_gpu_rmsnorm(c->gpu, xb, c->wide, x, c->d, c->out_norm, c->d, rows,
+                        c->m->info.rms_eps), "forward: output_norm");
+    if (rows > FOX_GPU_MAX_TOKENS)
+        GPU(fox_gpu_batch_gemv(c->gpu, 1, &c->out, xb, c->wide, rows, &logits, &c->vocab, 0),
+            "forward: output");
+    else
+        GPU(fox_gpu_gemv(c->gpu, c->out, xb, c->wide, rows, logits, c->vocab, 0),
+            "forward: output");
+    return FOX_OK;
+}
+
 /* one pass over all layers for M <= FOX_GPU_MAX_TOKENS tokens already in
  * dtok, at the position held in dpos; queued on the stream, no host sync.
  * want_logits: 0 none, 1 the last token's (dlogits row 0), 2 every token's
@@ -330,22 +391,8 @@ static fox_status forward_pass(fox_context *c, size_t M, int want_logits)
     GPU(fox_gpu_get_rows(c->gpu, c->embd, c->dtok, M, c->x, c->d, NULL), "forward: embed");
     for (l = 0; l < mi->n_layer; l++) {
         dev_layer SD;
-        const dev_layer *D = &c->L[l];
-        if (streaming(c)) {
-            /* this layer from its slot (loaded now if the prefetch did not
-             * reach it); the compute stream waits for its upload */
-            const fox_gpu_tensor *lt[FOX_LAYER_ROLES];
-            if ((st = fox_weights_use_layer(c->m->weights, l, lt)) != FOX_OK) return st;
-            SD = *D;
-            SD.attn_q = lt[FOX_ROLE_ATTN_Q];
-            SD.attn_k = lt[FOX_ROLE_ATTN_K];
-            SD.attn_v = lt[FOX_ROLE_ATTN_V];
-            SD.attn_out = lt[FOX_ROLE_ATTN_OUT];
-            SD.ffn_gate = lt[FOX_ROLE_FFN_GATE];
-            SD.ffn_up = lt[FOX_ROLE_FFN_UP];
-            SD.ffn_down = lt[FOX_ROLE_FFN_DOWN];
-            D = &SD;
-        }
+        const dev_layer *D;
+        if ((st = layer_of(c, l, &SD, &D)) != FOX_OK) return st;
         const fox_gpu_tensor *qkv[3] = { D->attn_q, D->attn_k, D->attn_v };
         float *qkv_out[3] = { c->q, c->k, c->v };
         size_t qkv_str[3] = { c->nq, c->nkv, c->nkv };
@@ -388,24 +435,160 @@ static fox_status forward_pass(fox_context *c, size_t M, int want_logits)
         }
         GPU(fox_gpu_gemv(c->gpu, D->ffn_down, c->hb, c->ff, M, c->x, c->d,
                          FOX_GPU_GEMV_ACCUMULATE), "forward: ffn_down");
-        if (streaming(c)) {
-            /* the layer-ahead load (src/forward.c:333-337): the next layer,
-             * or the first one of the next pass, goes up on the copy stream
-             * while this one computes */
-            fox_weights_done_layer(c->m->weights, l);
-            if ((st = fox_weights_prefetch_layer(c->m->weights, (l + 1) % mi->n_layer)) != FOX_OK)
-                return st;
-        }
+        if ((st = layer_done(c, l)) != FOX_OK) return st;
     }
     if (!want_logits) return FOX_OK;
     {
-        /* src/forward.c:401-408 on the last row, or on every row: each row's
-         * norm and head product are independent of the others */
         const size_t rows = want_logits == 2 ? M : 1;
-        GPU(fox_gpu_rmsnorm(c->gpu, c->xb, c->wide, c->x + (M - rows) * c->d, c->d, c->out_norm,
-                            c->d, rows, mi->rms_eps), "forward: output_norm");
-        GPU(fox_gpu_gemv(c->gpu, c->out, c->xb, c->wide, rows, c->dlogits, c->vocab, 0),
-            "forward: output");
+        return head(c, c->x + (M - rows) * c->d, c->xb, rows, c->dlogits);
+    }
+}
+
+/* y_i = W_i rmsnorm(x, norm_w) of a batched pass, one product for each run
+ * of equal types */
+static fox_status batch_project(fox_context *c, size_t n, const fox_gpu_tensor *const *ws,
+                                size_t M, const float *norm_w, float *const *outs,
+                                const size_t *strides)
+{
+    const float eps = c->m->info.rms_eps;
+    size_t i = 0;
+    int normed = 0;
+    while (i < n) {
+        size_t j = i + 1;
+        fox_gpu_status gs;
+        while (j < n && same_type(ws[i], ws[j])) j++;
+        gs = fox_gpu_batch_gemv_rmsnorm(c->gpu, j - i, ws + i, c->B.x, c->d, M, norm_w, eps,
+                                        outs + i, strides + i, 0);
+        if (gs == FOX_GPU_ERR_UNSUPPORTED) {
+            if (!normed)
+                GPU(fox_gpu_rmsnorm(c->gpu, c->B.xb, c->wide, c->B.x, c->d, norm_w, c->d, M, eps),
+                    "forward: norm");
+            normed = 1;
+            gs = fox_gpu_batch_gemv(c->gpu, j - i, ws + i, c->B.xb, c->wide, M, outs + i,
+                                    strides + i, 0);
+        }
+        if (gs != FOX_GPU_OK) return fox_gpu_failed(gs, "forward: projection");
+        i = j;
+    }
+    return FOX_OK;
+}
+
+static fox_status batch_add(fox_context *c, const fox_gpu_tensor *w, const float *x, size_t stride,
+                            size_t M)
+{
+    float *out = c->B.x;
+    GPU(fox_gpu_batch_gemv(c->gpu, 1, &w, x, stride, M, &out, &c->d, FOX_GPU_GEMV_ACCUMULATE),
+        "forward: projection");
+    return FOX_OK;
+}
+
+/* forward_pass for M > FOX_GPU_MAX_TOKENS tokens in B.tok at position
+ * B.pos[0]; the residual stream of every token ends in B.x */
+static fox_status batch_pass(fox_context *c, size_t M)
+{
+    const fox_model_info *mi = &c->m->info;
+    pass_buffers *B = &c->B;
+    const size_t kvl = (size_t)c->cfg.n_ctx * c->nkv;
+    const size_t vl = FOX_GPU_V_CACHE_FLOATS(c->cfg.n_ctx, c->nkv);
+    uint32_t l;
+    fox_status st;
+    fox_gpu_status gs;
+
+    GPU(fox_gpu_get_rows(c->gpu, c->embd, B->tok, M, B->x, c->d, NULL), "forward: embed");
+    for (l = 0; l < mi->n_layer; l++) {
+        dev_layer SD;
+        const dev_layer *D;
+        float *kc = c->kc + l * kvl, *vc = c->vc + l * vl;
+        if ((st = layer_of(c, l, &SD, &D)) != FOX_OK) return st;
+        {
+            const fox_gpu_tensor *qkv[3] = { D->attn_q, D->attn_k, D->attn_v };
+            float *out[3] = { B->q, B->k, B->v };
+            size_t str[3] = { c->nq, c->nkv, c->nkv };
+            if ((st = batch_project(c, 3, qkv, M, D->attn_norm, out, str)) != FOX_OK) return st;
+        }
+        GPU(fox_gpu_batch_rope_store(c->gpu, B->q, c->nq, B->k, c->nkv, B->v, c->nkv, mi->n_head,
+                                     mi->n_head_kv, c->hd, M, c->rc, c->rs, B->pos, c->cfg.n_ctx,
+                                     kc, vc), "forward: rope");
+        if (c->attn_mode == FOX_GPU_ATTN_EXACT) {
+            GPU(fox_gpu_batch_attention(c->gpu, B->xb, c->wide, B->q, c->nq, kc, vc, mi->n_head,
+                                        mi->n_head_kv, c->hd, M, B->pos, c->cfg.n_ctx),
+                "forward: attention");
+        } else {
+            size_t t;
+            for (t = 0; t < M; t += FOX_GPU_MAX_TOKENS) {
+                const size_t m = M - t < FOX_GPU_MAX_TOKENS ? M - t : FOX_GPU_MAX_TOKENS;
+                GPU(fox_gpu_attention(c->gpu, B->xb + t * c->wide, c->wide, B->q + t * c->nq, c->nq,
+                                      kc, vc, mi->n_head, mi->n_head_kv, c->hd, m,
+                                      B->pos + t / FOX_GPU_MAX_TOKENS, c->cfg.n_ctx, c->attn_mode),
+                    "forward: attention");
+            }
+        }
+        if ((st = batch_add(c, D->attn_out, B->xb, c->wide, M)) != FOX_OK) return st;
+        gs = fox_gpu_batch_gate_up_silu(c->gpu, D->ffn_gate, D->ffn_up, B->x, c->d, M, D->ffn_norm,
+                                        mi->rms_eps, B->hb, c->ff);
+        if (gs == FOX_GPU_ERR_UNSUPPORTED) {
+            const fox_gpu_tensor *gu[2] = { D->ffn_gate, D->ffn_up };
+            float *out[2] = { B->hb, B->hb2 };
+            size_t str[2] = { c->ff, c->ff };
+            if ((st = batch_project(c, 2, gu, M, D->ffn_norm, out, str)) != FOX_OK) return st;
+            GPU(fox_gpu_silu_mul(c->gpu, B->hb, B->hb2, c->ff, M, c->ff), "forward: swiglu");
+        } else if (gs != FOX_GPU_OK) {
+            return fox_gpu_failed(gs, "forward: gate/up");
+        }
+        if ((st = batch_add(c, D->ffn_down, B->hb, c->ff, M)) != FOX_OK) return st;
+        if ((st = layer_done(c, l)) != FOX_OK) return st;
+    }
+    return FOX_OK;
+}
+
+/* the buffers of batched passes; 0 where they cannot be had */
+static int batch_ready(fox_context *c)
+{
+    pass_buffers b;
+    struct { float **p; size_t n; } want[7] = {
+        { &b.x, c->d }, { &b.xb, c->wide }, { &b.q, c->nq }, { &b.k, c->nkv }, { &b.v, c->nkv },
+        { &b.hb, c->ff }, { &b.hb2, c->ff }
+    };
+    const int mark = c->n_allocs;
+    size_t i;
+    int ok = 1;
+    if (c->B.cap) return 1;
+    if (c->no_batch) return 0;
+    b.cap = c->cfg.n_ctx < FOX_GPU_BATCH_TOKENS ? c->cfg.n_ctx : FOX_GPU_BATCH_TOKENS;
+    for (i = 0; ok && i < 7; i++)
+        ok = dalloc(c, b.cap * want[i].n * 4, (void **)want[i].p) == FOX_OK;
+    ok = ok && dalloc(c, b.cap * 4, (void **)&b.tok) == FOX_OK;
+    ok = ok && dalloc(c, (b.cap / FOX_GPU_MAX_TOKENS + 1) * 4, (void **)&b.pos) == FOX_OK;
+    if (!ok) {
+        while (c->n_allocs > mark) fox_gpu_free(c->gpu, c->allocs[--c->n_allocs]);
+        c->no_batch = 1;
+        return 0;
+    }
+    c->B = b;
+    return 1;
+}
+
+/* tokens [done, done + M) as one batched pass; the logits wanted (all: every
+ * row's into `all`; else the last row's into dlogits when `last`) */
+static fox_status batch_eval(fox_context *c, const uint32_t *tokens, size_t M, int last, float *all)
+{
+    uint32_t pos[FOX_GPU_BATCH_TOKENS / FOX_GPU_MAX_TOKENS + 1];
+    const size_t np = (M + FOX_GPU_MAX_TOKENS - 1) / FOX_GPU_MAX_TOKENS;
+    size_t i, r;
+    fox_status st;
+    for (i = 0; i < np; i++) pos[i] = c->pos + (uint32_t)(i * FOX_GPU_MAX_TOKENS);
+    GPU(fox_gpu_memcpy_h2d(c->gpu, c->B.tok, tokens, M * 4), "eval: tokens");
+    GPU(fox_gpu_memcpy_h2d(c->gpu, c->B.pos, pos, np * 4), "eval: position");
+    if ((st = batch_pass(c, M)) != FOX_OK) return st;
+    if (!all) return last ? head(c, c->B.x + (M - 1) * c->d, c->B.xb, 1, c->dlogits) : FOX_OK;
+    if (!c->blogits &&
+        (st = dalloc(c, HEAD_ROWS * c->vocab * 4, (void **)&c->blogits)) != FOX_OK)
+        return st;
+    for (i = 0; i < M; i += r) {
+        r = M - i < HEAD_ROWS ? M - i : HEAD_ROWS;
+        if ((st = head(c, c->B.x + i * c->d, c->B.xb, r, c->blogits)) != FOX_OK) return st;
+        GPU(fox_gpu_memcpy_d2h(c->gpu, all + i * c->vocab, c->blogits, r * c->vocab * 4),
+            "eval: logits");
     }
     return FOX_OK;
 }
@@ -420,35 +603,64 @@ static fox_status check_tokens(const fox_context *c, const uint32_t *t, size_t n
     return FOX_OK;
 }
 
-/* tokens in chunks of at most n_batch (and FOX_GPU_MAX_TOKENS); all == NULL:
- * the last token's logits into c->logits, else every token's into all */
+/* chunk [done, done + chunk) of an evaluation at position `pos` */
+static fox_status check_chunk(const fox_context *c, const uint32_t *tokens, size_t chunk, size_t pos)
+{
+    if (pos + chunk > c->cfg.n_ctx)
+        return fox_fail(FOX_ERR_ARG, "forward: %zu tokens past position %zu would overrun the "
+                        "%u token context", chunk, pos, c->cfg.n_ctx);
+    return check_tokens(c, tokens, chunk);
+}
+
+/* all == NULL: the last token's logits into c->logits, else every token's
+ * into all.  The input is checked in chunks of at most n_batch (and
+ * FOX_GPU_MAX_TOKENS): the chunks before a bad one are evaluated, then its
+ * error is returned.  The good tokens run in batched passes where n_batch
+ * allows more than FOX_GPU_MAX_TOKENS and more than that are left, in such
+ * chunks otherwise. */
 static fox_status eval_chunks(fox_context *c, const uint32_t *tokens, size_t n, float *all)
 {
-    size_t done = 0;
+    size_t done = 0, good = 0, cap = c->cfg.n_batch;
     double t0;
-    fox_status st;
+    fox_status st, bad = FOX_OK;
 
     t0 = now_s();
     c->reads_at_start = fox_weights_reads(c->m->weights);
-    while (done < n) {
-        size_t chunk = n - done, cap = c->cfg.n_batch;
+    if (cap > FOX_GPU_MAX_TOKENS) cap = FOX_GPU_MAX_TOKENS;
+    while (good < n) {
+        const size_t chunk = n - good < cap ? n - good : cap;
+        if ((bad = check_chunk(c, tokens + good, chunk, (size_t)c->pos + good)) != FOX_OK) break;
+        good += chunk;
+    }
+    while (done < good) {
+        size_t left = good - done, chunk = left < cap ? left : cap;
         int last;
-        if (cap > FOX_GPU_MAX_TOKENS) cap = FOX_GPU_MAX_TOKENS;
-        if (chunk > cap) chunk = cap;
+        if (left > FOX_GPU_MAX_TOKENS && c->cfg.n_batch > FOX_GPU_MAX_TOKENS && batch_ready(c)) {
+            /* passes of about one size, whole groups of 64 tokens */
+            const size_t np = (left + c->B.cap - 1) / c->B.cap;
+            chunk = ((left + np - 1) / np + 63) & ~(size_t)63;
+            if (chunk > c->B.cap) chunk = c->B.cap;
+            if (chunk > left) chunk = left;
+        }
         last = done + chunk == n;
-        if ((size_t)c->pos + chunk > c->cfg.n_ctx)
-            return fox_fail(FOX_ERR_ARG, "forward: %zu tokens past position %u would overrun the "
-                            "%u token context", chunk, c->pos, c->cfg.n_ctx);
-        if ((st = check_tokens(c, tokens + done, chunk)) != FOX_OK) return st;
-        GPU(fox_gpu_memcpy_h2d(c->gpu, c->dtok, tokens + done, chunk * 4), "eval: tokens");
-        GPU(fox_gpu_memcpy_h2d(c->gpu, c->dpos, &c->pos, 4), "eval: position");
-        if ((st = forward_pass(c, chunk, all ? 2 : last)) != FOX_OK) return st;
-        if (all)
-            GPU(fox_gpu_memcpy_d2h(c->gpu, all + done * c->vocab, c->dlogits,
-                                   chunk * c->vocab * 4), "eval: logits");
+        if (chunk > FOX_GPU_MAX_TOKENS) {
+            if ((st = batch_eval(c, tokens + done, chunk, last, all ? all + done * c->vocab : NULL)) !=
+                FOX_OK)
+                return st;
+        } else {
+            GPU(fox_gpu_memcpy_h2d(c->gpu, c->dtok, tokens + done, chunk * 4), "eval: tokens");
+            GPU(fox_gpu_memcpy_h2d(c->gpu, c->dpos, &c->pos, 4), "eval: position");
+            if ((st = forward_pass(c, chunk, all ? 2 : last)) != FOX_OK) return st;
+            if (all)
+                GPU(fox_gpu_memcpy_d2h(c->gpu, all + done * c->vocab, c->dlogits,
+                                       chunk * c->vocab * 4), "eval: logits");
+        }
         c->pos += (uint32_t)chunk;
         done += chunk;
     }
+    /* (the check again: the message of its failure is the last one) */
+    if (bad != FOX_OK)
+        return check_chunk(c, tokens + good, n - good < cap ? n - good : cap, c->pos);
     if (!all) GPU(fox_gpu_memcpy_d2h(c->gpu, c->logits, c->dlogits, c->vocab * 4), "eval: logits");
     c->last_seconds = now_s() - t0;
     return FOX_OK;

@@ -1,0 +1,144 @@
+"""Batched passes (fox_gpu_batch_*: up to 1024 tokens) bit-identical to the
+oracle's single-token steps and to the decode kernels in passes of eight, at
+the edges of their tiles: 16 tokens and rows, 64-position score tiles, groups
+of four tiles, ragged last blocks."""
+import numpy as np
+import pytest
+
+import rustfox_amd as rf
+from rustfox_amd import synth
+from test_gpu_gemv import TYPES, bits, nonfinite_rows, oracle_gemv, same_or_both_nan, weights
+
+pytestmark = pytest.mark.gpu
+
+EPS = 1e-5
+
+
+@pytest.mark.parametrize("tname,K,Ns,M", [
+    ("TQ1_0", 256, [16], 9), ("TQ2_0", 1280, [40, 23], 17), ("TQ2_0", 2560, [130], 64),
+    ("TQ1_0", 768, [80, 16, 48], 33), ("TQ2_0", 512, [4100], 100), ("TQ2_0", 512, [9000], 200),
+    ("Q4_K", 256, [16], 9), ("Q4_K", 768, [33, 50], 20), ("Q4_K", 1024, [70], 65),
+    ("Q6_K", 256, [16], 9), ("Q6_K", 768, [29], 31), ("Q6_K", 1280, [64, 100], 48),
+    ("F16", 288, [50], 19), ("F32", 64, [9], 9),
+])
+def test_batch_gemv_bit_exact(gpu, oracle, tname, K, Ns, M):
+    rng = np.random.default_rng(K + M)
+    t = TYPES[tname]
+    Ws = [weights(rng, t, N, K) for N in Ns]
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    dx = gpu.array(x)
+    ts = [gpu.tensor(t, K, N, w) for N, w in zip(Ns, Ws)]
+    init = [rng.standard_normal((M, N)).astype(np.float32) for N in Ns]
+    outs = [gpu.array(i) for i in init]
+    gpu.batch_gemv(ts, dx, M, outs, flags=rf.GEMV_ACCUMULATE)
+    for N, W, o, i in zip(Ns, Ws, outs, init):
+        assert np.array_equal(bits(o.numpy()), bits(i + oracle_gemv(oracle, t, x, W, N, K))), N
+    if K % 256 == 0:
+        nw = rng.uniform(0.5, 1.5, K).astype(np.float32)
+        outs = [gpu.empty(M * N, np.float32) for N in Ns]
+        gpu.batch_gemv(ts, dx, M, outs, gpu.array(nw), EPS)
+        xn = np.stack([oracle.rmsnorm(r, nw, EPS) for r in x])
+        for N, W, o in zip(Ns, Ws, outs):
+            want = oracle_gemv(oracle, t, xn, W, N, K)
+            assert np.array_equal(bits(o.numpy()), bits(want).reshape(-1)), N
+
+
+@pytest.mark.parametrize("tname,K,ff,M", [("TQ1_0", 512, 96, 9), ("TQ2_0", 2560, 700, 50),
+                                          ("TQ2_0", 512, 8200, 65), ("Q4_K", 768, 40, 33)])
+def test_batch_gate_up_bit_exact(gpu, oracle, tname, K, ff, M):
+    rng = np.random.default_rng(K + ff + M)
+    t = TYPES[tname]
+    Wg, Wu = weights(rng, t, ff, K), weights(rng, t, ff, K)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    nw = rng.uniform(0.5, 1.5, K).astype(np.float32)
+    h = gpu.empty(M * ff, np.float32)
+    gpu.batch_gate_up_silu(gpu.tensor(t, K, ff, Wg), gpu.tensor(t, K, ff, Wu), gpu.array(x), M,
+                           gpu.array(nw), EPS, h)
+    got = h.numpy().reshape(M, ff)
+    for r in range(M):
+        xb = oracle.rmsnorm(x[r], nw, EPS)
+        want = oracle.silu_mul(oracle.gemv(t, xb, Wg, ff, K), oracle.gemv(t, xb, Wu, ff, K))
+        assert np.array_equal(bits(got[r]), bits(want)), f"token {r}"
+
+
+@pytest.mark.parametrize("tname", ["TQ2_0", "Q4_K", "Q6_K"])
+def test_batch_nonfinite_follows_the_reference(gpu, oracle, tname):
+    """Rows with NaN, inf and tiny values, and a weight block whose scale is
+    infinite or NaN (the conversion in place of the fused multiply-add)."""
+    rng = np.random.default_rng(5)
+    K, N, t = 512, 20, TYPES[tname]
+    W = weights(rng, t, N, K)
+    rows = [np.asarray(r, np.float32) for r in nonfinite_rows(rng, K)]
+    rows += [rng.standard_normal(K).astype(np.float32) for _ in range(9)]
+    x = np.stack(rows)
+    for special in (None, np.inf, np.nan):
+        w = W.copy()
+        if special is not None:
+            b = w.reshape(N * K // 256, -1)
+            at = {"TQ2_0": 64, "Q4_K": 0, "Q6_K": 208}[tname]
+            b[3, at:at + 2] = np.array([special], np.float16).view(np.uint8)
+        out = gpu.empty(len(rows) * N, np.float32)
+        gpu.batch_gemv([gpu.tensor(t, K, N, w)], gpu.array(x), len(rows), [out])
+        got = out.numpy().reshape(len(rows), N)
+        for r, xr in enumerate(rows):
+            assert same_or_both_nan(got[r], oracle.gemv(t, xr, w, N, K)), (special, r)
+
+
+@pytest.mark.parametrize("n_head,n_kv,hd,pos,M", [
+    (4, 2, 128, 0, 9), (8, 1, 64, 0, 70), (6, 6, 48, 61, 67), (5, 1, 128, 700, 33),
+    (4, 4, 256, 130, 20), (32, 8, 128, 0, 300), (2, 2, 20, 63, 65),
+])
+def test_batch_attention_equals_the_decode_kernels(gpu, n_head, n_kv, hd, pos, M):
+    rng = np.random.default_rng(n_head + hd + M)
+    n_ctx, kvd = pos + M, n_kv * hd
+    K, V = (rng.standard_normal((n_ctx, kvd)).astype(np.float32) for _ in range(2))
+    # (a later token's row must not reach an earlier token's sums)
+    V[-1, 0], K[-1, 0] = np.inf, np.nan
+    kc = gpu.empty(n_ctx * kvd, np.float32)
+    vc = gpu.empty((n_ctx + 3) // 4 * 4 * kvd, np.float32)
+    gpu.kv_write(kc, vc, kvd, n_ctx, 0, gpu.array(K), gpu.array(V), n_ctx)
+    q = rng.standard_normal((M, n_head * hd)).astype(np.float32)
+    out = gpu.empty(M * n_head * hd, np.float32)
+    gpu.batch_attention(out, gpu.array(q), kc, vc, n_head, n_kv, hd, M,
+                        gpu.array(np.array([pos], np.uint32)), n_ctx)
+    got = out.numpy().reshape(M, -1)
+    for t in range(0, M, 8):
+        m = min(8, M - t)
+        o = gpu.empty(m * n_head * hd, np.float32)
+        gpu.attention(o, gpu.array(q[t:t + m]), kc, vc, n_head, n_kv, hd, m,
+                      gpu.array(np.array([pos + t], np.uint32)), n_ctx, rf.ATTN_EXACT)
+        assert same_or_both_nan(got[t:t + m].reshape(-1), o.numpy()), f"tokens {t}.."
+
+
+@pytest.mark.parametrize("name,over", [
+    ("tiny-288", {}), ("tiny-512", {}),
+    ("8b", dict(n_layer=1, n_vocab=512, n_embd=512, n_ff=768, n_head=8, n_head_kv=2, head_dim=64)),
+])
+def test_prompt_equals_passes_of_eight(tmp_path, name, over):
+    """Prompts through batched passes (n_batch 32) and passes of eight: the
+    same logits, last and all, on an empty and a filled cache, in both
+    attention modes; an overrun leaves the position where passes of eight
+    leave it."""
+    s = synth.spec(name, n_ctx=160, **over)
+    path = str(tmp_path / "m.gguf")
+    synth.write_gguf(path, s)
+    ids = synth.prompt_ids(150, s.n_vocab)
+    with rf.Model(path) as m:
+        a, b = m.context(160, n_batch=32), m.context(160, n_batch=8)
+        for exact in (True, False):
+            for c in (a, b):
+                c.set_attention(exact)
+                c.reset()
+            for n0, n1 in ((0, 9), (9, 82), (82, 91), (91, 150)):
+                x, y = a.eval(ids[n0:n1]).copy(), b.eval(ids[n0:n1])
+                assert np.array_equal(bits(x), bits(y)), (exact, n0)
+        for c in (a, b):
+            c.set_attention(True)
+            c.reset()
+        assert np.array_equal(bits(a.eval_all(ids[:75])), bits(b.eval_all(ids[:75])))
+        for c in (a, b):
+            with pytest.raises(rf.FoxError):
+                c.eval(np.concatenate([ids, ids])[:100])
+            assert c.position == 75 + 80
+        a.close()
+        b.close()
