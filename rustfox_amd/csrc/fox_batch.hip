@@ -64,9 +64,24 @@ __device__ __forceinline__ int piece_off(int dl)
         const int s = e0 >> 5, o = e0 & 31;
         return ((s >> 1) * 4 + (o >> 3)) * 16 + (s & 1) * 8 + (o & 4);
     } else {
-        // quarter v = 2 half + s, sub-group c: elements 128 half + 32 c + 16 s
-        const int h = e0 >> 7, c = (e0 >> 5) & 3, s = (e0 >> 4) & 1;
-        return ((2 * h + s) * 4 + c) * 16 + (e0 & 15);
+        return e0;
+    }
+}
+
+// the same for up to eight tokens (few_gemm): the block's 2048 bytes hold, for
+// each operand load, the 16 bytes of every lane side by side; token 0's offset
+// (a token is 16 bytes on)
+template <int FMT>
+__device__ __forceinline__ int few_off(int dl)
+{
+    const int e0 = 4 * dl;
+    if (FMT == FMT_Q4K) {
+        // [sub-block quad][g][half][token]: eight elements of sub-blocks
+        // 4 qd + half and 4 qd + 2 + half
+        const int s = e0 >> 5, o = e0 & 31;
+        return (((s >> 2) * 4 + (o >> 3)) * 16 + (s & 1) * 8) * 16 + ((s >> 1) & 1) * 8 + (o & 4);
+    } else {
+        return (e0 >> 4) * 128 + (e0 & 15);                // [16-element piece][token]
     }
 }
 
@@ -131,12 +146,14 @@ __device__ __forceinline__ uint32_t wave_max_u(uint32_t v)
 
 // Token blockIdx.x: RMSNorm (NORM; src/ops.c:7-22), int8 quantisation and the
 // block sums.  512 threads; thread tid holds dwords tid + 512 r, so a wave
-// holds whole blocks (block wave + 8 r).  q: [token][K] bytes, each block's
-// 256 in piece_off order; aux: [token / 16][block][aux_quads][token % 16].
+// holds whole blocks (block wave + 8 r).  The K-quants without a norm have
+// nothing to share between blocks: there blockIdx.y takes 8 R blocks each.
+// q: [token][K] bytes, each block's 256 in piece_off order, or (few)
+// [block][2048], in few_off order; aux: [token / 16][block][aux_quads][token % 16].
 template <int FMT, bool NORM, int R>
 __global__ __launch_bounds__(512) void batch_prep(const float *__restrict__ x,
                                                   const float *__restrict__ norm_w, int K,
-                                                  size_t x_stride, float eps,
+                                                  size_t x_stride, float eps, int few,
                                                   uint8_t *__restrict__ q,
                                                   uint32_t *__restrict__ aux,
                                                   float *__restrict__ scale)
@@ -145,9 +162,10 @@ __global__ __launch_bounds__(512) void batch_prep(const float *__restrict__ x,
     __shared__ uint32_t ured[8];
     const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nb = K >> 8, nd = K >> 2;
+    const int b_first = FMT != FMT_TQ2 && !NORM ? (int)blockIdx.y * 8 * R : 0;
+    const int nb = (K >> 8) - b_first, nd = nb * 64;
     const float *xt = x + (size_t)t * x_stride;
-    const float4 *x4 = (const float4 *)xt, *w4 = (const float4 *)norm_w;
+    const float4 *x4 = (const float4 *)xt + b_first * 64, *w4 = (const float4 *)norm_w;
     float4 xv[R], wv[R];
 #pragma unroll
     for (int r = 0; r < R; r++) {
@@ -223,9 +241,11 @@ __global__ __launch_bounds__(512) void batch_prep(const float *__restrict__ x,
         qv = quant_of(am, m);
         if (tid == 0) scale[t] = qv.act;
     }
-    const int po = piece_off<FMT>(lane);
-    uint8_t *qt = q + (size_t)t * K;
-    uint32_t *at = aux + ((size_t)(t >> 4) * nb) * (aux_quads(FMT) * 4) + (t & 15);
+    const bool fw = FMT != FMT_TQ2 && few;
+    const size_t bs = fw ? 2048 : 256;
+    uint8_t *qt = q + (fw ? (size_t)t * 16 + few_off<FMT>(lane) : (size_t)t * K + piece_off<FMT>(lane)) +
+                  b_first * bs;
+    uint32_t *at = aux + ((size_t)(t >> 4) * (K >> 8) + b_first) * (aux_quads(FMT) * 4) + (t & 15);
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const int b = wave + 8 * r;
@@ -237,7 +257,7 @@ __global__ __launch_bounds__(512) void batch_prep(const float *__restrict__ x,
             qv = quant_of(am, m);
         }
         const uint32_t qd = quant4(qv, xv[r]);
-        *(uint32_t *)(qt + (size_t)b * 256 + po) = qd;
+        *(uint32_t *)(qt + b * bs) = qd;
         uint32_t *ab = at + (size_t)b * (aux_quads(FMT) * 4);
         if (FMT == FMT_TQ2) {
             const int s = wave_sum_i(__builtin_amdgcn_sdot4((int)qd, 0x01010101, 0, false));
@@ -311,23 +331,47 @@ struct RawBlock<FMT_Q4K> {
         h = *(const u4v *)(ch + 2048 + 16 * (lane & 15));
     }
 };
+// Q6_K: lane group g takes the 16 ql bytes 64 h + 16 g of half h of its row:
+// low nibbles sub-group c = g / 2 of quarter 2 h + g % 2, high nibbles c + 2
+// of the same quarter (a wave's load is a contiguous 64 bytes of 16 rows)
 template <>
 struct RawBlock<FMT_Q6K> {
-    u4v l[4], hq[4], sc;
+    u4v l[2], hq[2], sc;
     uint32_t d;
     __device__ __forceinline__ void load(const uint8_t *ch, int lane)
     {
         const int i = lane & 15, g = lane >> 4;
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int h = v >> 1, s = v & 1;
-            l[v] = *(const u4v *)(ch + 128 * i + 64 * h + 32 * (g & 1) + 16 * s);
-            hq[v] = *(const u4v *)(ch + 2048 + 64 * i + 32 * h + 16 * s);
+        for (int h = 0; h < 2; h++) {
+            l[h] = *(const u4v *)(ch + 128 * i + 64 * h + 16 * g);
+            hq[h] = *(const u4v *)(ch + 2048 + 64 * i + 32 * h + 16 * (g & 1));
         }
         sc = *(const u4v *)(ch + 3072 + 16 * i);
         d = *(const unsigned short *)(ch + 3328 + 2 * i);
     }
 };
+
+// the signed bytes 4 (q - 32) of half h (the 6-bit value shifted up, its top
+// bit flipped; the factor is taken out of the integer sums): hi = 0 the low
+// nibbles' sub-groups, 1 the high ones'
+__device__ __forceinline__ v4i q6_bytes(const RawBlock<FMT_Q6K> &w, int h, int hi, int g)
+{
+    const int sh = 2 * (g >> 1) + 4 * hi;
+    v4i r;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t lo = (hi ? w.l[h][i] >> 2 : w.l[h][i] << 2) & 0x3c3c3c3cu;
+        const uint32_t up = ((w.hq[h][i] >> sh) & 0x03030303u) << 6;
+        r[i] = (int)((lo | up) ^ 0x80808080u);
+    }
+    return r;
+}
+
+// scale byte n of the row, signed
+__device__ __forceinline__ int q6_scale(const u4v &sc, int n)
+{
+    return (int)(sc[n >> 2] << (24 - 8 * (n & 3))) >> 24;
+}
 
 __device__ __forceinline__ v4i mfma64(v4i a, v4i b, v4i c)
 {
@@ -452,54 +496,47 @@ __device__ __forceinline__ void block_terms(const RawBlock<FMT> (&raw)[R], const
         if (!odd) run(std::true_type{});
         else run(std::false_type{});
     } else {
-        // Q6_K: quarter v's four 16-element sub-groups are the four lane
-        // groups' bytes; sub-group c alone is the product with the other
-        // lane groups' weights zeroed.  Values q - 32 as signed bytes, times
-        // four (the 6-bit value with its top bit flipped, shifted up), the
-        // factor taken out of the integer sum.
+        // Q6_K: an operand's four lane groups are four 16-element sub-groups
+        // (group gg: quarter 2h + gg % 2, sub-group gg / 2, + 2 for the high
+        // nibbles); one alone is the product with the other groups' weights
+        // zeroed.
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int h = v >> 1, s = v & 1;
-            v4i w[R][4];
-            int sc[R][4];
+        for (int h = 0; h < 2; h++) {
+            v4i w[R][2];
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                v4i a;
+            for (int r = 0; r < R; r++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const uint32_t L = raw[r].l[v][i], H = raw[r].hq[v][i];
-                    const uint32_t lo = ((g < 2 ? L : L >> 4) & 0x0f0f0f0fu) << 2;
-                    const uint32_t hi = ((H >> (2 * g)) & 0x03030303u) << 6;
-                    a[i] = (int)((lo | hi) ^ 0x80808080u);
-                }
-#pragma unroll
-                for (int c4 = 0; c4 < 4; c4++) {
-                    const int m = g == c4 ? -1 : 0;
-                    w[r][c4] = v4i{a[0] & m, a[1] & m, a[2] & m, a[3] & m};
-                    // scale 8h + s + 2 c4 (signed byte)
-                    const int byte = 8 * h + s + 2 * c4;
-                    sc[r][c4] = (int)(raw[r].sc[byte >> 2] << (24 - 8 * (byte & 3))) >> 24;
-                }
-            }
+                for (int hi = 0; hi < 2; hi++) w[r][hi] = q6_bytes(raw[r], h, hi, g);
 #pragma unroll
             for (int c = 0; c < C; c++) {
-                v4i a = *(const v4i *)(bt + c * 16 * B_ROW + v * 64);
+                v4i x[2];
+                x[0] = *(const v4i *)(bt + c * 16 * B_ROW + h * 128);
+                x[1] = *(const v4i *)(bt + c * 16 * B_ROW + h * 128 + 64);
                 const f4v as = ((const f4v *)ax)[c * 4 + g];
-                asm volatile("" : "+v"(a));                // (see below)
+                asm volatile("" : "+v"(x[0]), "+v"(x[1]));    // (see below)
 #pragma unroll
                 for (int r = 0; r < R; r++) {
                     const v4i zero = {0, 0, 0, 0};
-                    v4i part = zero;
+                    v4i part[2] = {zero, zero};
 #pragma unroll
-                    for (int c4 = 0; c4 < 4; c4++) {
-                        const v4i D = mfma64(a, w[r][c4], zero);
+                    for (int gg = 0; gg < 4; gg++) {
+                        const int m = g == gg ? -1 : 0;
 #pragma unroll
-                        for (int k = 0; k < 4; k++) part[k] += __mul24(sc[r][c4], D[k]);
+                        for (int hi = 0; hi < 2; hi++) {
+                            const v4i wm = {w[r][hi][0] & m, w[r][hi][1] & m, w[r][hi][2] & m,
+                                            w[r][hi][3] & m};
+                            const v4i D = mfma64(x[hi], wm, zero);
+                            const int sc = q6_scale(raw[r].sc, 8 * h + (gg & 1) + 2 * ((gg >> 1) + 2 * hi));
+#pragma unroll
+                            for (int k = 0; k < 4; k++) part[gg & 1][k] += __mul24(sc, D[k]);
+                        }
                     }
                     const float d = half_bits_to_float(raw[r].d);
 #pragma unroll
-                    for (int k = 0; k < 4; k++)
-                        acc[r][c][k] = acc[r][c][k] + as[k] * d * (float)(part[k] >> 2);
+                    for (int s = 0; s < 2; s++)
+#pragma unroll
+                        for (int k = 0; k < 4; k++)
+                            acc[r][c][k] = acc[r][c][k] + as[k] * d * (float)(part[s][k] >> 2);
                 }
                 // (left to itself the compiler issues every matrix product of
                 // the block first and needs 256 more registers for them: the
@@ -659,6 +696,214 @@ __global__ __launch_bounds__(BT_THREADS, 2) void batch_gemm(BatchArgs a)
     }
 }
 
+// ------------------------------------------------- few tokens, K-quants
+
+// K-quant matrices against 2 .. 8 tokens: a workgroup per 16-row tile, its
+// waves take the blocks in turn (block wave + KS r) and write each block's
+// float terms to one of two LDS buffers, and 128 lanes (row, token) add them
+// in block order after each round (one barrier a round).  The weights are
+// the whole traffic, so what counts is bytes in flight and few instructions
+// per block:
+//   * the activations of a block are used once, so they go from L2 straight
+//     to registers, in the operand's layout; their sums and scales are in
+//     LDS (as register loads they cost a quarter of the vector memory time
+//     and the fourth wave per SIMD);
+//   * the MFMA's 16 operand rows are 8 tokens x 2: Q4_K's sub-blocks 2p and
+//     2p + 1 (a lane's 8 low-nibble and 8 high-nibble weights; the other
+//     half's activations zero), or Q6_K's quarters 2h and 2h + 1 (one
+//     sub-group at a time, the other lane groups' activations zero), so a lane
+//     forms the terms of its half only.
+// Q4_K 14336 x 4096, 8 tokens: 55.2 us in the workgroup-of-four kernel this
+// replaces.
+template <int FMT>
+struct FewTerms;                        // one lane's terms of a block, per token k
+template <>
+struct FewTerms<FMT_Q4K> { f4v t[4]; }; // sub-blocks 2p + half, p = 0 .. 3
+typedef float f2v __attribute__((ext_vector_type(2)));
+template <>
+struct FewTerms<FMT_Q6K> { f2v t[4]; }; // quarters half, 2 + half
+
+template <int FMT, int KS, int EPI>
+__global__ __launch_bounds__(KS * 64, FMT == FMT_Q4K ? 4 : 3) void few_gemm(BatchArgs a)
+{
+    constexpr int CH = batch_chunk(FMT), AQ = aux_quads(FMT);
+    typedef decltype(FewTerms<FMT>::t[0]) TV0;
+    typedef std::remove_reference_t<TV0> TV;
+    constexpr int NT = FMT == FMT_Q4K ? 4 : 2;             // terms per half
+    __shared__ TV terms[2][KS][2][8][16];                  // [buffer][slot][half][token][row]
+    extern __shared__ f4v axl[];                           // [block][AQ / 4][2]: aux of tokens 0 .. 7
+    const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nb = a.nb;
+    const int half = g >> 1, t4 = 4 * (g & 1);             // of this lane's sums: half, tokens t4 ..
+    const int ih = j >> 3;                                 // of its operand row
+    // (tokens past M: bytes that no token wrote, products that nothing reads)
+    const uint8_t *qrow = a.q + (FMT == FMT_Q4K ? lane : g * 8 + (j & 7)) * 16;
+    const int crow = tid & 15, ct = tid >> 4;              // of the combine: row, token (tid < 128)
+    float y[EPI == BE_SILU ? 2 : 1];
+    int tile = blockIdx.x, s = 0;
+    if (EPI != BE_SILU) {
+        while (s + 1 < a.nseg && tile >= a.tile_start[s + 1]) s++;
+        tile -= a.tile_start[s];
+    }
+    const int ns = (nb + KS - 1) / KS;
+    // (the first aux quads are requested before the weights and stored after
+    // those are under way)
+    const int nax = nb * (AQ / 2);
+    f4v ax0[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int i = min(tid + k * KS * 64, nax - 1);
+        ax0[k] = ((const f4v *)a.aux)[(i >> 1) * 4 + (i & 1)];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int it = 0; it < (EPI == BE_SILU ? 2 : 1); it++) {
+        const uint8_t *wp = a.w[EPI == BE_SILU ? it : s] + (size_t)tile * nb * CH;
+        struct Unit {
+            RawBlock<FMT> w;
+            u4v q[FMT == FMT_Q4K ? 2 : 4];
+        };
+        auto load = [&](int r, Unit &u) __attribute__((always_inline)) {
+            const int b = min(r * KS + wave, nb - 1);
+            u.w.load(wp + (size_t)b * CH, lane);
+            // Q4_K: loads of 1 KB, two operands each; Q6_K: of 512 bytes (the
+            // two halves' rows the same)
+#pragma unroll
+            for (int p = 0; p < (FMT == FMT_Q4K ? 2 : 4); p++)
+                u.q[p] = *(const u4v *)(qrow + (size_t)b * 2048 + p * (FMT == FMT_Q4K ? 1024 : 512));
+        };
+        auto compute = [&](int r, const Unit &u, FewTerms<FMT> &o) __attribute__((always_inline)) {
+            const f4v *ax = axl + min(r * KS + wave, nb - 1) * (AQ / 2) + (g & 1);
+            const f4v as = ax[AQ / 2 - 2];
+            if constexpr (FMT == FMT_Q4K) {
+                const uint32_t s0 = u.w.h[1], s1 = u.w.h[2], s2 = u.w.h[3];
+                // the scales and minima of sub-blocks half, half + 2 (bytes 0, 2)
+                const int sh = 8 * half;
+                const uint32_t sc[2] = {(s0 & 0x3f3f3f3fu) >> sh,
+                                        ((s2 & 0x0f0f0f0fu) | (((s0 >> 6) & 0x03030303u) << 4)) >> sh};
+                const uint32_t mn[2] = {(s1 & 0x3f3f3f3fu) >> sh,
+                                        (((s2 >> 4) & 0x0f0f0f0fu) | (((s1 >> 6) & 0x03030303u) << 4)) >> sh};
+                const float d = half_bits_to_float(u.w.h[0] & 0xffffu);
+                const float dmin = half_bits_to_float(u.w.h[0] >> 16);
+                const uint32_t m0 = ih ? 0u : ~0u, m1 = ~m0;
+                const v4i magic = {MAGIC_BITS, MAGIC_BITS, MAGIC_BITS, MAGIC_BITS};
+                auto run = [&](auto finite) __attribute__((always_inline)) {
+#pragma unroll
+                for (int p = 0; p < 4; p++) {
+                    const uint32_t a0 = p < 2 ? u.w.q0[2 * p] : u.w.q1[2 * p - 4];
+                    const uint32_t a1 = p < 2 ? u.w.q0[2 * p + 1] : u.w.q1[2 * p - 3];
+                    const v4i w = {(int)(a0 & 0x0f0f0f0fu), (int)(a1 & 0x0f0f0f0fu),
+                                   (int)((a0 >> 4) & 0x0f0f0f0fu), (int)((a1 >> 4) & 0x0f0f0f0fu)};
+                    const uint32_t x0 = u.q[p >> 1][2 * (p & 1)], x1 = u.q[p >> 1][2 * (p & 1) + 1];
+                    const v4i x = {(int)(x0 & m0), (int)(x1 & m0), (int)(x0 & m1), (int)(x1 & m1)};
+                    const v4i D = mfma64(x, w, magic);
+                    const f4v sq = ax[2 * (2 * p + half)];
+                    const float A = d * (float)((sc[p >> 1] >> (16 * (p & 1))) & 0xffu);
+                    const float B = dmin * (float)((mn[p >> 1] >> (16 * (p & 1))) & 0xffu);
+                    const float na = -MAGIC_F * A;
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const float pr = decltype(finite)::value
+                                             ? __builtin_fmaf(A, __int_as_float(D[k]), na)
+                                             : A * (float)(D[k] - MAGIC_BITS);
+                        o.t[k][p] = as[k] * (pr - B * sq[k]);
+                    }
+                }
+                };
+                if (!any_nonfinite(d)) run(std::true_type{});
+                else run(std::false_type{});
+            } else {
+                const float d = half_bits_to_float(u.w.d);
+                f4v dd;
+#pragma unroll
+                for (int k = 0; k < 4; k++) dd[k] = as[k] * d;
+                // sub-groups g / 2 = 0 and 1 of quarter 2h + ih
+                const uint32_t m0 = g == ih ? ~0u : 0u, m1 = g == 2 + ih ? ~0u : 0u;
+                const v4i zero = {0, 0, 0, 0};
+                const u4v sc = {u.w.sc[0] >> 8 * half, u.w.sc[1] >> 8 * half, u.w.sc[2] >> 8 * half,
+                                u.w.sc[3] >> 8 * half};
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    v4i part = zero;
+#pragma unroll
+                    for (int hi = 0; hi < 2; hi++) {
+                        const v4i w = q6_bytes(u.w, h, hi, g);
+                        const u4v q = u.q[2 * h + hi];
+                        const v4i x0 = {(int)(q[0] & m0), (int)(q[1] & m0), (int)(q[2] & m0), (int)(q[3] & m0)};
+                        const v4i x1 = {(int)(q[0] & m1), (int)(q[1] & m1), (int)(q[2] & m1), (int)(q[3] & m1)};
+                        const v4i D0 = mfma64(x0, w, zero), D1 = mfma64(x1, w, zero);
+                        // scales 8h + half + 4 hi (sub-group 2 hi) and + 2
+                        const int c0 = q6_scale(sc, 8 * h + 4 * hi), c1 = q6_scale(sc, 8 * h + 4 * hi + 2);
+#pragma unroll
+                        for (int k = 0; k < 4; k++)
+                            part[k] += __mul24(c0, D0[k]) + __mul24(c1, D1[k]);
+                    }
+#pragma unroll
+                    for (int k = 0; k < 4; k++) o.t[k][h] = dd[k] * (float)(part[k] >> 2);
+                }
+            }
+        };
+        float acc = 0.0f;
+        auto combine = [&](int r) __attribute__((always_inline)) {
+            if (tid >= 128) return;
+#pragma unroll
+            for (int w = 0; w < KS; w++) {
+                if (r * KS + w >= nb) break;               // (uniform)
+                const TV h0 = terms[r & 1][w][0][ct][crow], h1 = terms[r & 1][w][1][ct][crow];
+#pragma unroll
+                for (int p = 0; p < NT; p++) {
+                    acc = acc + h0[p];
+                    acc = acc + h1[p];
+                }
+            }
+        };
+        auto round = [&](int r, Unit &u) __attribute__((always_inline)) {
+            if (r < ns) {                                  // (uniform)
+                FewTerms<FMT> o;
+                compute(r, u, o);
+#pragma unroll
+                for (int k = 0; k < 4; k++) terms[r & 1][wave][half][t4 + k][j] = o.t[k];
+            }
+            load(r + 2, u);
+            // (the loads stay here and in this order: a unit's wait then
+            // leaves the unit after it in flight)
+            __builtin_amdgcn_sched_barrier(0);
+            __syncthreads();
+            combine(r);
+        };
+        // two units in flight; a buffer is written again two rounds later,
+        // past the barrier that its combine precedes
+        Unit u0, u1;
+        load(0, u0);
+        __builtin_amdgcn_sched_barrier(0);
+        load(1, u1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (it == 0) {
+#pragma unroll
+            for (int k = 0; k < 2; k++)
+                if (tid + k * KS * 64 < nax) axl[tid + k * KS * 64] = ax0[k];
+            for (int i = tid + 2 * KS * 64; i < nax; i += KS * 64)
+                axl[i] = ((const f4v *)a.aux)[(i >> 1) * 4 + (i & 1)];
+            __syncthreads();
+        }
+        // (always both: a way out between them would leave the compiler
+        // unsure at the loop's head how many loads follow the first unit's)
+        for (int r = 0; r < ns; r += 2) {
+            round(r, u0);
+            round(r + 1, u1);
+        }
+        y[it] = acc;
+        if (EPI == BE_SILU) __syncthreads();               // (the buffers start over)
+    }
+    if (tid >= 128 || ct >= a.M) return;
+    const int row = tile * 16 + crow;
+    if (row >= a.n_rows[s]) return;
+    float *o = a.out[s] + (size_t)ct * a.out_stride[s] + row;
+    if (EPI == BE_SILU) *o = fox_div(y[0], 1.0f + fox_expf(-y[0])) * y[EPI == BE_SILU];
+    else *o = (a.flags & FOX_GPU_GEMV_ACCUMULATE) ? *o + y[0] : y[0];
+}
+
 // ------------------------------------------------------------------ host
 
 static size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -672,16 +917,22 @@ struct BatchWs {
 };
 
 // the prepared operand of M tokens of width K in the context's workspace
-static fox_gpu_status batch_carve(fox_gpu_ctx *ctx, int fmt, size_t K, size_t M, BatchWs *w)
+// (fixed: memory that holds it, in place of the context's)
+static fox_gpu_status batch_carve(fox_gpu_ctx *ctx, int fmt, size_t K, size_t M, uint8_t *fixed,
+                                  BatchWs *w)
 {
-    const size_t nq = up256(M * K);
+    // (few_gemm's operand has room for eight tokens whatever M is)
+    const size_t nq = up256((M < FOX_GPU_MAX_TOKENS ? FOX_GPU_MAX_TOKENS : M) * K);
     const size_t na = up256((M + 15) / 16 * (K / 256) * (size_t)aux_quads(fmt) * 16);
     const size_t ns = up256(M * 4);
-    fox_gpu_status st = fox_ws_reserve(ctx, nq + na + ns);
-    if (st) return st;
-    w->q = ctx->ws;
-    w->aux = (uint32_t *)(ctx->ws + nq);
-    w->scale = (float *)(ctx->ws + nq + na);
+    if (!fixed) {
+        fox_gpu_status st = fox_ws_reserve(ctx, nq + na + ns);
+        if (st) return st;
+        fixed = ctx->ws;
+    }
+    w->q = fixed;
+    w->aux = (uint32_t *)(fixed + nq);
+    w->scale = (float *)(fixed + nq + na);
     return FOX_GPU_OK;
 }
 
@@ -719,6 +970,15 @@ static const void *gemm_kernel(int fmt, int R, int C, int epi)
     return gemm_c<FMT_Q6K, 1, BE_STORE>(C);
 }
 
+// eight waves per row tile where four would leave the chip part empty
+static const void *few_kernel(int fmt, bool wide, int epi)
+{
+#define FOX_FEW(f, e) (wide ? (const void *)few_gemm<f, 8, e> : (const void *)few_gemm<f, 4, e>)
+    if (fmt == FMT_Q4K) return epi == BE_SILU ? FOX_FEW(FMT_Q4K, BE_SILU) : FOX_FEW(FMT_Q4K, BE_STORE);
+    return epi == BE_SILU ? FOX_FEW(FMT_Q6K, BE_SILU) : FOX_FEW(FMT_Q6K, BE_STORE);
+#undef FOX_FEW
+}
+
 static fox_gpu_status batch_check(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor *const *ws,
                                   const float *x, size_t x_stride, size_t M, float *const *outs,
                                   const size_t *out_strides)
@@ -747,26 +1007,30 @@ static fox_gpu_status batch_check(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tens
 static fox_gpu_status batch_run(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor *const *ws,
                                 const float *x, size_t x_stride, size_t M, const float *norm_w,
                                 float eps, float *const *outs, const size_t *out_strides,
-                                unsigned flags, int epi)
+                                unsigned flags, int epi, uint8_t *fixed = nullptr)
 {
     const int fmt = fmt_of(ws[0]->type);
     const size_t K = (size_t)ws[0]->ne0;
     // (Q6_K gate/up pairs: two such tiles per wave do not fit its registers)
-    if (fmt < 0 || (fmt == FMT_Q6K && epi == BE_SILU) || K == 0 || K % 256 || K > 2048 * PREP_MAX_R || x_stride % 4 ||
+    if (fmt < 0 || (fmt == FMT_Q6K && epi == BE_SILU && M > FOX_GPU_MAX_TOKENS) || K == 0 || K % 256 || K > 2048 * PREP_MAX_R || x_stride % 4 ||
         ((uintptr_t)x | (uintptr_t)norm_w) % 16)
         return FOX_GPU_ERR_UNSUPPORTED;
     BatchWs w;
-    fox_gpu_status st = batch_carve(ctx, fmt, K, M, &w);
+    fox_gpu_status st = batch_carve(ctx, fmt, K, M, fixed, &w);
     if (st) return st;
     {
         const int r = (int)((K / 4 + 511) / 512);
         const void *k = fmt == FMT_TQ2 ? prep_fmt<FMT_TQ2>(norm_w != nullptr, r)
                       : fmt == FMT_Q4K ? prep_fmt<FMT_Q4K>(norm_w != nullptr, r)
                                        : prep_fmt<FMT_Q6K>(norm_w != nullptr, r);
-        int iK = (int)K;
-        void *args[] = {(void *)&x, (void *)&norm_w, (void *)&iK, (void *)&x_stride, (void *)&eps,
+        int iK = (int)K, few = fmt != FMT_TQ2 && M <= FOX_GPU_MAX_TOKENS;
+        void *args[] = {(void *)&x, (void *)&norm_w, (void *)&iK, (void *)&x_stride, (void *)&eps, (void *)&few,
                         (void *)&w.q, (void *)&w.aux, (void *)&w.scale};
-        hipError_t e = hipLaunchKernel(k, dim3((unsigned)M), dim3(512), args, 0, ctx->stream);
+        const bool split = fmt != FMT_TQ2 && !norm_w;      // (blocks apart on grid y, R = 1)
+        if (split) k = fmt == FMT_Q4K ? (const void *)batch_prep<FMT_Q4K, false, 1>
+                                      : (const void *)batch_prep<FMT_Q6K, false, 1>;
+        hipError_t e = hipLaunchKernel(k, dim3((unsigned)M, split ? (unsigned)r : 1u), dim3(512), args,
+                                       0, ctx->stream);
         if (e != hipSuccess) return fox_hip_fail(e, "batch: prepare");
         FOX_LAUNCHED("batch: prepare");
     }
@@ -789,6 +1053,20 @@ static fox_gpu_status batch_run(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor
         tiles += (int)ws[i]->n_tiles;
     }
     a.tile_start[n] = tiles;
+    if (fmt != FMT_TQ2 && M <= FOX_GPU_MAX_TOKENS) {
+        // K-quants, up to eight tokens: a workgroup per row tile
+        const int nt = epi == BE_SILU ? a.tile_start[1] : tiles;
+        const void *k = few_kernel(fmt, nt < 512, epi);
+        void *args[] = {(void *)&a};
+        const size_t lds = K / 256 * (size_t)aux_quads(fmt) * 8;
+        if (lds > 64 * 1024) return FOX_GPU_ERR_UNSUPPORTED;
+        hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e == hipSuccess)
+            e = hipLaunchKernel(k, dim3((unsigned)nt), dim3(nt < 512 ? 512 : 256), args, lds, ctx->stream);
+        if (e != hipSuccess) return fox_hip_fail(e, "batch: product");
+        FOX_LAUNCHED("batch: product");
+        return FOX_GPU_OK;
+    }
     // token groups of C 16-token tiles, as even as they come at C <= 4
     const int mt = (int)((M + 15) / 16), n_tg = (mt + 3) / 4, C = (mt + n_tg - 1) / n_tg;
     a.n_tg = (mt + C - 1) / C;
@@ -808,6 +1086,17 @@ static fox_gpu_status batch_run(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor
     if (e != hipSuccess) return fox_hip_fail(e, "batch: product");
     FOX_LAUNCHED("batch: product");
     return FOX_GPU_OK;
+}
+
+// fox_gpu_gemv's and fox_gpu_gemv_multi's K-quant products of 2 to
+// FOX_GPU_MAX_TOKENS tokens (arguments checked by the caller; the prepared
+// operand is smaller than gemv_blocks's, which `fixed` is sized for)
+fox_gpu_status fox_few_gemv(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor *const *ws,
+                            const float *x, size_t x_stride, size_t M, float *const *outs,
+                            const size_t *out_strides, unsigned flags, uint8_t *fixed)
+{
+    return batch_run(ctx, n, ws, x, x_stride, M, nullptr, 0.0f, outs, out_strides, flags, BE_STORE,
+                     fixed);
 }
 
 extern "C" fox_gpu_status fox_gpu_batch_gemv(fox_gpu_ctx *ctx, size_t n,

@@ -765,9 +765,12 @@ static fox_gpu_status gemv_launch_ws(fox_gpu_ctx *ctx, size_t n, const fox_gpu_t
                             "scratch; the fixed scratch holds %zu", M, K, fox_type_name(type),
                             need, fixed_cap);
         act_layout(fmt, K, M, fixed_ws, &w);
-    } else if ((st = carve(ctx, fmt, K, M, &w))) {
-        return st;
     }
+    if (x && !sums && M > 1 && fmt != FMT_TQ2) {
+        st = fox_few_gemv(ctx, n, ws, x, x_stride, M, outs, out_strides, flags, fixed_ws);
+        if (st != FOX_GPU_ERR_UNSUPPORTED) return st;
+    }
+    if (!fixed_ws && (st = carve(ctx, fmt, K, M, &w))) return st;
     if ((st = launch_prep(ctx, fmt, x, x_stride, q, scale, K, M, w, w.q, w.scale))) return st;
 
     Segs sg;

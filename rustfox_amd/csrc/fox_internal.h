@@ -199,3 +199,8 @@ fox_gpu_status fox_float_gemv(fox_gpu_ctx *ctx, const fox_gpu_tensor *w, const f
 fox_gpu_status fox_attn_softmax(fox_gpu_ctx *ctx, float *att, size_t att_stride, const float *tmax,
                                 int n_tiles, int n_head, const uint32_t *pos, int t_base, int n_ctx,
                                 int M);
+// K-quant products of several tokens (fox_batch.hip); FOX_GPU_ERR_UNSUPPORTED
+// (no error recorded) for inputs not 16-byte aligned and very wide rows
+fox_gpu_status fox_few_gemv(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor *const *ws,
+                            const float *x, size_t x_stride, size_t M, float *const *outs,
+                            const size_t *out_strides, unsigned flags, uint8_t *fixed);

@@ -313,18 +313,35 @@ static int same_type(const fox_gpu_tensor *a, const fox_gpu_tensor *b)
     return ta == tb && ka == kb;
 }
 
-/* y_i = W_i x for matrices sharing the input: one launch for each run of
- * equal types (q/k/v, gate/up) */
+/* y_i = W_i rmsnorm(x, norm_w) for matrices sharing the input, xb scratch for
+ * the normed rows: one product for each run of equal types (q/k/v, gate/up),
+ * the norm in its input stage where the type has one */
 static fox_status project_group(fox_context *c, size_t n, const fox_gpu_tensor *const *ws,
-                                const float *x, size_t x_stride, size_t M, float *const *outs,
-                                const size_t *strides)
+                                const float *x, float *xb, size_t M, const float *norm_w,
+                                float *const *outs, const size_t *strides)
 {
+    const float eps = c->m->info.rms_eps;
     size_t i = 0;
+    int normed = 0;
     while (i < n) {
         size_t j = i + 1;
+        fox_gpu_status gs = FOX_GPU_ERR_UNSUPPORTED;
         while (j < n && same_type(ws[i], ws[j])) j++;
-        GPU(fox_gpu_gemv_multi(c->gpu, j - i, ws + i, x, x_stride, M, outs + i, strides + i, 0),
-            "forward: projection");
+        if (M > 1)
+            gs = fox_gpu_batch_gemv_rmsnorm(c->gpu, j - i, ws + i, x, c->d, M, norm_w, eps, outs + i,
+                                            strides + i, 0);
+        if (gs == FOX_GPU_ERR_UNSUPPORTED) {
+            if (!normed)
+                GPU(fox_gpu_rmsnorm(c->gpu, xb, c->wide, x, c->d, norm_w, c->d, M, eps),
+                    "forward: norm");
+            normed = 1;
+            gs = M > FOX_GPU_MAX_TOKENS
+                     ? fox_gpu_batch_gemv(c->gpu, j - i, ws + i, xb, c->wide, M, outs + i,
+                                          strides + i, 0)
+                     : fox_gpu_gemv_multi(c->gpu, j - i, ws + i, xb, c->wide, M, outs + i,
+                                          strides + i, 0);
+        }
+        if (gs != FOX_GPU_OK) return fox_gpu_failed(gs, "forward: projection");
         i = j;
     }
     return FOX_OK;
@@ -407,9 +424,8 @@ static fox_status forward_pass(fox_context *c, size_t M, int want_logits)
                               D->attn_norm, mi->rms_eps, c->q, c->nq, c->rc, c->rs, c->dpos,
                               c->cfg.n_ctx, c->kc + l * kvl, c->vc + l * vl, c->hd);
         if (gs == FOX_GPU_ERR_UNSUPPORTED) {
-            GPU(fox_gpu_rmsnorm(c->gpu, c->xb, c->wide, c->x, c->d, D->attn_norm, c->d, M,
-                                mi->rms_eps), "forward: attn_norm");
-            if ((st = project_group(c, 3, qkv, c->xb, c->wide, M, qkv_out, qkv_str)) != FOX_OK)
+            if ((st = project_group(c, 3, qkv, c->x, c->xb, M, D->attn_norm, qkv_out, qkv_str)) !=
+                FOX_OK)
                 return st;
             GPU(fox_gpu_rope_store(c->gpu, c->q, c->nq, c->k, c->nkv, c->v, c->nkv, mi->n_head,
                                    mi->n_head_kv, c->hd, M, c->rc, c->rs, c->dpos, c->cfg.n_ctx,
@@ -424,10 +440,12 @@ static fox_status forward_pass(fox_context *c, size_t M, int want_logits)
                          FOX_GPU_GEMV_ACCUMULATE), "forward: attn_output");
         gs = fox_gpu_gate_up_silu(c->gpu, D->ffn_gate, D->ffn_up, c->x, c->d, M, D->ffn_norm,
                                   mi->rms_eps, c->hb, c->ff);
+        if (gs == FOX_GPU_ERR_UNSUPPORTED && M > 1)        /* (K-quants, several tokens) */
+            gs = fox_gpu_batch_gate_up_silu(c->gpu, D->ffn_gate, D->ffn_up, c->x, c->d, M,
+                                            D->ffn_norm, mi->rms_eps, c->hb, c->ff);
         if (gs == FOX_GPU_ERR_UNSUPPORTED) {
-            GPU(fox_gpu_rmsnorm(c->gpu, c->xb, c->wide, c->x, c->d, D->ffn_norm, c->d, M,
-                                mi->rms_eps), "forward: ffn_norm");
-            if ((st = project_group(c, 2, gu, c->xb, c->wide, M, gu_out, gu_str)) != FOX_OK)
+            if ((st = project_group(c, 2, gu, c->x, c->xb, M, D->ffn_norm, gu_out, gu_str)) !=
+                FOX_OK)
                 return st;
             GPU(fox_gpu_silu_mul(c->gpu, c->hb, c->hb2, c->ff, M, c->ff), "forward: swiglu");
         } else if (gs != FOX_GPU_OK) {
@@ -442,35 +460,6 @@ static fox_status forward_pass(fox_context *c, size_t M, int want_logits)
         const size_t rows = want_logits == 2 ? M : 1;
         return head(c, c->x + (M - rows) * c->d, c->xb, rows, c->dlogits);
     }
-}
-
-/* y_i = W_i rmsnorm(x, norm_w) of a batched pass, one product for each run
- * of equal types */
-static fox_status batch_project(fox_context *c, size_t n, const fox_gpu_tensor *const *ws,
-                                size_t M, const float *norm_w, float *const *outs,
-                                const size_t *strides)
-{
-    const float eps = c->m->info.rms_eps;
-    size_t i = 0;
-    int normed = 0;
-    while (i < n) {
-        size_t j = i + 1;
-        fox_gpu_status gs;
-        while (j < n && same_type(ws[i], ws[j])) j++;
-        gs = fox_gpu_batch_gemv_rmsnorm(c->gpu, j - i, ws + i, c->B.x, c->d, M, norm_w, eps,
-                                        outs + i, strides + i, 0);
-        if (gs == FOX_GPU_ERR_UNSUPPORTED) {
-            if (!normed)
-                GPU(fox_gpu_rmsnorm(c->gpu, c->B.xb, c->wide, c->B.x, c->d, norm_w, c->d, M, eps),
-                    "forward: norm");
-            normed = 1;
-            gs = fox_gpu_batch_gemv(c->gpu, j - i, ws + i, c->B.xb, c->wide, M, outs + i,
-                                    strides + i, 0);
-        }
-        if (gs != FOX_GPU_OK) return fox_gpu_failed(gs, "forward: projection");
-        i = j;
-    }
-    return FOX_OK;
 }
 
 static fox_status batch_add(fox_context *c, const fox_gpu_tensor *w, const float *x, size_t stride,
@@ -504,7 +493,8 @@ static fox_status batch_pass(fox_context *c, size_t M)
             const fox_gpu_tensor *qkv[3] = { D->attn_q, D->attn_k, D->attn_v };
             float *out[3] = { B->q, B->k, B->v };
             size_t str[3] = { c->nq, c->nkv, c->nkv };
-            if ((st = batch_project(c, 3, qkv, M, D->attn_norm, out, str)) != FOX_OK) return st;
+            if ((st = project_group(c, 3, qkv, B->x, B->xb, M, D->attn_norm, out, str)) != FOX_OK)
+                return st;
         }
         GPU(fox_gpu_batch_rope_store(c->gpu, B->q, c->nq, B->k, c->nkv, B->v, c->nkv, mi->n_head,
                                      mi->n_head_kv, c->hd, M, c->rc, c->rs, B->pos, c->cfg.n_ctx,
@@ -530,7 +520,8 @@ static fox_status batch_pass(fox_context *c, size_t M)
             const fox_gpu_tensor *gu[2] = { D->ffn_gate, D->ffn_up };
             float *out[2] = { B->hb, B->hb2 };
             size_t str[2] = { c->ff, c->ff };
-            if ((st = batch_project(c, 2, gu, M, D->ffn_norm, out, str)) != FOX_OK) return st;
+            if ((st = project_group(c, 2, gu, B->x, B->xb, M, D->ffn_norm, out, str)) != FOX_OK)
+                return st;
             GPU(fox_gpu_silu_mul(c->gpu, B->hb, B->hb2, c->ff, M, c->ff), "forward: swiglu");
         } else if (gs != FOX_GPU_OK) {
             return fox_gpu_failed(gs, "forward: gate/up");

@@ -43,7 +43,29 @@ def test_batch_gemv_bit_exact(gpu, oracle, tname, K, Ns, M):
             assert np.array_equal(bits(o.numpy()), bits(want).reshape(-1)), N
 
 
-@pytest.mark.parametrize("tname,K,ff,M", [("TQ1_0", 512, 96, 9), ("TQ2_0", 2560, 700, 50),
+@pytest.mark.parametrize("tname", ["Q4_K", "Q6_K"])
+@pytest.mark.parametrize("K,N,M", [(256, 16, 2), (1024, 40, 3), (2304, 8300, 8), (5376, 100, 5),
+                                   (14336, 33, 7)])
+def test_few_tokens_kquants_bit_exact(gpu, oracle, tname, K, N, M):
+    """Two to eight tokens: fewer, as many and more blocks than a workgroup's
+    four or eight waves, through fox_gpu_gemv and the normed batched call."""
+    rng = np.random.default_rng(K + M)
+    t = TYPES[tname]
+    W = np.concatenate([weights(rng, t, min(N, 64), K)] * -(-N // 64))[:N * synth.row_bytes(t, K)]
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    dw, dx = gpu.tensor(t, K, N, W), gpu.array(x)
+    init = rng.standard_normal((M, N)).astype(np.float32)
+    out = gpu.array(init)
+    gpu.gemv(dw, dx, M, out, flags=rf.GEMV_ACCUMULATE)
+    assert np.array_equal(bits(out.numpy()), bits(init + oracle_gemv(oracle, t, x, W, N, K)))
+    nw = rng.uniform(0.5, 1.5, K).astype(np.float32)
+    gpu.batch_gemv([dw], dx, M, [out], gpu.array(nw), EPS)
+    xn = np.stack([oracle.rmsnorm(r, nw, EPS) for r in x])
+    assert np.array_equal(bits(out.numpy()), bits(oracle_gemv(oracle, t, xn, W, N, K)))
+
+
+@pytest.mark.parametrize("tname,K,ff,M", [("Q4_K", 1280, 9000, 8), ("Q6_K", 512, 50, 2),
+                                          ("TQ1_0", 512, 96, 9), ("TQ2_0", 2560, 700, 50),
                                           ("TQ2_0", 512, 8200, 65), ("Q4_K", 768, 40, 33)])
 def test_batch_gate_up_bit_exact(gpu, oracle, tname, K, ff, M):
     rng = np.random.default_rng(K + ff + M)
@@ -71,6 +93,7 @@ def test_batch_nonfinite_follows_the_reference(gpu, oracle, tname):
     rows = [np.asarray(r, np.float32) for r in nonfinite_rows(rng, K)]
     rows += [rng.standard_normal(K).astype(np.float32) for _ in range(9)]
     x = np.stack(rows)
+    few = np.stack(rows[:7] + rows[-1:])
     for special in (None, np.inf, np.nan):
         w = W.copy()
         if special is not None:
@@ -81,6 +104,10 @@ def test_batch_nonfinite_follows_the_reference(gpu, oracle, tname):
         gpu.batch_gemv([gpu.tensor(t, K, N, w)], gpu.array(x), len(rows), [out])
         got = out.numpy().reshape(len(rows), N)
         for r, xr in enumerate(rows):
+            assert same_or_both_nan(got[r], oracle.gemv(t, xr, w, N, K)), (special, r)
+        gpu.gemv(gpu.tensor(t, K, N, w), gpu.array(few), 8, out)
+        got = out.numpy()[:8 * N].reshape(8, N)
+        for r, xr in enumerate(few):
             assert same_or_both_nan(got[r], oracle.gemv(t, xr, w, N, K)), (special, r)
 
 
