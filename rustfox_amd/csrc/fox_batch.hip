@@ -36,7 +36,7 @@
 #define BT_THREADS 256
 #define MAGIC_BITS 0x4B400000           // 12582912.0f = 1.5 * 2^23
 #define MAGIC_F 12582912.0f
-#define B_ROW 272                       // LDS bytes of one token's block (256 and a 16-byte pad)
+#define B_TILE 4096                     // operand bytes of 16 tokens and one block
 
 // 16-byte quads of per-token values per (16-token tile, block): TQ2_0 the
 // negated block sums (plus MAGIC_BITS), Q4_K eight sub-block sums and the
@@ -48,9 +48,11 @@ __host__ __device__ constexpr int aux_quads(int fmt)
 
 // ------------------------------------------------------------------ prep
 
-// where lane dl's dword (elements 4 dl .. 4 dl + 3 of a block) goes in the
-// token's 256 bytes: 16-byte piece (step, g) is what lane group g feeds to
-// MFMA step `step` (mirroring the weight decodes below)
+// Where lane dl's dword (elements 4 dl .. 4 dl + 3 of a block) goes in the
+// operand of a token tile and block, token 0's offset (a token is 16 bytes
+// on): [step][g][16 tokens][16 bytes], what lane group g feeds to MFMA step
+// `step` (mirroring the weight decodes below).  A wave's operand load is one
+// contiguous 1 KB.
 template <int FMT>
 __device__ __forceinline__ int piece_off(int dl)
 {
@@ -58,13 +60,13 @@ __device__ __forceinline__ int piece_off(int dl)
     if (FMT == FMT_TQ2) {
         const int half = e0 >> 7, l = (e0 >> 5) & 3, o = e0 & 31;
         const int g = 2 * half + (o >> 4), u = (o & 15) >> 2;
-        return (u * 4 + g) * 16 + l * 4;
+        return (u * 4 + g) * 256 + l * 4;
     } else if (FMT == FMT_Q4K) {
         // sub-blocks 2p and 2p + 1 side by side, eight elements of each
         const int s = e0 >> 5, o = e0 & 31;
-        return ((s >> 1) * 4 + (o >> 3)) * 16 + (s & 1) * 8 + (o & 4);
+        return ((s >> 1) * 4 + (o >> 3)) * 256 + (s & 1) * 8 + (o & 4);
     } else {
-        return e0;
+        return (e0 >> 4) * 256 + (e0 & 15);
     }
 }
 
@@ -148,19 +150,23 @@ __device__ __forceinline__ uint32_t wave_max_u(uint32_t v)
 // block sums.  512 threads; thread tid holds dwords tid + 512 r, so a wave
 // holds whole blocks (block wave + 8 r).  The K-quants without a norm have
 // nothing to share between blocks: there blockIdx.y takes 8 R blocks each.
-// q: [token][K] bytes, each block's 256 in piece_off order, or (few)
+// Eight tokens in a row run on one XCD (blockIdx % 8): they share the cache
+// lines of the operand.
+// q: [token / 16][block][4096], in piece_off order, or (few)
 // [block][2048], in few_off order; aux: [token / 16][block][aux_quads][token % 16].
 template <int FMT, bool NORM, int R>
 __global__ __launch_bounds__(512) void batch_prep(const float *__restrict__ x,
                                                   const float *__restrict__ norm_w, int K,
-                                                  size_t x_stride, float eps, int few,
+                                                  size_t x_stride, float eps, int M, int few,
                                                   uint8_t *__restrict__ q,
                                                   uint32_t *__restrict__ aux,
                                                   float *__restrict__ scale)
 {
     __shared__ double dred[8];
     __shared__ uint32_t ured[8];
-    const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int bx = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int t = few ? bx : (bx >> 6) * 64 + (bx & 7) * 8 + ((bx >> 3) & 7);
+    if (t >= M) return;                                     // (uniform)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b_first = FMT != FMT_TQ2 && !NORM ? (int)blockIdx.y * 8 * R : 0;
     const int nb = (K >> 8) - b_first, nd = nb * 64;
@@ -242,8 +248,9 @@ __global__ __launch_bounds__(512) void batch_prep(const float *__restrict__ x,
         if (tid == 0) scale[t] = qv.act;
     }
     const bool fw = FMT != FMT_TQ2 && few;
-    const size_t bs = fw ? 2048 : 256;
-    uint8_t *qt = q + (fw ? (size_t)t * 16 + few_off<FMT>(lane) : (size_t)t * K + piece_off<FMT>(lane)) +
+    const size_t bs = fw ? 2048 : B_TILE;
+    uint8_t *qt = q + (fw ? (size_t)t * 16 + few_off<FMT>(lane)
+                          : (size_t)(t >> 4) * (K >> 8) * B_TILE + (t & 15) * 16 + piece_off<FMT>(lane)) +
                   b_first * bs;
     uint32_t *at = aux + ((size_t)(t >> 4) * (K >> 8) + b_first) * (aux_quads(FMT) * 4) + (t & 15);
 #pragma unroll
@@ -385,14 +392,14 @@ __device__ __forceinline__ bool any_nonfinite(float d)
 }
 
 // One block of R row tiles against C token tiles, its float terms added to
-// acc.  bl: the block's token rows in LDS (tile c at bl + c * 16 * B_ROW),
+// acc.  bl: the block's operand in LDS (tile c at bl + c * B_TILE),
 // ax: its aux (tile c at ax + c * aux_quads quads).
 template <int FMT, int R, int C>
 __device__ __forceinline__ void block_terms(const RawBlock<FMT> (&raw)[R], const uint8_t *bl,
                                             const u4v *ax, int lane, f4v (&acc)[R][C])
 {
-    const int j = lane & 15, g = lane >> 4;
-    const uint8_t *bt = bl + j * B_ROW + g * 16;
+    const int g = lane >> 4;
+    const uint8_t *bt = bl + lane * 16;
     if constexpr (FMT == FMT_TQ2) {
         v4i D[R][C], corr[C];
 #pragma unroll
@@ -408,7 +415,7 @@ __device__ __forceinline__ void block_terms(const RawBlock<FMT> (&raw)[R], const
             }
 #pragma unroll
             for (int c = 0; c < C; c++) {
-                const v4i a = *(const v4i *)(bt + c * 16 * B_ROW + u * 64);
+                const v4i a = *(const v4i *)(bt + c * B_TILE + u * 1024);
 #pragma unroll
                 for (int r = 0; r < R; r++) D[r][c] = mfma64(a, w[r], u == 0 ? corr[c] : D[r][c]);
             }
@@ -468,7 +475,7 @@ __device__ __forceinline__ void block_terms(const RawBlock<FMT> (&raw)[R], const
 #pragma unroll
                 for (int c = 0; c < C; c++) {
                     typedef long l2v __attribute__((ext_vector_type(2)));
-                    const l2v a = *(const l2v *)(bt + c * 16 * B_ROW + p * 64);
+                    const l2v a = *(const l2v *)(bt + c * B_TILE + p * 1024);
                     const f4v as = ((const f4v *)ax)[c * 36 + 32 + g];
 #pragma unroll
                     for (int hh = 0; hh < 2; hh++) {
@@ -510,8 +517,8 @@ __device__ __forceinline__ void block_terms(const RawBlock<FMT> (&raw)[R], const
 #pragma unroll
             for (int c = 0; c < C; c++) {
                 v4i x[2];
-                x[0] = *(const v4i *)(bt + c * 16 * B_ROW + h * 128);
-                x[1] = *(const v4i *)(bt + c * 16 * B_ROW + h * 128 + 64);
+                x[0] = *(const v4i *)(bt + c * B_TILE + h * 2048);
+                x[1] = *(const v4i *)(bt + c * B_TILE + h * 2048 + 1024);
                 const f4v as = ((const f4v *)ax)[c * 4 + g];
                 asm volatile("" : "+v"(x[0]), "+v"(x[1]));    // (see below)
 #pragma unroll
@@ -558,7 +565,7 @@ template <int FMT, int R, int C, int EPI>
 __global__ __launch_bounds__(BT_THREADS, 2) void batch_gemm(BatchArgs a)
 {
     constexpr int KB = stage_blocks(FMT, C), CH = batch_chunk(FMT), AQ = aux_quads(FMT);
-    constexpr int BB = KB * C * 16 * B_ROW, NAX = KB * C * AQ;
+    constexpr int BB = KB * C * B_TILE, NAX = KB * C * AQ;
     static_assert(NAX <= BT_THREADS, "one aux quad per thread and stage");
     static_assert(EPI != BE_SILU || R % 2 == 0, "gate and up tiles in pairs");
     __shared__ __align__(16) uint8_t Bs[2][BB];
@@ -569,7 +576,7 @@ __global__ __launch_bounds__(BT_THREADS, 2) void batch_gemm(BatchArgs a)
     const int item = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if (item >= a.n_wg || (int)(blockIdx.x >> 3) >= per) return;    // (uniform)
     const int rg = item / a.n_tg, tg = item - rg * a.n_tg;
-    const int nb = a.nb, K = nb * 256, ntt = (a.M + 15) >> 4;
+    const int nb = a.nb, ntt = (a.M + 15) >> 4;
 
     // this wave's tiles: weights, segment and tile within it (tiles past the
     // end repeat the last one and are not written)
@@ -595,20 +602,19 @@ __global__ __launch_bounds__(BT_THREADS, 2) void batch_gemm(BatchArgs a)
         wp[r] = a.w[seg[r]] + (size_t)tl[r] * nb * CH;
     }
 
-    // staging: piece i = (block kb, tile c) of a stage, thread tid its token
-    // row tid / 16, 16-byte piece tid % 16
-    const int st = tid >> 4, sp = tid & 15;
+    // staging: piece i = (block kb, tile c) of a stage, 4 KB, 16 bytes of it
+    // per thread
     const uint8_t *qrow[C];
 #pragma unroll
     for (int c = 0; c < C; c++)
-        qrow[c] = a.q + (size_t)min((tg * C + c) * 16 + st, a.M - 1) * K + sp * 16;
+        qrow[c] = a.q + (size_t)min(tg * C + c, ntt - 1) * nb * B_TILE + tid * 16;
     u4v br[KB * C], ar = {0, 0, 0, 0};
     auto fetch = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
         for (int kb = 0; kb < KB; kb++)
 #pragma unroll
             for (int c = 0; c < C; c++)
-                br[kb * C + c] = *(const u4v *)(qrow[c] + (size_t)min(s * KB + kb, nb - 1) * 256);
+                br[kb * C + c] = *(const u4v *)(qrow[c] + (size_t)min(s * KB + kb, nb - 1) * B_TILE);
         const int ai = min(tid, NAX - 1), i = ai / AQ, kb = i / C, c = i - kb * C;
         ar = ((const u4v *)a.aux)[((size_t)min(tg * C + c, ntt - 1) * nb + min(s * KB + kb, nb - 1)) * AQ +
                                   (ai - i * AQ)];
@@ -616,7 +622,7 @@ __global__ __launch_bounds__(BT_THREADS, 2) void batch_gemm(BatchArgs a)
     auto stash = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < KB * C; i++)
-            *(u4v *)(Bs[buf] + (i * 16 + st) * B_ROW + sp * 16) = br[i];
+            *(u4v *)(Bs[buf] + i * B_TILE + tid * 16) = br[i];
         if (tid < NAX) As[buf][tid] = ar;
     };
     RawBlock<FMT> cur[KB][R], nxt[KB][R];
@@ -645,7 +651,7 @@ __global__ __launch_bounds__(BT_THREADS, 2) void batch_gemm(BatchArgs a)
 #pragma unroll
         for (int kb = 0; kb < KB; kb++)
             if (s * KB + kb < nb)                            // (uniform)
-                block_terms<FMT, R, C>(cur[kb], Bs[buf] + kb * C * 16 * B_ROW,
+                block_terms<FMT, R, C>(cur[kb], Bs[buf] + kb * C * B_TILE,
                                        &As[buf][kb * C * AQ], lane, acc);
         // the other buffer was last read before the previous barrier
         stash(buf ^ 1);
@@ -904,6 +910,203 @@ __global__ __launch_bounds__(KS * 64, FMT == FMT_Q4K ? 4 : 3) void few_gemm(Batc
     else *o = (a.flags & FOX_GPU_GEMV_ACCUMULATE) ? *o + y[0] : y[0];
 }
 
+// ------------------------------------------- few row tiles: blocks split
+
+// batch_gemm's waves each walk the whole of K, so a matrix of few rows leaves
+// the chip part empty and every block waits for its loads (Q6_K 4096 x 14336,
+// 16 tokens: 59 us, here 26; Q4_K 4096 x 4096 19, here 10.5).  Here a workgroup is one row tile and one token tile, its
+// KS waves take units of U blocks in turn, operands straight from L2 to
+// registers, and pass the float terms through LDS to 256 lanes (token, row)
+// that add them in block order, as in few_gemm.
+template <int FMT>
+struct SplitTerms;                      // one lane's terms of a unit, per token k
+template <>
+struct SplitTerms<FMT_TQ2> { static constexpr int U = 2, NV = 1; typedef f2v V; };   // two blocks
+template <>
+struct SplitTerms<FMT_Q4K> { static constexpr int U = 1, NV = 2; typedef f4v V; };   // sub-blocks 4v ..
+template <>
+struct SplitTerms<FMT_Q6K> { static constexpr int U = 1, NV = 1; typedef f4v V; };   // quarters
+
+#define SPLIT_KS 4
+template <int FMT, int EPI>
+__global__ __launch_bounds__(256, FMT == FMT_Q4K ? 2 : 3) void split_gemm(BatchArgs a)
+{
+    typedef SplitTerms<FMT> ST;
+    typedef typename ST::V V;
+    constexpr int KS = SPLIT_KS, U = ST::U, NV = ST::NV, CH = batch_chunk(FMT), AQ = aux_quads(FMT);
+    __shared__ V terms[2][KS][NV][16][16];                 // [buffer][slot][..][token][row]
+    const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nb = a.nb, tt = blockIdx.y;
+    const uint8_t *qp = a.q + (size_t)tt * nb * B_TILE + lane * 16;
+    const f4v *axp = (const f4v *)a.aux + (size_t)tt * nb * AQ + g;
+    const int crow = tid & 15, ct = tid >> 4;              // of the combine: row, token
+    float y[EPI == BE_SILU ? 2 : 1];
+    int tile = blockIdx.x, s = 0;
+    if (EPI != BE_SILU) {
+        while (s + 1 < a.nseg && tile >= a.tile_start[s + 1]) s++;
+        tile -= a.tile_start[s];
+    }
+    const int nu = (nb + U - 1) / U, ns = (nu + KS - 1) / KS;
+#pragma unroll
+    for (int it = 0; it < (EPI == BE_SILU ? 2 : 1); it++) {
+        const uint8_t *wp = a.w[EPI == BE_SILU ? it : s] + (size_t)tile * nb * CH;
+        struct Unit {
+            RawBlock<FMT> w[U];
+            v4i x[U][4];
+            f4v ax[U][FMT == FMT_Q4K ? 9 : 1];
+        };
+        auto load = [&](int r, Unit &u) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < U; i++) {
+                const int b = min((r * KS + wave) * U + i, nb - 1);
+                u.w[i].load(wp + (size_t)b * CH, lane);
+#pragma unroll
+                for (int p = 0; p < 4; p++) u.x[i][p] = *(const v4i *)(qp + (size_t)b * B_TILE + p * 1024);
+#pragma unroll
+                for (int p = 0; p < (FMT == FMT_Q4K ? 9 : 1); p++) u.ax[i][p] = axp[(size_t)b * AQ + 4 * p];
+            }
+        };
+        auto compute = [&](const Unit &u, V (*o)[NV][16][16]) __attribute__((always_inline)) {
+            V t[NV][4];
+            if constexpr (FMT == FMT_TQ2) {
+#pragma unroll
+                for (int i = 0; i < U; i++) {
+                    v4i D = __builtin_bit_cast(v4i, u.ax[i][0]);
+#pragma unroll
+                    for (int p = 0; p < 4; p++) {
+                        const uint32_t d = u.w[i].qs[p];
+                        const v4i w = {(int)(d & 0x03030303u), (int)((d >> 2) & 0x03030303u),
+                                       (int)((d >> 4) & 0x03030303u), (int)((d >> 6) & 0x03030303u)};
+                        D = mfma64(u.x[i][p], w, D);
+                    }
+                    const float d = half_bits_to_float(u.w[i].d);
+                    if (!any_nonfinite(d)) {
+                        const float nd = -MAGIC_F * d;
+#pragma unroll
+                        for (int k = 0; k < 4; k++) t[0][k][i] = __builtin_fmaf(d, __int_as_float(D[k]), nd);
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < 4; k++) t[0][k][i] = d * (float)(D[k] - MAGIC_BITS);
+                    }
+                }
+            } else if constexpr (FMT == FMT_Q4K) {
+                // (batch_gemm's terms, block_terms)
+                const RawBlock<FMT> &raw = u.w[0];
+                const uint32_t s0 = raw.h[1], s1 = raw.h[2], s2 = raw.h[3];
+                const uint32_t sc[2] = {s0 & 0x3f3f3f3fu,
+                                        (s2 & 0x0f0f0f0fu) | (((s0 >> 6) & 0x03030303u) << 4)};
+                const uint32_t mn[2] = {s1 & 0x3f3f3f3fu,
+                                        ((s2 >> 4) & 0x0f0f0f0fu) | (((s1 >> 6) & 0x03030303u) << 4)};
+                const float d = half_bits_to_float(raw.h[0] & 0xffffu);
+                const float dmin = half_bits_to_float(raw.h[0] >> 16);
+                const v4i magic = {MAGIC_BITS, MAGIC_BITS, MAGIC_BITS, MAGIC_BITS};
+                const f4v as = u.ax[0][8];
+                auto run = [&](auto finite) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int sb = 0; sb < 8; sb++) {
+                        const int p = sb >> 1, hh = sb & 1;
+                        const uint32_t a0 = (p < 2 ? raw.q0[2 * p] : raw.q1[2 * p - 4]) >> (4 * hh);
+                        const uint32_t a1 = (p < 2 ? raw.q0[2 * p + 1] : raw.q1[2 * p - 3]) >> (4 * hh);
+                        const long w = (long)((uint64_t)(a0 & 0x0f0f0f0fu) | (uint64_t)(a1 & 0x0f0f0f0fu) << 32);
+                        const long x = (long)((uint64_t)(uint32_t)u.x[0][p][2 * hh] |
+                                              (uint64_t)(uint32_t)u.x[0][p][2 * hh + 1] << 32);
+                        const v4i D = __builtin_amdgcn_mfma_i32_16x16x32_i8(x, w, magic, 0, 0, 0);
+                        const float A = d * (float)((sc[sb >> 2] >> (8 * (sb & 3))) & 0xffu);
+                        const float B = dmin * (float)((mn[sb >> 2] >> (8 * (sb & 3))) & 0xffu);
+                        const float na = -MAGIC_F * A;
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+                            const float pr = decltype(finite)::value
+                                                 ? __builtin_fmaf(A, __int_as_float(D[k]), na)
+                                                 : A * (float)(D[k] - MAGIC_BITS);
+                            t[sb >> 2][k][sb & 3] = as[k] * (pr - B * u.ax[0][sb][k]);
+                        }
+                    }
+                };
+                if (!any_nonfinite(d)) run(std::true_type{});
+                else run(std::false_type{});
+            } else {
+                const float d = half_bits_to_float(u.w[0].d);
+                const v4i zero = {0, 0, 0, 0};
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    v4i part[2] = {zero, zero};
+#pragma unroll
+                    for (int hi = 0; hi < 2; hi++) {
+                        const v4i w = q6_bytes(u.w[0], h, hi, g);
+#pragma unroll
+                        for (int gg = 0; gg < 4; gg++) {
+                            const int m = g == gg ? -1 : 0;
+                            const v4i wm = {w[0] & m, w[1] & m, w[2] & m, w[3] & m};
+                            const v4i D = mfma64(u.x[0][2 * h + hi], wm, zero);
+                            const int sc = q6_scale(u.w[0].sc, 8 * h + (gg & 1) + 2 * ((gg >> 1) + 2 * hi));
+#pragma unroll
+                            for (int k = 0; k < 4; k++) part[gg & 1][k] += __mul24(sc, D[k]);
+                        }
+                    }
+#pragma unroll
+                    for (int v = 0; v < 2; v++)
+#pragma unroll
+                        for (int k = 0; k < 4; k++)
+                            t[0][k][2 * h + v] = u.ax[0][0][k] * d * (float)(part[v][k] >> 2);
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < NV; v++)
+#pragma unroll
+                for (int k = 0; k < 4; k++) (*o)[v][4 * g + k][j] = t[v][k];
+        };
+        float acc = 0.0f;
+        auto combine = [&](int r) __attribute__((always_inline)) {
+#pragma unroll
+            for (int w = 0; w < KS; w++) {
+                const int b = (r * KS + w) * U;
+                if (b >= nb) break;                        // (uniform)
+#pragma unroll
+                for (int v = 0; v < NV; v++) {
+                    const V x = terms[r & 1][w][v][ct][crow];
+                    if (FMT == FMT_TQ2) {
+                        acc = acc + x[0];
+                        if (b + 1 < nb) acc = acc + x[1];  // (uniform)
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc = acc + x[i];
+                    }
+                }
+            }
+        };
+        auto round = [&](int r, Unit &u) __attribute__((always_inline)) {
+            if (r < ns) compute(u, &terms[r & 1][wave]);   // (uniform)
+            load(r + 2, u);
+            __builtin_amdgcn_sched_barrier(0);             // (as in few_gemm)
+            __syncthreads();
+            combine(r);
+        };
+        Unit u0, u1;
+        load(0, u0);
+        __builtin_amdgcn_sched_barrier(0);
+        load(1, u1);
+        __builtin_amdgcn_sched_barrier(0);
+        for (int r = 0; r < ns; r += 2) {
+            round(r, u0);
+            round(r + 1, u1);
+        }
+        y[it] = acc;
+        if (EPI == BE_SILU) __syncthreads();               // (the buffers start over)
+    }
+    const int t = tt * 16 + ct, row = tile * 16 + crow;
+    if (t >= a.M || row >= a.n_rows[s]) return;
+    if (FMT == FMT_TQ2) {
+        const float sc = a.scale[t];
+#pragma unroll
+        for (int it = 0; it < (EPI == BE_SILU ? 2 : 1); it++) y[it] = y[it] * sc;
+    }
+    float *o = a.out[s] + (size_t)t * a.out_stride[s] + row;
+    if (EPI == BE_SILU) *o = fox_div(y[0], 1.0f + fox_expf(-y[0])) * y[EPI == BE_SILU];
+    else *o = (a.flags & FOX_GPU_GEMV_ACCUMULATE) ? *o + y[0] : y[0];
+}
+
 // ------------------------------------------------------------------ host
 
 static size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -922,7 +1125,7 @@ static fox_gpu_status batch_carve(fox_gpu_ctx *ctx, int fmt, size_t K, size_t M,
                                   BatchWs *w)
 {
     // (few_gemm's operand has room for eight tokens whatever M is)
-    const size_t nq = up256((M < FOX_GPU_MAX_TOKENS ? FOX_GPU_MAX_TOKENS : M) * K);
+    const size_t nq = M <= FOX_GPU_MAX_TOKENS && fmt != FMT_TQ2 ? FOX_GPU_MAX_TOKENS * K : (M + 15) / 16 * 16 * K;
     const size_t na = up256((M + 15) / 16 * (K / 256) * (size_t)aux_quads(fmt) * 16);
     const size_t ns = up256(M * 4);
     if (!fixed) {
@@ -979,6 +1182,23 @@ static const void *few_kernel(int fmt, bool wide, int epi)
 #undef FOX_FEW
 }
 
+static const void *split_kernel(int fmt, int epi)
+{
+#define FOX_SPLIT(f) (epi == BE_SILU ? (const void *)split_gemm<f, BE_SILU> : (const void *)split_gemm<f, BE_STORE>)
+    return fmt == FMT_TQ2 ? FOX_SPLIT(FMT_TQ2) : fmt == FMT_Q4K ? FOX_SPLIT(FMT_Q4K) : FOX_SPLIT(FMT_Q6K);
+#undef FOX_SPLIT
+}
+
+// split_gemm where batch_gemm would have too few waves to hide its loads: by
+// row tiles times token groups, a measured line per format (us, split / whole):
+// ternary 160 tiles x 2 groups (K 9728) 20 / 29, 336 x 2 (K 4096) 22 / 18;
+// Q4_K (K 4096) 256 x 2 27 / 36, 256 x 4 59 / 53, 896 x 1 23 / 20; Q6_K
+// (K 14336) 256 x 2 66 / 130, 256 x 4 143 / 162.
+static bool split_better(int fmt, int tiles, int mt, int n_cu)
+{
+    return tiles * ((mt + 3) / 4) < (fmt == FMT_TQ2 ? 2 : fmt == FMT_Q4K ? 3 : 5) * n_cu;
+}
+
 static fox_gpu_status batch_check(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor *const *ws,
                                   const float *x, size_t x_stride, size_t M, float *const *outs,
                                   const size_t *out_strides)
@@ -1012,7 +1232,8 @@ static fox_gpu_status batch_run(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor
     const int fmt = fmt_of(ws[0]->type);
     const size_t K = (size_t)ws[0]->ne0;
     // (Q6_K gate/up pairs: two such tiles per wave do not fit its registers)
-    if (fmt < 0 || (fmt == FMT_Q6K && epi == BE_SILU && M > FOX_GPU_MAX_TOKENS) || K == 0 || K % 256 || K > 2048 * PREP_MAX_R || x_stride % 4 ||
+    if (fmt < 0 || (fmt == FMT_Q6K && epi == BE_SILU && M > FOX_GPU_MAX_TOKENS &&
+                    !split_better(fmt, (int)ws[0]->n_tiles, (int)((M + 15) / 16), ctx->n_cu)) || K == 0 || K % 256 || K > 2048 * PREP_MAX_R || x_stride % 4 ||
         ((uintptr_t)x | (uintptr_t)norm_w) % 16)
         return FOX_GPU_ERR_UNSUPPORTED;
     BatchWs w;
@@ -1023,14 +1244,15 @@ static fox_gpu_status batch_run(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor
         const void *k = fmt == FMT_TQ2 ? prep_fmt<FMT_TQ2>(norm_w != nullptr, r)
                       : fmt == FMT_Q4K ? prep_fmt<FMT_Q4K>(norm_w != nullptr, r)
                                        : prep_fmt<FMT_Q6K>(norm_w != nullptr, r);
-        int iK = (int)K, few = fmt != FMT_TQ2 && M <= FOX_GPU_MAX_TOKENS;
-        void *args[] = {(void *)&x, (void *)&norm_w, (void *)&iK, (void *)&x_stride, (void *)&eps, (void *)&few,
+        int iK = (int)K, iM = (int)M, few = fmt != FMT_TQ2 && M <= FOX_GPU_MAX_TOKENS;
+        void *args[] = {(void *)&x, (void *)&norm_w, (void *)&iK, (void *)&x_stride, (void *)&eps, (void *)&iM,
+                        (void *)&few,
                         (void *)&w.q, (void *)&w.aux, (void *)&w.scale};
         const bool split = fmt != FMT_TQ2 && !norm_w;      // (blocks apart on grid y, R = 1)
         if (split) k = fmt == FMT_Q4K ? (const void *)batch_prep<FMT_Q4K, false, 1>
                                       : (const void *)batch_prep<FMT_Q6K, false, 1>;
-        hipError_t e = hipLaunchKernel(k, dim3((unsigned)M, split ? (unsigned)r : 1u), dim3(512), args,
-                                       0, ctx->stream);
+        hipError_t e = hipLaunchKernel(k, dim3(few ? (unsigned)M : (unsigned)((M + 63) / 64 * 64), split ? (unsigned)r : 1u),
+                                       dim3(512), args, 0, ctx->stream);
         if (e != hipSuccess) return fox_hip_fail(e, "batch: prepare");
         FOX_LAUNCHED("batch: prepare");
     }
@@ -1067,8 +1289,18 @@ static fox_gpu_status batch_run(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor
         FOX_LAUNCHED("batch: product");
         return FOX_GPU_OK;
     }
+    const int mt = (int)((M + 15) / 16);
+    const int wt = epi == BE_SILU ? a.tile_start[1] : tiles;        // workgroup tiles
+    if (split_better(fmt, wt, mt, ctx->n_cu)) {
+        const void *k = split_kernel(fmt, epi);
+        void *args[] = {(void *)&a};
+        hipError_t e = hipLaunchKernel(k, dim3((unsigned)wt, (unsigned)mt), dim3(256), args, 0, ctx->stream);
+        if (e != hipSuccess) return fox_hip_fail(e, "batch: product");
+        FOX_LAUNCHED("batch: product");
+        return FOX_GPU_OK;
+    }
     // token groups of C 16-token tiles, as even as they come at C <= 4
-    const int mt = (int)((M + 15) / 16), n_tg = (mt + 3) / 4, C = (mt + n_tg - 1) / n_tg;
+    const int n_tg = (mt + 3) / 4, C = (mt + n_tg - 1) / n_tg;
     a.n_tg = (mt + C - 1) / C;
     // row tiles per wave: more share each token operand read from LDS (the
     // ternary kernel's LDS reads take as long as its MFMAs below four), as
