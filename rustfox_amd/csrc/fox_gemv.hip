@@ -424,177 +424,201 @@ __global__ __launch_bounds__(blk_waves(FMT) * 64) void gemv_blocks(
 // -------------------------------------------------------- float weights
 
 // F16 / F32 rows (src/kernels.c:81-96): each lane owns one row and adds
-// w[k] * x[k] sequentially in k, exactly the reference's order.  A
-// workgroup owns one 256-row tile of the tiled float layout.  Its chunks
-// (128 bytes of every row, 32 KB contiguous) stream through LDS in halves
-// (64 bytes of every row per step; rows padded by a dword against bank
-// conflicts), double buffered: the next step's loads are in flight while a
-// step is summed.  The activations of a step ride along in the same
-// buffers.  (Half steps keep a workgroup's LDS near 35 KB, so that every
-// tile of a large head is resident at once: with whole chunks only two
-// workgroups fit a CU and the last tiles run in a second, mostly idle
-// round.)
-#define FR 256      // rows per tile of the layout
-
-// RW rows per workgroup (FR, or FR / 2: two workgroups per tile, each
-// reading its half of every chunk, which spreads a large head's rows more
-// evenly over the compute units)
-template <typename WT, int MT, int RW>
-__global__ __launch_bounds__(RW) void gemv_float(const WT *__restrict__ W, int K, int N,
+// w[k] * x[k] sequentially in k for TM tokens, exactly the reference's order.
+// A workgroup is one wave over 64 rows of the tiled layout, whose 128-byte
+// row chunks (8 KB contiguous for the 64 rows) go through LDS from
+// coalesced registers to the lanes' rows (row stride padded by a quad
+// against bank conflicts); two chunks are in flight from memory while a third
+// is summed and a fourth is on its way through LDS.  One wave needs no
+// barrier.  The activations are the same for every lane: they are read
+// through scalar loads, so a term costs no LDS read.  An f16 product is one
+// fused multiply-add from the half and -0.0 (which leaves every product as it
+// is), with no conversion before it.
+//
+// Large heads are bound by memory (151936 x 2560 in f16, 778 MB: one token
+// 137 us, four 166, eight 217; with a workgroup per 256 rows, the activations
+// through LDS and a bounds test per token they took 146, 511 and 777), small
+// matrices by the chain of K adds per row and token: there the tokens are
+// spread over more waves (float_tokens; 1223 x 8816, six tokens: 2105 -> 76
+// us).
+template <typename WT, int TM>
+__global__ __launch_bounds__(64) void gemv_float(const WT *__restrict__ W, int K, int N,
                                                  const float *__restrict__ x, int x_stride,
-                                                 int M, float *__restrict__ out,
-                                                 int out_stride, unsigned flags)
+                                                 int M, float *__restrict__ out, int out_stride,
+                                                 unsigned flags, int n_tg, int n_rg)
 {
-    constexpr int FK = 64 / sizeof(WT);                // elements of a step (half a row chunk)
-    constexpr int RDW = FK * sizeof(WT) / 4;           // dwords of a row per step
-    constexpr int RSTR = RDW + 1;                       // padded row stride
-    constexpr int PPR = RDW / 4;                        // 16-byte pieces per row and step
-    constexpr int NP = PPR;                             // pieces per thread
-    __shared__ uint32_t wl[2][RW * RSTR];
-    __shared__ float xs[2][MT * FK];
-    if (MT == 1) {
-        M = 1;
-    } else {
-        // (a batched pass: token groups of MT on the grid's second axis)
-        const int t0 = (int)blockIdx.y * MT;
-        x += (size_t)t0 * x_stride;
-        out += (size_t)t0 * out_stride;
-        M = min(MT, M - t0);
-    }
-    const int tid = threadIdx.x;
-    const int r0 = blockIdx.x * RW;
-    const int nchunk = (K + FK - 1) / FK;               // steps
-    const int nch128 = (K + 2 * FK - 1) / (2 * FK);     // 128-byte chunks of the layout
-    // this tile's chunks, 32 KB each (rows and columns zero-padded)
-    const uint4 *tw = (const uint4 *)W + (size_t)(blockIdx.x / (FR / RW)) * nch128 * (FR * 2 * PPR) +
-                      (size_t)(blockIdx.x % (FR / RW)) * RW * 2 * PPR;
-
-    constexpr int XPT = (MT * FK + RW - 1) / RW;        // activations staged per thread
-    uint4 R[NP];
-    float xr[XPT];
-    // global -> registers for chunk c (rows past N and columns past K read 0)
-    auto fetch = [&](int c) {
-        const int k0 = c * FK, kn = K - k0 < FK ? K - k0 : FK;
-        // half c & 1 of chunk c / 2: pieces (row, part) at row * 2 PPR + part
-        const uint4 *cw = tw + (size_t)(c >> 1) * (FR * 2 * PPR) + (c & 1) * PPR;
+    typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+    constexpr int FK = FOX_FCHUNK / (int)sizeof(WT);       // elements of a row chunk
+    constexpr int EQ = 16 / (int)sizeof(WT);               // elements of a 16-byte piece
+    constexpr int RSTR = 9;                                // LDS row stride in quads
+    __shared__ u4v rows[64 * RSTR];
+    const int lane = threadIdx.x;
+    // a row group's token groups on one XCD (blockIdx % 8), one after another
+    const int k8 = (int)blockIdx.x >> 3, tg = k8 % n_tg, rg = (k8 / n_tg) * 8 + ((int)blockIdx.x & 7);
+    if (rg >= n_rg) return;                                // (uniform)
+    const int t0 = tg * TM, nt = min(TM, M - t0);
+    const int nchunk = (K + FK - 1) / FK, nfull = K / FK;
+    // this group's pieces: chunk c at c * 32 KB
+    const u4v *tw = (const u4v *)W + (size_t)(rg >> 2) * nchunk * (FOX_FTILE * 8) + (rg & 3) * 512 + lane;
+    // (tokens past the last repeat it and are not written)
+    const float *xt[TM];
 #pragma unroll
-        for (int i = 0; i < NP; i++) {
-            const int pc = tid + i * RW, r = pc / PPR, part = pc - r * PPR;
-            R[i] = cw[r * 2 * PPR + part];
-        }
+    for (int t = 0; t < TM; t++) xt[t] = x + (size_t)(t0 + min(t, nt - 1)) * x_stride;
+    auto fetch = [&](int c, u4v (&r)[8]) __attribute__((always_inline)) {
+        const u4v *p = tw + (size_t)min(c, nchunk - 1) * (FOX_FTILE * 8);
 #pragma unroll
-        for (int v = 0; v < XPT; v++) {
-            const int e = tid + v * RW;
-            xr[v] = 0.0f;
-            if (e < M * FK) {
-                const int t = e / FK, kk = e - t * FK;
-                if (kk < kn) xr[v] = x[(size_t)t * x_stride + k0 + kk];
-            }
-        }
+        for (int i = 0; i < 8; i++) r[i] = p[64 * i];
     };
-    auto stash = [&](int buf) {
+    auto turn = [&](const u4v (&r)[8], u4v (&w)[8]) __attribute__((always_inline)) {
+        __syncthreads();                                   // (one wave: an ordering of LDS accesses)
 #pragma unroll
-        for (int i = 0; i < NP; i++) {
-            const int pc = tid + i * RW, r = pc / PPR, part = pc - r * PPR;
-            uint32_t *d = &wl[buf][r * RSTR + part * 4];
-            d[0] = R[i].x;
-            d[1] = R[i].y;
-            d[2] = R[i].z;
-            d[3] = R[i].w;
-        }
-#pragma unroll
-        for (int v = 0; v < XPT; v++) {
-            const int e = tid + v * RW;
-            if (e < M * FK) xs[buf][e] = xr[v];
-        }
-    };
-
-    float acc[MT];
-#pragma unroll
-    for (int t = 0; t < MT; t++) acc[t] = 0.0f;
-
-    fetch(0);
-    stash(0);
-    if (nchunk > 1) fetch(1);
-    __syncthreads();
-    for (int c = 0; c < nchunk; c++) {
-        const int buf = c & 1;
-        const int kn = K - c * FK < FK ? K - c * FK : FK;
-        const uint32_t *myw = &wl[buf][tid * RSTR];
-        const float *xb = xs[buf];
-        if (kn == FK) {
-#pragma unroll 8
-            for (int kk = 0; kk < FK; kk++) {
-                const uint32_t dword = myw[kk / (4 / (int)sizeof(WT))];
-                float w;
-                if (sizeof(WT) == 2)
-                    w = half_bits_to_float((dword >> (16 * (kk & 1))) & 0xFFFFu);
-                else
-                    w = __builtin_bit_cast(float, dword);
-#pragma unroll
-                for (int t = 0; t < MT; t++)
-                    if (t < M) acc[t] = acc[t] + w * xb[t * FK + kk];
-            }
-        } else {
-            for (int kk = 0; kk < kn; kk++) {
-                const uint32_t dword = myw[kk / (4 / (int)sizeof(WT))];
-                float w;
-                if (sizeof(WT) == 2)
-                    w = half_bits_to_float((dword >> (16 * (kk & 1))) & 0xFFFFu);
-                else
-                    w = __builtin_bit_cast(float, dword);
-#pragma unroll
-                for (int t = 0; t < MT; t++)
-                    if (t < M) acc[t] = acc[t] + w * xb[t * FK + kk];
-            }
-        }
-        if (c + 1 < nchunk) {
-            // the other buffer was last read before the previous barrier
-            stash(buf ^ 1);
-            if (c + 2 < nchunk) fetch(c + 2);
-        }
+        for (int i = 0; i < 8; i++) rows[((lane >> 3) + 8 * i) * RSTR + (lane & 7)] = r[i];
         __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 8; i++) w[i] = rows[lane * RSTR + i];
+    };
+    float acc[TM];
+#pragma unroll
+    for (int t = 0; t < TM; t++) acc[t] = 0.0f;
+    float nz = -0.0f;
+    asm("" : "+v"(nz));                                    // (known, it would be folded away)
+    auto term = [&](const u4v &q, int e, float xv) __attribute__((always_inline)) {
+        if constexpr (sizeof(WT) == 2) {
+            const uint32_t d = q[e >> 1];
+            const _Float16 h = __builtin_bit_cast(_Float16, (unsigned short)(e & 1 ? d >> 16 : d));
+            return __builtin_fmaf((float)h, xv, nz);
+        } else {
+            return __builtin_bit_cast(float, (uint32_t)q[e]) * xv;
+        }
+    };
+    // the activations of GK elements of every token, in scalar registers one
+    // group ahead: scalar loads return in no order, so a wait is for all of
+    // them, and the next group's are issued after the wait for this one's
+    // (the empty statement holds it in place) and return while it is summed
+    // (loaded where they are used, a 64-element chunk waited eight times)
+    constexpr int NE = TM == 1 ? 4 : TM == 2 ? 2 : 1, GK = 8 * NE, NG = FK / GK;
+    typedef float f8v __attribute__((ext_vector_type(8), aligned(4)));
+    f8v xn[TM * NE];
+    auto x_load = [&](int k) __attribute__((always_inline)) {
+        const int kc = min(k, K - GK);
+#pragma unroll
+        for (int t = 0; t < TM; t++)
+#pragma unroll
+            for (int n = 0; n < NE; n++) xn[t * NE + n] = *(const f8v *)(xt[t] + kc + 8 * n);
+    };
+    auto sums = [&](const u4v (&w)[8], int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int gi = 0; gi < NG; gi++) {
+            f8v xc[TM * NE];
+#pragma unroll
+            for (int i = 0; i < TM * NE; i++) {
+                xc[i] = xn[i];
+                asm volatile("" : "+s"(xc[i]));
+            }
+            x_load(c * FK + (gi + 1) * GK);
+            __builtin_amdgcn_sched_barrier(0);
+            // (eight elements' products before their adds: an add right after
+            // its product waits a state for it)
+#pragma unroll
+            for (int n = 0; n < NE; n++) {
+                float pr[TM][8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const int k = gi * GK + 8 * n + e;
+#pragma unroll
+                    for (int t = 0; t < TM; t++) pr[t][e] = term(w[k / EQ], k % EQ, xc[t * NE + n][e]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+#pragma unroll
+                    for (int t = 0; t < TM; t++) acc[t] = acc[t] + pr[t][e];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    u4v ra[8], rb[8], wa[8], wb[8];
+    fetch(0, ra);
+    fetch(1, rb);
+    turn(ra, wa);
+    fetch(2, ra);
+    if (nfull > 0) x_load(0);
+    // chunk c in w, c + 1 and c + 2 in registers
+    auto step = [&](int c, u4v (&w)[8], u4v (&wn)[8], u4v (&r)[8]) __attribute__((always_inline)) {
+        turn(r, wn);
+        fetch(c + 3, r);
+        if (c < nfull) {                                   // (uniform)
+            sums(w, c);
+        } else if (c < nchunk) {
+            // the ragged last chunk (uniform tests)
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+#pragma unroll
+                for (int e = 0; e < EQ; e++) {
+                    const int k = c * FK + i * EQ + e;
+                    if (k < K) {
+#pragma unroll
+                        for (int t = 0; t < TM; t++) acc[t] = acc[t] + term(w[i], e, xt[t][k]);
+                    }
+                }
+        }
+    };
+    for (int c = 0; c < nchunk; c += 2) {
+        step(c, wa, wb, rb);
+        step(c + 1, wb, wa, ra);
     }
-    const int row = r0 + tid;
+    const int row = rg * 64 + lane;
     if (row >= N) return;
 #pragma unroll
-    for (int t = 0; t < MT; t++) {
-        if (t >= M) break;
-        float *o = out + (size_t)t * out_stride + row;
+    for (int t = 0; t < TM; t++) {
+        if (t >= nt) break;
+        float *o = out + (size_t)(t0 + t) * out_stride + row;
         *o = (flags & FOX_GPU_GEMV_ACCUMULATE) ? *o + acc[t] : acc[t];
     }
 }
 
 // ----------------------------------------------------------------- host
 
-// F16 / F32 weights, any number of tokens (groups of FOX_GPU_MAX_TOKENS)
+// Tokens per wave: as few as leave one wave per SIMD at most (a wave's time is
+// its tokens' terms one after another, and idle SIMDs cost nothing), up to
+// four where the rows alone fill the chip (more spill scalar registers; the
+// second wave of a row group finds the weights in its XCD's L2)
+static int float_tokens(int n_rg, size_t M, int n_cu)
+{
+    int tm = 1;
+    while (tm < 4 && (size_t)tm < M &&
+           (size_t)n_rg * ((M + tm - 1) / tm) > 4 * (size_t)n_cu)
+        tm++;
+    const int n_tg = (int)((M + tm - 1) / tm);
+    return (int)((M + n_tg - 1) / n_tg);                   // (groups of about one size)
+}
+
+template <typename WT>
+static const void *float_kernel(int tm)
+{
+    switch (tm) {
+    case 1: return (const void *)gemv_float<WT, 1>;
+    case 2: return (const void *)gemv_float<WT, 2>;
+    case 3: return (const void *)gemv_float<WT, 3>;
+    default: return (const void *)gemv_float<WT, 4>;
+    }
+}
+
+// F16 / F32 weights, any number of tokens
 fox_gpu_status fox_float_gemv(fox_gpu_ctx *ctx, const fox_gpu_tensor *w, const float *x,
                               size_t x_stride, size_t M, float *out, size_t out_stride,
                               unsigned flags)
 {
-    const int N = (int)w->ne1, K = (int)w->ne0;
-    // one token: half-tile workgroups (a 151936-row head is 1187 of
-    // them: 4.6 per compute unit, against 2.3 whole tiles)
-    constexpr int RH = FR / 2;
-    dim3 grid((unsigned)((N + FR - 1) / FR),
-              (unsigned)((M + FOX_GPU_MAX_TOKENS - 1) / FOX_GPU_MAX_TOKENS)), block(FR);
-    dim3 grid1((unsigned)((N + RH - 1) / RH)), block1(RH);
-    const _Float16 *wh = (const _Float16 *)w->d;
-    const float *wf = (const float *)w->d;
-    if (w->type == FOX_GPU_F16 && M == 1)
-        hipLaunchKernelGGL((gemv_float<_Float16, 1, RH>), grid1, block1, 0, ctx->stream, wh, K, N, x,
-                           (int)x_stride, (int)M, out, (int)out_stride, flags);
-    else if (w->type == FOX_GPU_F16)
-        hipLaunchKernelGGL((gemv_float<_Float16, FOX_GPU_MAX_TOKENS, FR>), grid, block, 0,
-                           ctx->stream, wh, K, N, x, (int)x_stride, (int)M, out, (int)out_stride,
-                           flags);
-    else if (M == 1)
-        hipLaunchKernelGGL((gemv_float<float, 1, RH>), grid1, block1, 0, ctx->stream, wf, K, N, x,
-                           (int)x_stride, (int)M, out, (int)out_stride, flags);
-    else
-        hipLaunchKernelGGL((gemv_float<float, FOX_GPU_MAX_TOKENS, FR>), grid, block, 0,
-                           ctx->stream, wf, K, N, x, (int)x_stride, (int)M, out, (int)out_stride,
-                           flags);
+    int N = (int)w->ne1, K = (int)w->ne0, xs = (int)x_stride, os = (int)out_stride, iM = (int)M;
+    int n_rg = (N + 63) / 64;
+    const int tm = float_tokens(n_rg, M, ctx->n_cu);
+    int n_tg = (int)((M + tm - 1) / tm);
+    const void *k = w->type == FOX_GPU_F16 ? float_kernel<_Float16>(tm) : float_kernel<float>(tm);
+    void *args[] = {(void *)&w->d, (void *)&K, (void *)&N, (void *)&x, (void *)&xs, (void *)&iM,
+                    (void *)&out, (void *)&os, (void *)&flags, (void *)&n_tg, (void *)&n_rg};
+    hipError_t e = hipLaunchKernel(k, dim3((unsigned)((n_rg + 7) / 8 * 8 * n_tg)), dim3(64), args, 0,
+                                   ctx->stream);
+    if (e != hipSuccess) return fox_hip_fail(e, "gemv_float");
     FOX_LAUNCHED("gemv_float");
     return FOX_GPU_OK;
 }
