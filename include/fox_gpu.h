@@ -91,6 +91,10 @@ fox_gpu_status fox_gpu_free(fox_gpu_ctx *ctx, void *ptr);
 /* blocking copies; the device-to-host copy first waits for queued work */
 fox_gpu_status fox_gpu_memcpy_h2d(fox_gpu_ctx *ctx, void *dst, const void *src, size_t n);
 fox_gpu_status fox_gpu_memcpy_d2h(fox_gpu_ctx *ctx, void *dst, const void *src, size_t n);
+/* n <= 16 words into device memory, stream-ordered; the values travel with
+ * the call, so `words` may be reused at once and nothing waits (a step's
+ * token ids and position) */
+fox_gpu_status fox_gpu_store_u32(fox_gpu_ctx *ctx, uint32_t *dst, const uint32_t *words, size_t n);
 /* stream-ordered device copy and byte fill (a kernel, safe under capture) */
 fox_gpu_status fox_gpu_memcpy_d2d(fox_gpu_ctx *ctx, void *dst, const void *src, size_t n);
 fox_gpu_status fox_gpu_memset(fox_gpu_ctx *ctx, void *dst, int value, size_t n);

@@ -208,6 +208,27 @@ extern "C" fox_gpu_status fox_gpu_memcpy_d2h(fox_gpu_ctx *ctx, void *dst, const 
     return FOX_GPU_OK;
 }
 
+struct Words {
+    uint32_t w[16];
+};
+
+__global__ void store_u32_k(uint32_t *dst, int n, Words v)
+{
+    if ((int)threadIdx.x < n) dst[threadIdx.x] = v.w[threadIdx.x];
+}
+
+extern "C" fox_gpu_status fox_gpu_store_u32(fox_gpu_ctx *ctx, uint32_t *dst, const uint32_t *words,
+                                            size_t n)
+{
+    Words v = {};
+    if (!ctx || !dst || !words || n == 0 || n > 16)
+        return fox_fail(FOX_GPU_ERR_ARG, "store_u32: bad argument");
+    memcpy(v.w, words, n * sizeof(uint32_t));
+    hipLaunchKernelGGL(store_u32_k, dim3(1), dim3(64), 0, ctx->stream, dst, (int)n, v);
+    FOX_LAUNCHED("store_u32");
+    return FOX_GPU_OK;
+}
+
 extern "C" fox_gpu_status fox_gpu_memcpy_d2d(fox_gpu_ctx *ctx, void *dst, const void *src, size_t n)
 {
     if (!ctx || (!dst && n) || (!src && n)) return fox_fail(FOX_GPU_ERR_ARG, "memcpy_d2d: null pointer");

@@ -54,7 +54,10 @@ struct fox_context {
     float *kc, *vc, *rc, *rs;
     uint32_t *dtok, *dpos, *dhist, *dzero;
     float *norms;                  /* all norm vectors, n_embd floats each */
-    float *logits;                 /* host */
+    /* pinned host memory of log_rows rows, the first the last token's logits
+     * (copies to pageable memory pin it page by page each time) */
+    float *logits;
+    size_t log_rows;
     double last_seconds;
     uint64_t reads_at_start;
     /* batched passes: allocated at the first one (cap 0 before, and where
@@ -122,8 +125,8 @@ void fox_context_destroy(fox_context *c)
         fox_gpu_sync(c->gpu);
         for (i = 0; i < c->n_allocs; i++) fox_gpu_free(c->gpu, c->allocs[i]);
     }
+    if (c->logits) fox_gpu_host_free(c->gpu, c->logits);
     free(c->L);
-    free(c->logits);
     free(c);
 }
 
@@ -178,7 +181,13 @@ fox_status fox_context_create(fox_model *m, const fox_context_config *cfg, fox_c
     }
     nb = FOX_GPU_MAX_TOKENS;
 
-    c->logits = (float *)calloc(c->vocab, sizeof(float));
+    /* (up to nb rows where they are small: fox_eval_all's way out) */
+    c->log_rows = c->vocab ? ((size_t)1 << 18) / c->vocab : 1;
+    if (c->log_rows < 1) c->log_rows = 1;
+    if (c->log_rows > nb) c->log_rows = nb;
+    if (fox_gpu_host_alloc(c->gpu, (c->log_rows * c->vocab + 1) * sizeof(float),
+                           (void **)&c->logits) == FOX_GPU_OK)
+        memset(c->logits, 0, c->vocab * sizeof(float));
     c->L = (dev_layer *)calloc(mi->n_layer, sizeof(dev_layer));
     if (!c->logits || !c->L) { fox_context_destroy(c); return fox_fail(FOX_ERR_NOMEM, "context: tables"); }
 
@@ -196,12 +205,12 @@ fox_status fox_context_create(fox_model *m, const fox_context_config *cfg, fox_c
     ALLOC(c->vc, (size_t)mi->n_layer * FOX_GPU_V_CACHE_FLOATS(k.n_ctx, c->nkv) * 4)
     ALLOC(c->rc, (size_t)k.n_ctx * (c->hd / 2) * 4)
     ALLOC(c->rs, (size_t)k.n_ctx * (c->hd / 2) * 4)
-    ALLOC(c->dtok, nb * 4)
-    ALLOC(c->dpos, 4)
+    ALLOC(c->dtok, (nb + 1) * 4)                  /* the tokens, then the position */
     ALLOC(c->dhist, (size_t)k.n_ctx * 4)
     ALLOC(c->dzero, 4)
     ALLOC(c->norms, (2 * (size_t)mi->n_layer + 1) * c->d * 4)
 #undef ALLOC
+    c->dpos = c->dtok + nb;
     if (fox_gpu_memcpy_h2d(c->gpu, c->dzero, &zero, 4) != FOX_GPU_OK ||
         fox_gpu_memset(c->gpu, c->kc, 0, (size_t)mi->n_layer * k.n_ctx * c->nkv * 4) != FOX_GPU_OK ||
         fox_gpu_memset(c->gpu, c->vc, 0,
@@ -532,6 +541,19 @@ static fox_status batch_pass(fox_context *c, size_t M)
     return FOX_OK;
 }
 
+/* `rows` rows of logits to the caller's memory, through the pinned rows */
+static fox_status logits_out(fox_context *c, float *dst, const float *src, size_t rows)
+{
+    size_t i, r;
+    for (i = 0; i < rows; i += r) {
+        r = rows - i < c->log_rows ? rows - i : c->log_rows;
+        GPU(fox_gpu_memcpy_d2h(c->gpu, c->logits, src + i * c->vocab, r * c->vocab * 4),
+            "eval: logits");
+        memcpy(dst + i * c->vocab, c->logits, r * c->vocab * 4);
+    }
+    return FOX_OK;
+}
+
 /* the buffers of batched passes; 0 where they cannot be had */
 static int batch_ready(fox_context *c)
 {
@@ -569,7 +591,10 @@ static fox_status batch_eval(fox_context *c, const uint32_t *tokens, size_t M, i
     fox_status st;
     for (i = 0; i < np; i++) pos[i] = c->pos + (uint32_t)(i * FOX_GPU_MAX_TOKENS);
     GPU(fox_gpu_memcpy_h2d(c->gpu, c->B.tok, tokens, M * 4), "eval: tokens");
-    GPU(fox_gpu_memcpy_h2d(c->gpu, c->B.pos, pos, np * 4), "eval: position");
+    if (c->attn_mode == FOX_GPU_ATTN_EXACT)
+        GPU(fox_gpu_store_u32(c->gpu, c->B.pos, pos, 1), "eval: position");
+    else
+        GPU(fox_gpu_memcpy_h2d(c->gpu, c->B.pos, pos, np * 4), "eval: position");
     if ((st = batch_pass(c, M)) != FOX_OK) return st;
     if (!all) return last ? head(c, c->B.x + (M - 1) * c->d, c->B.xb, 1, c->dlogits) : FOX_OK;
     if (!c->blogits &&
@@ -578,8 +603,7 @@ static fox_status batch_eval(fox_context *c, const uint32_t *tokens, size_t M, i
     for (i = 0; i < M; i += r) {
         r = M - i < HEAD_ROWS ? M - i : HEAD_ROWS;
         if ((st = head(c, c->B.x + i * c->d, c->B.xb, r, c->blogits)) != FOX_OK) return st;
-        GPU(fox_gpu_memcpy_d2h(c->gpu, all + i * c->vocab, c->blogits, r * c->vocab * 4),
-            "eval: logits");
+        if ((st = logits_out(c, all + i * c->vocab, c->blogits, r)) != FOX_OK) return st;
     }
     return FOX_OK;
 }
@@ -639,12 +663,14 @@ static fox_status eval_chunks(fox_context *c, const uint32_t *tokens, size_t n, 
                 FOX_OK)
                 return st;
         } else {
-            GPU(fox_gpu_memcpy_h2d(c->gpu, c->dtok, tokens + done, chunk * 4), "eval: tokens");
-            GPU(fox_gpu_memcpy_h2d(c->gpu, c->dpos, &c->pos, 4), "eval: position");
+            uint32_t in[FOX_GPU_MAX_TOKENS + 1] = { 0 };
+            memcpy(in, tokens + done, chunk * 4);
+            in[FOX_GPU_MAX_TOKENS] = c->pos;               /* (dpos follows dtok) */
+            GPU(fox_gpu_store_u32(c->gpu, c->dtok, in, FOX_GPU_MAX_TOKENS + 1), "eval: tokens");
             if ((st = forward_pass(c, chunk, all ? 2 : last)) != FOX_OK) return st;
-            if (all)
-                GPU(fox_gpu_memcpy_d2h(c->gpu, all + done * c->vocab, c->dlogits,
-                                       chunk * c->vocab * 4), "eval: logits");
+            if (all &&
+                (st = logits_out(c, all + done * c->vocab, c->dlogits, chunk)) != FOX_OK)
+                return st;
         }
         c->pos += (uint32_t)chunk;
         done += chunk;
@@ -697,8 +723,8 @@ fox_status fox_decode_greedy(fox_context *c, uint32_t token, size_t n_steps, uin
                         "token context", n_steps, c->pos, c->cfg.n_ctx);
     if ((st = check_tokens(c, &token, 1)) != FOX_OK) return st;
     t0 = now_s();
-    GPU(fox_gpu_memcpy_h2d(c->gpu, c->dtok, &token, 4), "decode: token");
-    GPU(fox_gpu_memcpy_h2d(c->gpu, c->dpos, &c->pos, 4), "decode: position");
+    GPU(fox_gpu_store_u32(c->gpu, c->dtok, &token, 1), "decode: token");
+    GPU(fox_gpu_store_u32(c->gpu, c->dpos, &c->pos, 1), "decode: position");
     /* the first step runs eagerly (it also sizes every workspace), the rest
      * replay one captured graph; FOX_GRAPHS=0 keeps every step eager (for
      * profilers that cannot follow graph launches), and so does streaming
