@@ -1466,6 +1466,150 @@ __global__ __launch_bounds__(256) void attn_avm(const float *__restrict__ att, s
     }
 }
 
+// The values without a hand-over, where attn_avm's workgroups (one per compute
+// unit) would take several rounds: a workgroup of two waves per (query head,
+// CW = 64 / TPW columns, 2 TPW tokens), lane (token, column) running its whole
+// sum, a product and an add per position.  V quads and weights go through LDS
+// a block of BQ quads at a time, double buffered, two more blocks in flight in
+// registers.  A position costs about 17 clocks whatever the heads and tokens
+// up to two workgroups per compute unit, against attn_avm's 12 per round.
+// (27B-class heads, 8 tokens at 8200 positions, two rounds: 77.8 -> 61.3 us;
+// 80 heads over 16, whose five heads attn_avm pads to eight, 8 tokens at 6000
+// positions: attention 353 -> 126 us.  One round: 48 rows x 3 tokens at 7000
+// positions 35.8 there, 57.9 here.)
+template <int TPW>
+__global__ __launch_bounds__(128) void attn_avt(const float *__restrict__ att, size_t att_stride,
+                                                const float *__restrict__ vc, int n_head,
+                                                int n_head_kv, int hd,
+                                                const uint32_t *__restrict__ pos, int n_ctx,
+                                                float *__restrict__ out, size_t out_stride, int M)
+{
+    typedef float f4v __attribute__((ext_vector_type(4)));
+    constexpr int CW = 64 / TPW, TT = 2 * TPW, BQ = 1024 / CW, AS = BQ + 1;
+    constexpr int NA = (TT * BQ + 127) / 128;
+    __shared__ f4v Vs[2][BQ * CW], A[2][TT * AS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
+    // workgroup -> (column group u of the kv heads, query head, token group):
+    // everything that reads one column group on one XCD (blockIdx % 8)
+    const int G = n_head / n_head_kv, ncg = (hd + CW - 1) / CW, nr = G * ((M + TT - 1) / TT);
+    const int bx = blockIdx.x, rest = (bx >> 3) % nr, u = (bx & 7) + 8 * ((bx >> 3) / nr);
+    if (u >= n_head_kv * ncg) return;                      // (uniform: the grid's padding)
+    const int t0 = rest / G * TT, nt = min(TT, M - t0);
+    const int kvh = u / ncg, c0 = (u - kvh * ncg) * CW, h = kvh * G + rest % G;
+    const int kvd = n_head_kv * hd;
+    auto upto_of = [&](int tl) { return (int)min((size_t)pos[0] + (size_t)(t0 + tl) + 1, (size_t)n_ctx); };
+    const int nq_all = (upto_of(nt - 1) + 3) >> 2;         // quads of the longest token
+    const int nq_full = upto_of(0) >> 2;                   // quads whole for every token
+    const int nblk = (nq_all + BQ - 1) / BQ;
+    const int col = lane % CW, tl = wave * TPW + lane / CW;
+    const int my_upto = upto_of(min(tl, nt - 1));
+    struct Slot { f4v v[8], a[NA]; };
+    // thread tid's quads of block b: k (128 / CW) + tid / CW of column tid % CW,
+    // and of the weights quad idx % BQ of token idx / BQ, idx = tid + 128 k: a
+    // uniform address and a thread's constant offset, but for the last block,
+    // whose quads past the end repeat the last one
+    const char *vbase = (const char *)vc + ((size_t)kvh * hd + c0) * 16;
+    const char *abase = (const char *)(att + ((size_t)t0 * n_head + h) * att_stride);
+    const uint32_t vstep = (uint32_t)kvd * 16;             // bytes from quad to quad
+    const uint32_t vcol = (uint32_t)min(tid % CW, hd - 1 - c0) * 16;
+    const uint32_t voff = (uint32_t)(tid / CW) * vstep + vcol;
+    uint32_t arow[NA];
+#pragma unroll
+    for (int k = 0; k < NA; k++)
+        arow[k] = (uint32_t)min(min(tid + 128 * k, TT * BQ - 1) / BQ, nt - 1) * (uint32_t)(n_head * att_stride * 4);
+    auto load = [&](int b, Slot &s) __attribute__((always_inline)) {
+        if ((b + 1) * BQ <= nq_all) {                      // (uniform)
+            const char *vb = vbase + (size_t)(b * BQ) * vstep, *ab = abase + (size_t)(b * BQ) * 16;
+#pragma unroll
+            for (int k = 0; k < 8; k++) s.v[k] = *(const f4v *)(vb + (size_t)(k * (128 / CW)) * vstep + voff);
+#pragma unroll
+            for (int k = 0; k < NA; k++)
+                s.a[k] = *(const f4v *)(ab + (arow[k] + (uint32_t)(min(tid + 128 * k, TT * BQ - 1) % BQ) * 16));
+        } else {
+            b = min(b, nblk - 1);
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const int qq = min(b * BQ + tid / CW + k * (128 / CW), nq_all - 1);
+                s.v[k] = *(const f4v *)(vbase + (size_t)qq * vstep + vcol);
+            }
+#pragma unroll
+            for (int k = 0; k < NA; k++) {
+                const int qq = min(b * BQ + min(tid + 128 * k, TT * BQ - 1) % BQ, nq_all - 1);
+                s.a[k] = *(const f4v *)(abase + (arow[k] + (size_t)qq * 16));
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto stash = [&](int buf, const Slot &s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) Vs[buf][tid + 128 * k] = s.v[k];
+#pragma unroll
+        for (int k = 0; k < NA; k++) {
+            const int idx = tid + 128 * k;
+            if (idx < TT * BQ) A[buf][idx / BQ * AS + idx % BQ] = s.a[k];
+        }
+    };
+    float acc = 0.0f;
+    auto sums = [&](int b) __attribute__((always_inline)) {
+        const f4v *vp = Vs[b & 1] + col, *ap = A[b & 1] + tl * AS;
+        if ((b + 1) * BQ <= nq_full) {                     // (uniform)
+            // operands six quads ahead of their sums (each wave has its SIMD to
+            // itself: nobody else's work would cover the reads)
+            f4v v[8], w[8];
+            auto read = [&](int q) __attribute__((always_inline)) {
+                v[q & 7] = vp[q * CW];
+                w[q & 7] = ap[q];
+            };
+#pragma unroll
+            for (int q = 0; q < 6; q++) read(q);
+            // the next quad's products between this one's adds: an add issued
+            // right after the add or the product it needs would wait a state
+            f4v p = v[0] * w[0];
+#pragma unroll
+            for (int q = 0; q < BQ; q++) {
+                if (q + 6 < BQ) read(q + 6);
+                __builtin_amdgcn_sched_barrier(0);
+                f4v pn = p;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    if (q + 1 < BQ) pn[e] = v[(q + 1) & 7][e] * w[(q + 1) & 7][e];
+                    acc = acc + p[e];
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                p = pn;
+            }
+        } else {
+            const int n = min(BQ, nq_all - b * BQ);
+            for (int i = 0; i < n; i++) {
+                const f4v v = vp[i * CW], w = ap[i];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float s = acc + w[e] * v[e];
+                    acc = 4 * (b * BQ + i) + e < my_upto ? s : acc;
+                }
+            }
+        }
+    };
+    Slot s0, s1;
+    load(0, s0);
+    load(1, s1);
+    stash(0, s0);
+    load(2, s0);
+    __syncthreads();
+    // block b in LDS, b + 1 and b + 2 in registers
+    for (int b = 0; b < nblk; b += 2) {
+        sums(b);
+        stash((b + 1) & 1, s1);
+        load(b + 3, s1);
+        __syncthreads();
+        if (b + 1 < nblk) sums(b + 1);                     // (uniform)
+        stash(b & 1, s0);
+        load(b + 4, s0);
+        __syncthreads();
+    }
+    if (tl < nt && c0 + col < hd) out[(size_t)(t0 + tl) * out_stride + (size_t)h * hd + c0 + col] = acc;
+}
+
 fox_gpu_status fox_attn_softmax(fox_gpu_ctx *ctx, float *att, size_t att_stride, const float *tmax,
                                 int n_tiles, int n_head, const uint32_t *pos, int t_base, int n_ctx,
                                 int M)
@@ -1483,6 +1627,12 @@ fox_gpu_status fox_attn_softmax(fox_gpu_ctx *ctx, float *att, size_t att_stride,
                        ctx->stream, att, att_stride, tmax, n_tiles, n_head, pos, n_ctx, t_base);
     FOX_LAUNCHED("attention softmax");
     return FOX_GPU_OK;
+}
+
+// column groups of `cols` over the kv heads
+static size_t n_kv_groups(size_t n_head_kv, size_t head_dim, size_t cols)
+{
+    return n_head_kv * ((head_dim + cols - 1) / cols);
 }
 
 extern "C" fox_gpu_status fox_gpu_attention(fox_gpu_ctx *ctx, float *out, size_t out_stride,
@@ -1587,6 +1737,26 @@ extern "C" fox_gpu_status fox_gpu_attention(fox_gpu_ctx *ctx, float *out, size_t
         if ((st = fox_attn_softmax(ctx, att, att_stride, tmax, n_tiles, (int)n_head, pos, 0,
                                    (int)n_ctx, (int)M)))
             return st;
+        // one attn_avm workgroup per compute unit at a time (its LDS): more of
+        // them than compute units take several rounds, and attn_avt is faster
+        const size_t avm_wg = n_kv_groups(n_head_kv, head_dim, dcm) * ((M + MT - 1) / MT);
+        if (avm_wg > (size_t)ctx->n_cu && M > 1) {
+            // (eight tokens to a workgroup from five on, so that they share V;
+            // fewer leave a wave more columns)
+            const int tpw = M > 4 ? 4 : M > 2 ? 2 : 1, iM = (int)M;
+            const size_t nu = n_kv_groups(n_head_kv, head_dim, 64 / tpw);
+            const size_t nwg = (nu + 7) / 8 * 8 * gqa * ((M + 2 * tpw - 1) / (2 * tpw));
+            const void *av = tpw == 4 ? (const void *)attn_avt<4> : tpw == 2 ? (const void *)attn_avt<2>
+                                                                             : (const void *)attn_avt<1>;
+            const int in_head = (int)n_head;
+            void *args[] = {(void *)&att, (void *)&att_stride, (void *)&v_cache, (void *)&in_head,
+                            (void *)&ikv, (void *)&ihd, (void *)&pos, (void *)&ictx, (void *)&out,
+                            (void *)&os, (void *)&iM};
+            hipError_t e = hipLaunchKernel(av, dim3((unsigned)nwg), dim3(128), args, 0, ctx->stream);
+            if (e != hipSuccess) return fox_hip_fail(e, "attention values");
+            FOX_LAUNCHED("attention values");
+            return FOX_GPU_OK;
+        }
         const void *avm = gp == 1 ? (const void *)attn_avm<1> : gp == 2 ? (const void *)attn_avm<2>
                         : gp == 4 ? (const void *)attn_avm<4> : (const void *)attn_avm<8>;
         const size_t avm_lds = 2 * 64 * MV_PS * 16;

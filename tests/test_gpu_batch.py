@@ -178,3 +178,29 @@ def test_prompt_equals_passes_of_eight(tmp_path, name, over):
             assert c.position == 75 + 80
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("n_head,n_kv,hd,pos,M", [
+    (40, 8, 128, 250, 2), (80, 16, 128, 61, 4), (80, 16, 128, 127, 3), (40, 8, 100, 511, 7),
+    (32, 16, 128, 1020, 8), (64, 32, 64, 254, 5), (40, 8, 72, 0, 2),
+])
+def test_many_heads_equal_single_tokens(gpu, n_head, n_kv, hd, pos, M):
+    """Two to eight tokens of many heads (attn_avt: more value workgroups than
+    compute units): each token as a call of its own gives it."""
+    rng = np.random.default_rng(n_head + hd + M)
+    n_ctx, kvd = pos + M, n_kv * hd
+    K, V = (rng.standard_normal((n_ctx, kvd)).astype(np.float32) for _ in range(2))
+    V[-1, 0], V[-1, -1] = np.inf, np.nan           # (must not reach the tokens before)
+    kc = gpu.empty(n_ctx * kvd, np.float32)
+    vc = gpu.empty((n_ctx + 3) // 4 * 4 * kvd, np.float32)
+    gpu.kv_write(kc, vc, kvd, n_ctx, 0, gpu.array(K), gpu.array(V), n_ctx)
+    q = rng.standard_normal((M, n_head * hd)).astype(np.float32)
+    out = gpu.empty(M * n_head * hd, np.float32)
+    gpu.attention(out, gpu.array(q), kc, vc, n_head, n_kv, hd, M,
+                  gpu.array(np.array([pos], np.uint32)), n_ctx, rf.ATTN_EXACT)
+    got = out.numpy().reshape(M, -1)
+    for t in range(M):
+        o = gpu.empty(n_head * hd, np.float32)
+        gpu.attention(o, gpu.array(q[t]), kc, vc, n_head, n_kv, hd, 1,
+                      gpu.array(np.array([pos + t], np.uint32)), n_ctx, rf.ATTN_EXACT)
+        assert same_or_both_nan(got[t], o.numpy()), f"token {t}"
