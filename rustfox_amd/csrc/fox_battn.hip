@@ -3,7 +3,7 @@
 // bit-identical to the kernels of fox_ops.hip:
 //   batt_qk   scores: a thread owns a register tile of (token, position)
 //             pairs and adds their products in dimension order;
-//   attn_sm   (fox_ops.hip) the softmax per (head, token);
+//   batt_sm   the exps and their sum: a wave per 16 (or 4) tokens of a head;
 //   batt_av   values: a thread owns a register tile of (token, column) pairs
 //             and adds a_j v_j in position order.
 // With many tokens the independent sums fill the chip by themselves, so each
@@ -127,15 +127,107 @@ __global__ __launch_bounds__(256) void batt_qk(const float *__restrict__ q, size
     }
 }
 
+// Softmax of ROWS tokens of one head per wave, no wave waiting for another:
+// lane (r, c) = (lane / LPR, lane % LPR) computes four consecutive exps of row
+// r a chunk (16 LPR bytes a row), e_j = expf(s_j - max) goes back over the
+// scores and into the wave's LDS, and lane r of the first ROWS adds row r's
+// chunk in position order.  1 / sum is left in the row's first tile maximum
+// for batt_av, which forms a_j = e_j * (1 / sum) as it stages them.  Bound by
+// the exps (about 240 clocks per wave and element); the chains cost CP adds
+// per chunk of 256 exps, 16 with ROWS = 16.  ROWS = 4 where 16 would leave
+// most SIMDs without a wave.  (A workgroup per row, attn_sm, took 133 us per
+// layer for 1024 tokens of 32 heads.)
+template <int ROWS>
+__global__ __launch_bounds__(256) void batt_sm(float *__restrict__ att, size_t att_stride,
+                                               float *__restrict__ tmax, int n_tiles, int n_head,
+                                               const uint32_t *__restrict__ pos, int t_base,
+                                               int n_ctx, int M)
+{
+    constexpr int LPR = 64 / ROWS, CP = 4 * LPR, RS = LPR + 1;
+    __shared__ f4v E[4][ROWS * RS];
+    __shared__ uint64_t tab[32];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (tid < 32) tab[tid] = fox_exp2_tab[tid];
+    __syncthreads();
+    // (row groups from the last, longest one on)
+    const int h = blockIdx.x, g0 = ((M + ROWS - 1) / ROWS - 1 - ((int)blockIdx.y * 4 + wave)) * ROWS;
+    if (g0 < 0) return;                                    // (uniform over the wave)
+    const size_t pz = (size_t)pos[0] + (size_t)t_base;
+    auto upto_of = [&](int t) { return (int)min(pz + (size_t)min(t, M - 1) + 1, (size_t)n_ctx); };
+    const int r = lane / LPR, c = lane % LPR, t = min(g0 + r, M - 1);
+    const int upto = upto_of(t);
+    float *row = att + ((size_t)t * n_head + h) * att_stride;
+    float *tm = tmax + ((size_t)t * n_head + h) * n_tiles;
+    // src/ops.c:26-30: a NaN first score stays the maximum
+    float m = -INFINITY;
+    for (int i = c; i < (upto + BQ_POS - 1) / BQ_POS; i += LPR) {
+        const float v = tm[i];
+        m = v > m ? v : m;
+    }
+    auto mx = [](float a, float b) { return b > a ? b : a; };
+    m = mx(m, dpp_t<0xB1, 0xF>(m, m));
+    m = mx(m, dpp_t<0x4E, 0xF>(m, m));
+    if (LPR == 16) {
+        m = mx(m, dpp_t<0x141, 0xF>(m, m));
+        m = mx(m, dpp_t<0x140, 0xF>(m, m));
+    }
+    const float s0 = row[0];
+    if (s0 != s0) m = s0;
+    const int nch = (upto_of(g0 + ROWS - 1) + CP - 1) / CP, full = upto_of(g0) / CP;
+    const int up_ch = upto_of(g0 + (lane & (ROWS - 1)));   // of the row this lane sums
+    auto load = [&](int k) { return ((const f4v *)row)[min(k * LPR + c, (upto - 1) >> 2)]; };
+    f4v *Ew = E[wave];
+    f4v nxt = load(0);
+    float sum = 0.0f;
+    for (int k = 0; k < nch; k++) {
+        const f4v s = nxt;
+        nxt = load(min(k + 1, nch - 1));
+        const int j = k * CP + 4 * c;
+        f4v e;
+#pragma unroll
+        for (int i = 0; i < 4; i++) e[i] = fox_expf_t(s[i] - m, tab);
+        Ew[r * RS + c] = e;
+        if (j < upto && g0 + r < M) ((f4v *)row)[k * LPR + c] = e;
+        __builtin_amdgcn_wave_barrier();                   // (a wave's LDS accesses run in order)
+        if (lane < ROWS) {
+            const f4v *er = Ew + lane * RS;
+            if (k < full) {                                // (uniform)
+#pragma unroll
+                for (int q = 0; q < LPR; q++) {
+                    const f4v x = er[q];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) sum = sum + x[i];
+                }
+            } else {
+                for (int q = 0; q < LPR; q++) {
+                    const f4v x = er[q];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const float y = sum + x[i];
+                        sum = k * CP + 4 * q + i < up_ch ? y : sum;
+                    }
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    // src/ops.c:35-38: a_j = e_j * (1 / sum) when the sum is positive, else e_j
+    if (lane < ROWS && g0 + lane < M)
+        tmax[((size_t)(g0 + lane) * n_head + h) * n_tiles] = sum > 0.0f ? fox_div(1.0f, sum) : 1.0f;
+}
+
 // Values of one query head for CW columns and 256 * 4 / CW * TI tokens: thread
 // (cx, ty) = (tid % (CW / 4), tid / (CW / 4)) owns columns cx + CW / 4 * k and
 // tokens ty * TI + i.  Position quads are staged BV_Q at a time (the cache
 // keeps a column's four positions side by side); a quad costs TI + 4 LDS
 // reads and 32 TI vector instructions.  Positions at or past a token's end
-// are not added (quads that reach one take the masked form).
+// are not added (quads that reach one take the masked form).  att holds e_j,
+// inv each (token, head)'s factor, inv_stride apart.
 #define BV_Q 8
 template <int CW, int TI>
 __global__ __launch_bounds__(256) void batt_av(const float *__restrict__ att, size_t att_stride,
+                                               const float *__restrict__ inv, int inv_stride,
                                                const float *__restrict__ vc, int n_head,
                                                int n_head_kv, int hd,
                                                const uint32_t *__restrict__ pos, int t_base,
@@ -157,6 +249,12 @@ __global__ __launch_bounds__(256) void batt_av(const float *__restrict__ att, si
     const int nq_max = (upto_of(t_last) + 3) >> 2;         // quads of the longest token
     const int nq_full = upto_of(t0) >> 2;                  // quads whole for every token
     f4v vr[NV], ar[NA];
+    float ai[NA];
+#pragma unroll
+    for (int u = 0; u < NA; u++) {
+        const int idx = min(tid + 256 * u, TT * BV_Q - 1), t = min(t0 + idx / BV_Q, t_last);
+        ai[u] = inv[((size_t)t * n_head + h) * inv_stride];
+    }
     auto fetch = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < NV; u++) {
@@ -177,7 +275,7 @@ __global__ __launch_bounds__(256) void batt_av(const float *__restrict__ att, si
 #pragma unroll
         for (int u = 0; u < NA; u++) {
             const int idx = tid + 256 * u;
-            if (idx < TT * BV_Q) A[buf][idx / BV_Q * AS + idx % BV_Q] = ar[u];
+            if (idx < TT * BV_Q) A[buf][idx / BV_Q * AS + idx % BV_Q] = ar[u] * ai[u];
         }
     };
     float acc[TI][4];
@@ -301,8 +399,17 @@ extern "C" fox_gpu_status fox_gpu_batch_attention(fox_gpu_ctx *ctx, float *out, 
             if (e != hipSuccess) return fox_hip_fail(e, "attention scores");
             FOX_LAUNCHED("attention scores");
         }
-        if ((st = fox_attn_softmax(ctx, att, att_stride, tmax, n_tiles, inh, pos, itb, ictx, m)))
-            return st;
+        {
+            const bool r16 = (size_t)((m + 15) / 16) * n_head >= 4 * (size_t)ctx->n_cu;
+            const int rows = r16 ? 16 : 4;
+            const void *k = r16 ? (const void *)batt_sm<16> : (const void *)batt_sm<4>;
+            void *args[] = {(void *)&att, (void *)&att_stride, (void *)&tmax, (void *)&n_tiles,
+                            (void *)&inh, (void *)&pos, (void *)&itb, (void *)&ictx, (void *)&m};
+            hipError_t e = hipLaunchKernel(k, dim3((unsigned)n_head, (unsigned)((m + 4 * rows - 1) / (4 * rows))),
+                                           dim3(256), args, 0, ctx->stream);
+            if (e != hipSuccess) return fox_hip_fail(e, "attention softmax");
+            FOX_LAUNCHED("attention softmax");
+        }
         {
             // tokens per thread: as many as leave every compute unit two
             // workgroups
@@ -315,7 +422,8 @@ extern "C" fox_gpu_status fox_gpu_batch_attention(fox_gpu_ctx *ctx, float *out, 
                                                                  : (const void *)batt_av<w, 1>)
             const void *k = cw == 64 ? FOX_AV(64) : FOX_AV(128);
 #undef FOX_AV
-            void *args[] = {(void *)&att, (void *)&att_stride, (void *)&v_cache, (void *)&inh,
+            void *args[] = {(void *)&att, (void *)&att_stride, (void *)&tmax, (void *)&n_tiles, (void *)&v_cache,
+                            (void *)&inh,
                             (void *)&ikv, (void *)&ihd, (void *)&pos, (void *)&itb, (void *)&ictx,
                             (void *)&orow, (void *)&out_stride, (void *)&m};
             hipError_t e = hipLaunchKernel(k, dim3((unsigned)n_head, (unsigned)((m + ny * ti - 1) / (ny * ti)),

@@ -192,13 +192,6 @@ fox_gpu_status fox_gemv_launch(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor 
 fox_gpu_status fox_float_gemv(fox_gpu_ctx *ctx, const fox_gpu_tensor *w, const float *x,
                               size_t x_stride, size_t M, float *out, size_t out_stride,
                               unsigned flags);
-// exact attention's softmax over M tokens' scores (fox_ops.hip): att
-// [token][head][att_stride], tmax [token][head][n_tiles] maxima of 64
-// positions; the weights a_j are written over the scores.  Token t is at
-// position pos[0] + t_base + t
-fox_gpu_status fox_attn_softmax(fox_gpu_ctx *ctx, float *att, size_t att_stride, const float *tmax,
-                                int n_tiles, int n_head, const uint32_t *pos, int t_base, int n_ctx,
-                                int M);
 // K-quant products of several tokens (fox_batch.hip); FOX_GPU_ERR_UNSUPPORTED
 // (no error recorded) for inputs not 16-byte aligned and very wide rows
 fox_gpu_status fox_few_gemv(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor *const *ws,

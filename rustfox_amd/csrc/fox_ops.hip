@@ -1237,7 +1237,7 @@ __global__ __launch_bounds__(256) void attn_hv(const float *__restrict__ att, si
 __global__ __launch_bounds__(256) void attn_sm(float *__restrict__ att, size_t att_stride,
                                                const float *__restrict__ tmax, int n_tiles,
                                                int n_head, const uint32_t *__restrict__ pos,
-                                               int n_ctx, int t_base)
+                                               int n_ctx)
 {
     extern __shared__ float4 sm_lds[];
     float *e = (float *)sm_lds;                    // [ceil4(upto)]
@@ -1245,7 +1245,7 @@ __global__ __launch_bounds__(256) void attn_sm(float *__restrict__ att, size_t a
     __shared__ uint64_t tab[32];
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_index();
     const int h = blockIdx.x, t = blockIdx.y;
-    const int upto = (int)min((size_t)pos[0] + (size_t)(t_base + t) + 1, (size_t)n_ctx);
+    const int upto = (int)min((size_t)pos[0] + (size_t)t + 1, (size_t)n_ctx);
     float *row = att + ((size_t)t * n_head + h) * att_stride;
     const bool producer = wave > 0;
     const int L = tid - 64;
@@ -1610,9 +1610,8 @@ __global__ __launch_bounds__(128) void attn_avt(const float *__restrict__ att, s
     if (tl < nt && c0 + col < hd) out[(size_t)(t0 + tl) * out_stride + (size_t)h * hd + c0 + col] = acc;
 }
 
-fox_gpu_status fox_attn_softmax(fox_gpu_ctx *ctx, float *att, size_t att_stride, const float *tmax,
-                                int n_tiles, int n_head, const uint32_t *pos, int t_base, int n_ctx,
-                                int M)
+static fox_gpu_status attn_softmax(fox_gpu_ctx *ctx, float *att, size_t att_stride, const float *tmax,
+                                   int n_tiles, int n_head, const uint32_t *pos, int n_ctx, int M)
 {
     // (SUM_CHUNK floats past the weights: softmax_sum_block reads whole
     // chunks of SUM_CHUNK)
@@ -1624,7 +1623,7 @@ fox_gpu_status fox_attn_softmax(fox_gpu_ctx *ctx, float *att, size_t att_stride,
         if (e != hipSuccess) return fox_hip_fail(e, "attention: LDS size");
     }
     hipLaunchKernelGGL(attn_sm, dim3((unsigned)n_head, (unsigned)M), dim3(256), sm_lds,
-                       ctx->stream, att, att_stride, tmax, n_tiles, n_head, pos, n_ctx, t_base);
+                       ctx->stream, att, att_stride, tmax, n_tiles, n_head, pos, n_ctx);
     FOX_LAUNCHED("attention softmax");
     return FOX_GPU_OK;
 }
@@ -1734,8 +1733,7 @@ extern "C" fox_gpu_status fox_gpu_attention(fox_gpu_ctx *ctx, float *out, size_t
         // workgroup
         const int gp = gqa == 1 ? 1 : gqa == 2 ? 2 : gqa <= 4 ? 4 : 8;
         const size_t dcm = AV_CH / gp;
-        if ((st = fox_attn_softmax(ctx, att, att_stride, tmax, n_tiles, (int)n_head, pos, 0,
-                                   (int)n_ctx, (int)M)))
+        if ((st = attn_softmax(ctx, att, att_stride, tmax, n_tiles, (int)n_head, pos, (int)n_ctx, (int)M)))
             return st;
         // one attn_avm workgroup per compute unit at a time (its LDS): more of
         // them than compute units take several rounds, and attn_avt is faster
