@@ -1320,9 +1320,10 @@ static fox_gpu_status batch_run(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor
     return FOX_GPU_OK;
 }
 
-// fox_gpu_gemv's and fox_gpu_gemv_multi's K-quant products of 2 to
-// FOX_GPU_MAX_TOKENS tokens (arguments checked by the caller; the prepared
-// operand is smaller than gemv_blocks's, which `fixed` is sized for)
+// fox_gpu_gemv's and fox_gpu_gemv_multi's products of 2 to FOX_GPU_MAX_TOKENS
+// tokens that fox_fused_gemv leaves: the K-quants and some ternary ones
+// (arguments checked by the caller; `fixed` holds FOX_NOALLOC_SCRATCH bytes,
+// several times the operand of the widest row batch_run takes)
 fox_gpu_status fox_few_gemv(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor *const *ws,
                             const float *x, size_t x_stride, size_t M, float *const *outs,
                             const size_t *out_strides, unsigned flags, uint8_t *fixed)

@@ -1696,6 +1696,20 @@ static fox_gpu_status fused_go(fox_gpu_ctx *ctx, const FusedArgs &a, int grid, u
 
 // (the K-quant kernels take f32 input and write outputs: int8 input with
 // per-block scales and the block-sum requests take the unfused path)
+// Ternary products of several tokens that batch_gemm (fox_batch.hip) runs
+// faster: where the operand and the terms leave room for one workgroup per
+// compute unit only (above 80 KB) and that one would take several rounds of
+// items.  (8 tokens, us here / there: gate/up 2 x 21504 x 5376 30.2 / 24.4,
+// 24000 x 8192 25.6 / 19.7; two workgroups per compute unit, 24000 x 5376 15.5 /
+// 15.9; one round, 2560 x 9728 9.5 / 10.5.)  Wider rows than five input
+// dwords per thread stay (19968 x 20000, 4 tokens: 34.6 / 37.0), and so does a
+// capped grid.
+static bool batch_better(const fox_gpu_ctx *ctx, int fmt, size_t K, size_t M, int nslab, size_t n_work)
+{
+    return fmt == FMT_TQ2 && M > 2 && ctx->max_wg == 0 && n_work >= 2 * (size_t)ctx->n_cu &&
+           K <= 5 * 4 * FWG && fused_lds(fmt, (int)K, (int)M, nslab).total > 80 * 1024;
+}
+
 // (fixed: the caller's scratch for fused_prep's output, or null for the
 // context's workspace)
 template <int IN, int EPI>
@@ -1769,6 +1783,8 @@ fox_gpu_status fox_fused_gemv(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor *
     a.q_in = q;
     a.scale_in = scale;
     a.sums = sums;
+    if (x && outs && !sums && batch_better(ctx, fmt, K, M, 1, (size_t)tiles))
+        return FOX_GPU_ERR_UNSUPPORTED;                    // (fox_few_gemv takes it)
     if ((!x && !q) || (!sums && (!outs || (q && !scale))))
         return fox_fail(FOX_GPU_ERR_ARG, "fused gemv: missing activations, scale or output");
     if (sums) return fused_dispatch<IN_Q, EPI_SUMS>(ctx, fmt, a, tiles);
@@ -1932,6 +1948,8 @@ extern "C" fox_gpu_status fox_gpu_gate_up_silu(fox_gpu_ctx *ctx, const fox_gpu_t
                          str, M))
             return fox_fail(FOX_GPU_ERR_ARG, "gate_up_silu: h_out overlaps the input");
     }
+    if (batch_better(ctx, fmt, K, M, 2, (size_t)wg->n_tiles))
+        return fox_gpu_batch_gate_up_silu(ctx, wg, wu, x, x_stride, M, norm_w, eps, h_out, h_stride);
     const fox_gpu_tensor *ws[2] = {wg, wu};
     float *outs[2] = {h_out, nullptr};
     size_t strides[2] = {h_stride, h_stride};

@@ -790,7 +790,7 @@ static fox_gpu_status gemv_launch_ws(fox_gpu_ctx *ctx, size_t n, const fox_gpu_t
                             need, fixed_cap);
         act_layout(fmt, K, M, fixed_ws, &w);
     }
-    if (x && !sums && M > 1 && fmt != FMT_TQ2) {
+    if (x && !sums && M > 1) {
         st = fox_few_gemv(ctx, n, ws, x, x_stride, M, outs, out_strides, flags, fixed_ws);
         if (st != FOX_GPU_ERR_UNSUPPORTED) return st;
     }

@@ -192,7 +192,7 @@ fox_gpu_status fox_gemv_launch(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor 
 fox_gpu_status fox_float_gemv(fox_gpu_ctx *ctx, const fox_gpu_tensor *w, const float *x,
                               size_t x_stride, size_t M, float *out, size_t out_stride,
                               unsigned flags);
-// K-quant products of several tokens (fox_batch.hip); FOX_GPU_ERR_UNSUPPORTED
+// products of several tokens that the one-launch path leaves (fox_batch.hip); FOX_GPU_ERR_UNSUPPORTED
 // (no error recorded) for inputs not 16-byte aligned and very wide rows
 fox_gpu_status fox_few_gemv(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor *const *ws,
                             const float *x, size_t x_stride, size_t M, float *const *outs,
