@@ -257,7 +257,8 @@ fox_weights          *fox_model_weights(fox_model *m);
 /* include/fox/fox.h:433-451 */
 typedef struct {
     uint32_t n_ctx;
-    uint32_t n_batch;
+    uint32_t n_batch;     /* up to 8: tokens per pass; more: passes of up to 1024
+                             (results do not depend on it) */
     int      n_threads;   /* kept for the ABI; the GPU path ignores it */
 } fox_context_config;
 

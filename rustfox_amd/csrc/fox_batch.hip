@@ -1,5 +1,7 @@
 // fox_batch.hip -- projections of a batched pass (a prompt's tokens, more
-// than the FOX_GPU_MAX_TOKENS of the decode kernels), bit-identical to them.
+// than the FOX_GPU_MAX_TOKENS of the decode kernels), bit-identical to them,
+// and of a few tokens where the one-launch kernels of fox_fused.hip do not
+// apply (few_gemm: the K-quants) or are slower.
 //
 // batch_prep quantises the tokens once (optionally RMS-normalised first), a
 // workgroup per token, and batch_gemm is an int8 MFMA matrix product over
@@ -24,8 +26,8 @@
 // codes, 28 shared by the wave's token tiles) and by the vector unit on the
 // K-quants (5 instructions per 32-element sub-block and output for Q4_K).
 // Measured: two 4B-class layers over a 1024-token prompt 22.0 ms in passes of
-// eight, 1.32 ms batched; two 8B-class layers over 77 tokens on 1024 cached
-// rows 7.24 -> 1.02 ms.  A 1024-token gate/up (2 x 9728 x 2560, ternary) takes
+// eight, 1.12 ms batched; two 8B-class layers over 77 tokens on 1024 cached
+// rows 7.24 -> 0.71 ms.  A 1024-token gate/up (2 x 9728 x 2560, ternary) takes
 // 100 us, a 77-token one of the 8B class (Q4_K, 2 x 14336 x 4096) 77 us.
 #include "fox_gemv_dev.h"
 #include "fox_math.h"
@@ -719,8 +721,8 @@ __global__ __launch_bounds__(BT_THREADS, 2) void batch_gemm(BatchArgs a)
 //     half's activations zero), or Q6_K's quarters 2h and 2h + 1 (one
 //     sub-group at a time, the other lane groups' activations zero), so a lane
 //     forms the terms of its half only.
-// Q4_K 14336 x 4096, 8 tokens: 55.2 us in the workgroup-of-four kernel this
-// replaces.
+// Q4_K 14336 x 4096, 8 tokens, preparation included: 13.1 us (55.2 with
+// act_prep and gemv_blocks); Q6_K 4096 x 14336: 17.8 (93).
 template <int FMT>
 struct FewTerms;                        // one lane's terms of a block, per token k
 template <>

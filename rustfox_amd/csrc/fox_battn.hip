@@ -9,7 +9,9 @@
 // With many tokens the independent sums fill the chip by themselves, so each
 // runs one add at a time in its own register and the kernels are bound by
 // the vector unit: a product and an add per term (the reference rounds both,
-// so neither a fused multiply-add nor the matrix cores apply).
+// so neither a fused multiply-add nor the matrix cores apply).  A 1024-token
+// prompt of 32 heads of 128: scores 114 us and values 110 us per layer, where
+// the vector unit needs 109 each (2.15 G terms, a product and an add each).
 #include "fox_internal.h"
 #include "fox_gemv_dev.h"
 #include "fox_math.h"

@@ -12,6 +12,11 @@
 //     the reference's row loop does (ternary.c:226-246, 303-325, kernels.c:571-661),
 //     so outputs equal the reference built without FMA contraction.
 //
+// Products of f32 activations run in fox_fused.hip (ternary, and one token of
+// the K-quants) and fox_batch.hip (several tokens of the K-quants, wide ternary
+// rows); the block kernel here serves given int8 activations, block sums and
+// inputs that are not 16-byte aligned.
+//
 // Work split: one workgroup (4 waves) per 16-row tile and segment; waves take
 // 256-element blocks round-robin; each block is one 16 x 256 slab reduced by
 // four v_mfma_i32_16x16x64_i8, the token dimension (M <= 8) riding in the

@@ -778,7 +778,10 @@ __global__ __launch_bounds__(256) void attn_fdm(const float *__restrict__ part,
 //   attn_sm + attn_avm   several tokens, or a context longer than attn_hv's
 //             LDS holds: the softmax per (head, token), a_j written over the
 //             scores, then the value chains of MT tokens per workgroup fed by
-//             the same block pipeline as attn_hv.
+//             the same block pipeline as attn_hv;
+//   attn_avt  in its place where its workgroups outnumber the compute units:
+//             a lane per (query head, token, column), products and adds in one.
+// (More than eight tokens, a batched pass: fox_battn.hip.)
 
 #define SC_TILE 64
 #define QK_TPW 4            // tokens per scores workgroup (the K tile is read once for them)

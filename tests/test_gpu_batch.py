@@ -204,3 +204,20 @@ def test_many_heads_equal_single_tokens(gpu, n_head, n_kv, hd, pos, M):
         gpu.attention(o, gpu.array(q[t]), kc, vc, n_head, n_kv, hd, 1,
                       gpu.array(np.array([pos + t], np.uint32)), n_ctx, rf.ATTN_EXACT)
         assert same_or_both_nan(got[t], o.numpy()), f"token {t}"
+
+
+def test_streamed_prompt_equals_resident(tmp_path):
+    """A batched prompt over layers streamed through slots: the resident
+    model's logits."""
+    s = synth.spec("tiny-512", n_ctx=128)
+    path = str(tmp_path / "m.gguf")
+    synth.write_gguf(path, s)
+    ids = synth.prompt_ids(100, s.n_vocab)
+    with rf.Model(path) as m:
+        c = m.context(128)
+        want = c.eval(ids).copy()
+        c.close()
+    with rf.Model(path, mode=rf.WEIGHTS_STREAM) as m:
+        c = m.context(128)
+        assert np.array_equal(bits(c.eval(ids)), bits(want))
+        c.close()
