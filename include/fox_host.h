@@ -275,7 +275,8 @@ fox_status fox_eval(fox_context *ctx, const uint32_t *tokens, size_t n_tokens,
  * those of token i (as fox_eval would return after tokens[0..i]), into
  * caller-owned host memory of n_tokens * n_vocab floats: speculative
  * verification checks all drafted positions in one pass.  RustFox computes
- * the last position's only (src/forward.c:401-408). */
+ * the last position's only (src/forward.c:401-408).  The row an earlier
+ * fox_eval handed out is left as it is. */
 fox_status fox_eval_all(fox_context *ctx, const uint32_t *tokens, size_t n_tokens,
                         float *logits);
 uint32_t   fox_context_position(const fox_context *ctx);

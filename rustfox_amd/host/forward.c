@@ -54,9 +54,10 @@ struct fox_context {
     float *kc, *vc, *rc, *rs;
     uint32_t *dtok, *dpos, *dhist, *dzero;
     float *norms;                  /* all norm vectors, n_embd floats each */
-    /* pinned host memory of log_rows rows, the first the last token's logits
-     * (copies to pageable memory pin it page by page each time) */
-    float *logits;
+    /* pinned host memory (copies to pageable memory pin it page by page each
+     * time): the row fox_eval hands out, then log_rows rows that
+     * fox_eval_all's logits pass through */
+    float *logits, *log_stage;
     size_t log_rows;
     double last_seconds;
     uint64_t reads_at_start;
@@ -181,13 +182,15 @@ fox_status fox_context_create(fox_model *m, const fox_context_config *cfg, fox_c
     }
     nb = FOX_GPU_MAX_TOKENS;
 
-    /* (up to nb rows where they are small: fox_eval_all's way out) */
+    /* (fox_eval_all's way out: up to nb rows where they are small) */
     c->log_rows = c->vocab ? ((size_t)1 << 18) / c->vocab : 1;
     if (c->log_rows < 1) c->log_rows = 1;
     if (c->log_rows > nb) c->log_rows = nb;
-    if (fox_gpu_host_alloc(c->gpu, (c->log_rows * c->vocab + 1) * sizeof(float),
-                           (void **)&c->logits) == FOX_GPU_OK)
+    if (fox_gpu_host_alloc(c->gpu, ((1 + c->log_rows) * c->vocab + 1) * sizeof(float),
+                           (void **)&c->logits) == FOX_GPU_OK) {
         memset(c->logits, 0, c->vocab * sizeof(float));
+        c->log_stage = c->logits + c->vocab;
+    }
     c->L = (dev_layer *)calloc(mi->n_layer, sizeof(dev_layer));
     if (!c->logits || !c->L) { fox_context_destroy(c); return fox_fail(FOX_ERR_NOMEM, "context: tables"); }
 
@@ -547,9 +550,9 @@ static fox_status logits_out(fox_context *c, float *dst, const float *src, size_
     size_t i, r;
     for (i = 0; i < rows; i += r) {
         r = rows - i < c->log_rows ? rows - i : c->log_rows;
-        GPU(fox_gpu_memcpy_d2h(c->gpu, c->logits, src + i * c->vocab, r * c->vocab * 4),
+        GPU(fox_gpu_memcpy_d2h(c->gpu, c->log_stage, src + i * c->vocab, r * c->vocab * 4),
             "eval: logits");
-        memcpy(dst + i * c->vocab, c->logits, r * c->vocab * 4);
+        memcpy(dst + i * c->vocab, c->log_stage, r * c->vocab * 4);
     }
     return FOX_OK;
 }
