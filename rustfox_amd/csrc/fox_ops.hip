@@ -1741,7 +1741,10 @@ extern "C" fox_gpu_status fox_gpu_attention(fox_gpu_ctx *ctx, float *out, size_t
         // one attn_avm workgroup per compute unit at a time (its LDS): more of
         // them than compute units take several rounds, and attn_avt is faster
         const size_t avm_wg = n_kv_groups(n_head_kv, head_dim, dcm) * ((M + MT - 1) / MT);
-        if (avm_wg > (size_t)ctx->n_cu && M > 1) {
+        // (attn_avt's lanes address the up to eight rows of a workgroup with
+        // 32-bit byte offsets)
+        const bool near_rows = 8 * n_head * att_stride * sizeof(float) <= (size_t)1 << 32;
+        if (avm_wg > (size_t)ctx->n_cu && M > 1 && near_rows) {
             // (eight tokens to a workgroup from five on, so that they share V;
             // fewer leave a wave more columns)
             const int tpw = M > 4 ? 4 : M > 2 ? 2 : 1, iM = (int)M;

@@ -206,6 +206,27 @@ def test_many_heads_equal_single_tokens(gpu, n_head, n_kv, hd, pos, M):
         assert same_or_both_nan(got[t], o.numpy()), f"token {t}"
 
 
+def test_weights_past_32_bit_offsets(gpu):
+    """Score rows of 5120 heads over a 32768-position cache: eight tokens' rows
+    are more than 4 GB apart."""
+    rng = np.random.default_rng(1)
+    n_head, n_kv, hd, pos, M, n_ctx = 5120, 640, 4, 70, 8, 32768
+    n, kvd = pos + M, n_kv * hd
+    K, V = (rng.standard_normal((n, kvd)).astype(np.float32) for _ in range(2))
+    kc, vc = (gpu.empty(n_ctx * kvd, np.float32) for _ in range(2))
+    gpu.kv_write(kc, vc, kvd, n_ctx, 0, gpu.array(K), gpu.array(V), n)
+    q = rng.standard_normal((M, n_head * hd)).astype(np.float32)
+    out = gpu.empty(M * n_head * hd, np.float32)
+    gpu.attention(out, gpu.array(q), kc, vc, n_head, n_kv, hd, M,
+                  gpu.array(np.array([pos], np.uint32)), n_ctx, rf.ATTN_EXACT)
+    got = out.numpy().reshape(M, -1)
+    for t in range(M):
+        o = gpu.empty(n_head * hd, np.float32)
+        gpu.attention(o, gpu.array(q[t]), kc, vc, n_head, n_kv, hd, 1,
+                      gpu.array(np.array([pos + t], np.uint32)), n_ctx, rf.ATTN_EXACT)
+        assert np.array_equal(bits(got[t]), bits(o.numpy())), f"token {t}"
+
+
 def test_streamed_prompt_equals_resident(tmp_path):
     """A batched prompt over layers streamed through slots: the resident
     model's logits."""
