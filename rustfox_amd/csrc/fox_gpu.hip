@@ -17,6 +17,10 @@ fox_gpu_status fox_fail(fox_gpu_status st, const char *fmt, ...)
     va_start(ap, fmt);
     vsnprintf(g_err, sizeof(g_err), fmt, ap);
     va_end(ap);
+    // a HIP call's failure is reported here and now: left pending, the next
+    // launch check would report it again, for a call that worked (a caller
+    // may go on after a refused allocation)
+    if (st == FOX_GPU_ERR_NOMEM || st == FOX_GPU_ERR_INTERNAL) (void)hipGetLastError();
     return st;
 }
 

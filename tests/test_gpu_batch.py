@@ -242,3 +242,16 @@ def test_streamed_prompt_equals_resident(tmp_path):
         c = m.context(128)
         assert np.array_equal(bits(c.eval(ids)), bits(want))
         c.close()
+
+
+def test_a_refused_allocation_fails_no_later_call(gpu):
+    """An allocation that the device refuses is that call's error only: the
+    next launch does not report it again."""
+    x = np.random.default_rng(2).standard_normal((9, 512)).astype(np.float32)
+    W = weights(np.random.default_rng(3), TYPES["TQ2_0"], 40, 512)
+    w, dx, out = gpu.tensor(TYPES["TQ2_0"], 512, 40, W), gpu.array(x), gpu.empty(9 * 40, np.float32)
+    with pytest.raises(rf.FoxError) as e:
+        gpu.empty(1 << 48, np.float32)
+    assert e.value.status == 3
+    gpu.batch_gemv([w], dx, 9, [out])
+    assert np.isfinite(out.numpy()).all()
