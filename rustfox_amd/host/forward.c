@@ -31,8 +31,10 @@ typedef struct {
     float *attn_norm, *ffn_norm;   /* device f32 [n_embd] */
 } dev_layer;
 
-/* device activations of a pass of up to `cap` tokens */
+/* device activations of a pass of up to `cap` tokens: one allocation, carved,
+ * and hb2, which only a gate/up that runs as two products needs */
 typedef struct {
+    void  *block;
     float *x, *xb, *q, *k, *v, *hb, *hb2;
     uint32_t *tok, *pos;           /* pos[i]: the position of token 8 i */
     size_t cap;
@@ -61,8 +63,9 @@ struct fox_context {
     size_t log_rows;
     double last_seconds;
     uint64_t reads_at_start;
-    /* batched passes: allocated at the first one (cap 0 before, and where
-     * the memory is not there: passes of FOX_GPU_MAX_TOKENS then) */
+    /* batched passes: allocated at the first one and again at a larger one
+     * (cap 0 before, and where the memory is not there: passes of
+     * FOX_GPU_MAX_TOKENS then) */
     pass_buffers B;
     float *blogits;                /* HEAD_ROWS rows, at the first batched fox_eval_all */
     int no_batch;
@@ -117,6 +120,13 @@ void fox_context_config_default(fox_context_config *cfg, const fox_model *m)
     if (cfg->n_ctx == 0) cfg->n_ctx = 2048;
 }
 
+static void batch_free(fox_context *c)
+{
+    fox_gpu_free(c->gpu, c->B.hb2);
+    fox_gpu_free(c->gpu, c->B.block);
+    memset(&c->B, 0, sizeof(c->B));
+}
+
 void fox_context_destroy(fox_context *c)
 {
     int i;
@@ -124,6 +134,7 @@ void fox_context_destroy(fox_context *c)
     if (c->greedy) fox_gpu_graph_free(c->greedy);
     if (c->gpu) {
         fox_gpu_sync(c->gpu);
+        batch_free(c);
         for (i = 0; i < c->n_allocs; i++) fox_gpu_free(c->gpu, c->allocs[i]);
     }
     if (c->logits) fox_gpu_host_free(c->gpu, c->logits);
@@ -532,6 +543,10 @@ static fox_status batch_pass(fox_context *c, size_t M)
             const fox_gpu_tensor *gu[2] = { D->ffn_gate, D->ffn_up };
             float *out[2] = { B->hb, B->hb2 };
             size_t str[2] = { c->ff, c->ff };
+            if (!B->hb2) {
+                GPU(fox_gpu_malloc(c->gpu, B->cap * c->ff * 4, (void **)&B->hb2), "forward: swiglu");
+                out[1] = B->hb2;
+            }
             if ((st = project_group(c, 2, gu, B->x, B->xb, M, D->ffn_norm, out, str)) != FOX_OK)
                 return st;
             GPU(fox_gpu_silu_mul(c->gpu, B->hb, B->hb2, c->ff, M, c->ff), "forward: swiglu");
@@ -557,31 +572,39 @@ static fox_status logits_out(fox_context *c, float *dst, const float *src, size_
     return FOX_OK;
 }
 
-/* the buffers of batched passes; 0 where they cannot be had */
-static int batch_ready(fox_context *c)
+/* the buffers of batched passes of n tokens, or of as many as can be had (B.cap);
+ * 0 where none can.  Sized in steps, so that a short prompt does not pay for a
+ * long one's memory; they grow with the prompts.  (Nine allocations for 1024
+ * tokens made a context's first prompt of nine tokens 0.2 ms slower than
+ * its second, and than two passes of the decode kernels.) */
+static int batch_ready(fox_context *c, size_t n)
 {
     pass_buffers b;
-    struct { float **p; size_t n; } want[7] = {
+    struct { void *p; size_t row; } part[8] = {
         { &b.x, c->d }, { &b.xb, c->wide }, { &b.q, c->nq }, { &b.k, c->nkv }, { &b.v, c->nkv },
-        { &b.hb, c->ff }, { &b.hb2, c->ff }
+        { &b.hb, c->ff }, { &b.tok, 1 }, { &b.pos, 1 }
     };
-    const int mark = c->n_allocs;
-    size_t i;
-    int ok = 1;
-    if (c->B.cap) return 1;
+    size_t cap = 64, i;
+    if (c->B.cap >= n) return 1;
     if (c->no_batch) return 0;
-    b.cap = c->cfg.n_ctx < FOX_GPU_BATCH_TOKENS ? c->cfg.n_ctx : FOX_GPU_BATCH_TOKENS;
-    for (i = 0; ok && i < 7; i++)
-        ok = dalloc(c, b.cap * want[i].n * 4, (void **)want[i].p) == FOX_OK;
-    ok = ok && dalloc(c, b.cap * 4, (void **)&b.tok) == FOX_OK;
-    ok = ok && dalloc(c, (b.cap / FOX_GPU_MAX_TOKENS + 1) * 4, (void **)&b.pos) == FOX_OK;
-    if (!ok) {
-        while (c->n_allocs > mark) fox_gpu_free(c->gpu, c->allocs[--c->n_allocs]);
-        c->no_batch = 1;
-        return 0;
+    while (cap < n) cap *= 4;
+    batch_free(c);
+    for (; cap >= 64; cap /= 4) {
+        size_t bytes = 0;
+        memset(&b, 0, sizeof(b));
+        for (i = 0; i < 8; i++) bytes += (cap * part[i].row * 4 + 255) & ~(size_t)255;
+        if (fox_gpu_malloc(c->gpu, bytes, &b.block) != FOX_GPU_OK) continue;
+        bytes = 0;
+        for (i = 0; i < 8; i++) {
+            *(void **)part[i].p = (char *)b.block + bytes;
+            bytes += (cap * part[i].row * 4 + 255) & ~(size_t)255;
+        }
+        b.cap = cap;
+        c->B = b;
+        return 1;
     }
-    c->B = b;
-    return 1;
+    c->no_batch = 1;
+    return 0;
 }
 
 /* tokens [done, done + M) as one batched pass; the logits wanted (all: every
@@ -653,7 +676,8 @@ static fox_status eval_chunks(fox_context *c, const uint32_t *tokens, size_t n, 
     while (done < good) {
         size_t left = good - done, chunk = left < cap ? left : cap;
         int last;
-        if (left > FOX_GPU_MAX_TOKENS && c->cfg.n_batch > FOX_GPU_MAX_TOKENS && batch_ready(c)) {
+        if (left > FOX_GPU_MAX_TOKENS && c->cfg.n_batch > FOX_GPU_MAX_TOKENS &&
+            batch_ready(c, left < FOX_GPU_BATCH_TOKENS ? left : FOX_GPU_BATCH_TOKENS)) {
             /* passes of about one size, whole groups of 64 tokens */
             const size_t np = (left + c->B.cap - 1) / c->B.cap;
             chunk = ((left + np - 1) / np + 63) & ~(size_t)63;

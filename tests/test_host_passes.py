@@ -30,3 +30,43 @@ def test_eval_all_leaves_the_logits_of_eval(model, n):
     assert st == 0 and np.array_equal(got, model.want(ids))
     assert np.array_equal(model.row(p), model.want([9])[0])
     model.lib.fox_context_destroy(c)
+
+
+def test_a_short_prompt_takes_a_short_prompts_memory(model):
+    """Buffers of batched passes come in one allocation sized for the prompt,
+    grow with longer ones, are kept for shorter ones and go with the context."""
+    d, wide, q, kv, ff = 512, 512, 512, 512, 768
+    before = model.get("live")
+    c = model.context(2048, 32)
+    base = model.get("live")
+    model.set("mallocs", 0)
+    st, p = model.eval(c, np.arange(9))
+    assert st == 0 and np.array_equal(model.row(p), model.want([8])[0])
+    assert model.get("mallocs") == 1 and model.get("batches") == 2      # (two layers)
+    assert model.get("live") - base <= 64 * 4 * (d + wide + q + 2 * kv + ff + 2) + 8 * 256
+    ids = np.arange(300)
+    st, p = model.eval(c, ids)
+    assert st == 0 and np.array_equal(model.row(p), model.want(ids)[-1])
+    assert model.get("mallocs") == 2 and model.get("max_batch") == 300
+    st, _ = model.eval(c, np.arange(20))
+    assert st == 0 and model.get("mallocs") == 2
+    st, _ = model.eval(c, np.arange(600) % 500)
+    assert st == 0 and model.get("mallocs") == 2
+    model.lib.fox_context_destroy(c)
+    assert model.get("live") == before
+
+
+def test_passes_of_what_memory_there_is(model):
+    """Where the buffers of the whole prompt cannot be had: passes of 256, of
+    64, and of eight tokens, with the same logits."""
+    ids = np.arange(500)
+    per = 4 * (512 * 5 + 768 + 2)
+    for limit, largest in ((0, 500), (300 * per, 256), (100 * per, 64), (10 * per, 0)):
+        c = model.context(512, 32)
+        model.set("max_batch", 0)
+        model.set("fail_above", limit)
+        st, p = model.eval(c, ids)
+        assert st == 0 and np.array_equal(model.row(p), model.want(ids)[-1])
+        assert model.get("max_batch") == largest
+        model.set("fail_above", 0)
+        model.lib.fox_context_destroy(c)
