@@ -254,11 +254,13 @@ void       fox_model_close(fox_model *m);
 const fox_model_info *fox_model_get_info(const fox_model *m);
 fox_weights          *fox_model_weights(fox_model *m);
 
-/* include/fox/fox.h:433-451 */
+/* include/fox/fox.h:433-451.  n_batch bounds the tokens of one pass, and with
+ * them a pass's memory, at up to 1024; 0 and FOX_BATCH_DEFAULT (the reference's
+ * default) leave the choice to the library.  Results do not depend on it. */
+#define FOX_BATCH_DEFAULT 32
 typedef struct {
     uint32_t n_ctx;
-    uint32_t n_batch;     /* up to 8: tokens per pass; more: passes of up to 1024
-                             (results do not depend on it) */
+    uint32_t n_batch;
     int      n_threads;   /* kept for the ABI; the GPU path ignores it */
 } fox_context_config;
 

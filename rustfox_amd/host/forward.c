@@ -13,8 +13,8 @@
  * (fox_gpu.h) per layer; the RoPE tables are built on the host in double exactly as
  * src/forward.c:104-118 and uploaded.  fox_eval cuts its input into passes:
  * of at most FOX_GPU_MAX_TOKENS tokens (the decode kernels), or, where
- * n_batch is larger than that and as many tokens are left, of up to
- * FOX_GPU_BATCH_TOKENS (the batched kernels; a 1024-token prompt of the
+ * n_batch is larger than that and as many tokens are left, of up to n_batch
+ * (by default FOX_GPU_BATCH_TOKENS; the batched kernels; a 1024-token prompt of the
  * 4B-class layers in passes of 8 read the weights 128 times).  The result is
  * that of the reference's n_batch chunks because a token depends only on the
  * cache rows before it (batched == stepped, tests/test_forward.c:258-272).
@@ -67,6 +67,7 @@ struct fox_context {
      * (cap 0 before, and where the memory is not there: passes of
      * FOX_GPU_MAX_TOKENS then) */
     pass_buffers B;
+    size_t pass_max;               /* most tokens of a pass (n_batch) */
     float *blogits;                /* HEAD_ROWS rows, at the first batched fox_eval_all */
     int no_batch;
     fox_gpu_graph *greedy;
@@ -115,7 +116,7 @@ void fox_context_config_default(fox_context_config *cfg, const fox_model *m)
     if (!cfg) return;
     memset(cfg, 0, sizeof(*cfg));
     cfg->n_ctx = m ? m->info.n_ctx_train : 2048;
-    cfg->n_batch = 32;
+    cfg->n_batch = FOX_BATCH_DEFAULT;
     cfg->n_threads = 0;
     if (cfg->n_ctx == 0) cfg->n_ctx = 2048;
 }
@@ -156,7 +157,7 @@ fox_status fox_context_create(fox_model *m, const fox_context_config *cfg, fox_c
     fox_context_config k;
     const fox_model_info *mi;
     fox_status st;
-    size_t nb, half, p, i;
+    size_t nb, half, p, i, pass_max;
     float *tc, *ts;
     uint32_t l, zero = 0;
 
@@ -170,7 +171,10 @@ fox_status fox_context_create(fox_model *m, const fox_context_config *cfg, fox_c
     else fox_context_config_default(&k, m);
     if (k.n_ctx == 0) k.n_ctx = m->info.n_ctx_train;
     if (k.n_ctx == 0) k.n_ctx = 2048;
-    if (k.n_batch == 0) k.n_batch = 32;
+    if (k.n_batch == 0) k.n_batch = FOX_BATCH_DEFAULT;
+    pass_max = k.n_batch == FOX_BATCH_DEFAULT || k.n_batch > FOX_GPU_BATCH_TOKENS
+                   ? FOX_GPU_BATCH_TOKENS : k.n_batch;
+    if (pass_max > k.n_ctx) pass_max = k.n_ctx;
     if (k.n_batch > k.n_ctx) k.n_batch = k.n_ctx;
     mi = &m->info;
 
@@ -178,6 +182,7 @@ fox_status fox_context_create(fox_model *m, const fox_context_config *cfg, fox_c
     if (!c) return fox_fail(FOX_ERR_NOMEM, "context: handle");
     c->m = m;
     c->cfg = k;
+    c->pass_max = pass_max;
     c->gpu = m->weights->gpu;
     c->d = mi->n_embd;
     c->hd = mi->head_dim;
@@ -584,12 +589,13 @@ static int batch_ready(fox_context *c, size_t n)
         { &b.x, c->d }, { &b.xb, c->wide }, { &b.q, c->nq }, { &b.k, c->nkv }, { &b.v, c->nkv },
         { &b.hb, c->ff }, { &b.tok, 1 }, { &b.pos, 1 }
     };
-    size_t cap = 64, i;
+    size_t step = 64, i;
     if (c->B.cap >= n) return 1;
     if (c->no_batch) return 0;
-    while (cap < n) cap *= 4;
+    while (step < n) step *= 4;
     batch_free(c);
-    for (; cap >= 64; cap /= 4) {
+    for (; step >= 64; step /= 4) {
+        const size_t cap = step < c->pass_max ? step : c->pass_max;
         size_t bytes = 0;
         memset(&b, 0, sizeof(b));
         for (i = 0; i < 8; i++) bytes += (cap * part[i].row * 4 + 255) & ~(size_t)255;
@@ -656,9 +662,9 @@ static fox_status check_chunk(const fox_context *c, const uint32_t *tokens, size
 /* all == NULL: the last token's logits into c->logits, else every token's
  * into all.  The input is checked in chunks of at most n_batch (and
  * FOX_GPU_MAX_TOKENS): the chunks before a bad one are evaluated, then its
- * error is returned.  The good tokens run in batched passes where n_batch
- * allows more than FOX_GPU_MAX_TOKENS and more than that are left, in such
- * chunks otherwise. */
+ * error is returned.  The good tokens run in batched passes of at most pass_max
+ * where that and what is left are more than FOX_GPU_MAX_TOKENS, in such chunks
+ * otherwise. */
 static fox_status eval_chunks(fox_context *c, const uint32_t *tokens, size_t n, float *all)
 {
     size_t done = 0, good = 0, cap = c->cfg.n_batch;
@@ -676,12 +682,13 @@ static fox_status eval_chunks(fox_context *c, const uint32_t *tokens, size_t n, 
     while (done < good) {
         size_t left = good - done, chunk = left < cap ? left : cap;
         int last;
-        if (left > FOX_GPU_MAX_TOKENS && c->cfg.n_batch > FOX_GPU_MAX_TOKENS &&
-            batch_ready(c, left < FOX_GPU_BATCH_TOKENS ? left : FOX_GPU_BATCH_TOKENS)) {
+        if (left > FOX_GPU_MAX_TOKENS && c->pass_max > FOX_GPU_MAX_TOKENS &&
+            batch_ready(c, left < c->pass_max ? left : c->pass_max)) {
             /* passes of about one size, whole groups of 64 tokens */
-            const size_t np = (left + c->B.cap - 1) / c->B.cap;
+            const size_t most = c->B.cap < c->pass_max ? c->B.cap : c->pass_max;
+            const size_t np = (left + most - 1) / most;
             chunk = ((left + np - 1) / np + 63) & ~(size_t)63;
-            if (chunk > c->B.cap) chunk = c->B.cap;
+            if (chunk > most) chunk = most;
             if (chunk > left) chunk = left;
         }
         last = done + chunk == n;

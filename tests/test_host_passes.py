@@ -70,3 +70,20 @@ def test_passes_of_what_memory_there_is(model):
         assert model.get("max_batch") == largest
         model.set("fail_above", 0)
         model.lib.fox_context_destroy(c)
+
+
+@pytest.mark.parametrize("n_batch,largest", [(3, 0), (8, 0), (9, 9), (16, 16), (200, 192), (0, 500),
+                                             (32, 500), (5000, 500)])
+def test_n_batch_bounds_a_pass(model, n_batch, largest):
+    """A caller's n_batch bounds the tokens of a pass and its memory (three even
+    passes of whole groups of 64 where 200 are allowed); 0 and the default
+    leave them to the library."""
+    ids = np.arange(500)
+    c = model.context(512, n_batch)
+    base = model.get("live")
+    st, p = model.eval(c, ids)
+    assert st == 0 and np.array_equal(model.row(p), model.want(ids)[-1])
+    assert model.get("max_batch") == largest
+    if 8 < n_batch < 32:
+        assert model.get("live") - base <= n_batch * 4 * (512 * 5 + 768 + 2) + 8 * 256
+    model.lib.fox_context_destroy(c)
