@@ -345,7 +345,8 @@ __global__ __launch_bounds__(256) void batt_av(const float *__restrict__ att, si
     }
 }
 
-// scores of one run of tokens at most this many bytes
+// scores of one run of tokens at most this many bytes, or those of 64 tokens
+// where these are more (64 heads over 32768 positions: 520 MB)
 #define BATT_BYTES ((size_t)256 << 20)
 
 extern "C" fox_gpu_status fox_gpu_batch_attention(fox_gpu_ctx *ctx, float *out, size_t out_stride,

@@ -693,9 +693,17 @@ static fox_status eval_chunks(fox_context *c, const uint32_t *tokens, size_t n, 
         }
         last = done + chunk == n;
         if (chunk > FOX_GPU_MAX_TOKENS) {
-            if ((st = batch_eval(c, tokens + done, chunk, last, all ? all + done * c->vocab : NULL)) !=
-                FOX_OK)
-                return st;
+            st = batch_eval(c, tokens + done, chunk, last, all ? all + done * c->vocab : NULL);
+            if (st == FOX_ERR_NOMEM && fox_gpu_sync(c->gpu) == FOX_GPU_OK) {
+                /* a workspace or the logits rows could not be had: the same
+                 * tokens again in passes of the decode kernels (they write
+                 * the same cache rows; what the pass queued has ended, so
+                 * nothing reads a layer's slot that is loaded again) */
+                batch_free(c);
+                c->no_batch = 1;
+                continue;
+            }
+            if (st != FOX_OK) return st;
         } else {
             uint32_t in[FOX_GPU_MAX_TOKENS + 1] = { 0 };
             memcpy(in, tokens + done, chunk * 4);

@@ -87,3 +87,37 @@ def test_n_batch_bounds_a_pass(model, n_batch, largest):
     if 8 < n_batch < 32:
         assert model.get("live") - base <= n_batch * 4 * (512 * 5 + 768 + 2) + 8 * 256
     model.lib.fox_context_destroy(c)
+
+
+def test_a_pass_without_memory_runs_in_passes_of_eight(model):
+    """Batched attention's workspace refused, in the first and in a later pass:
+    the same logits through the decode kernels, and no further attempt."""
+    for first in (20, 64):
+        c = model.context(2048, 64)
+        ids = np.arange(first + 40)
+        if first == 64:
+            assert model.eval(c, ids[:64])[0] == 0
+        model.set("max_batch", 0)
+        model.set("eights", 0)
+        model.fail_attention(1)
+        n = 64 if first == 64 else 0
+        st, p = model.eval(c, ids[n:])
+        assert st == 0 and np.array_equal(model.row(p), model.want(ids)[-1])
+        assert model.lib.fox_context_position(c) == len(ids)
+        assert model.get("eights") == 2 * -(-(len(ids) - n) // 8)       # (two layers)
+        model.set("batches", 0)
+        st, p = model.eval(c, ids)
+        assert st == 0 and model.get("batches") == 0
+        model.lib.fox_context_destroy(c)
+
+
+def test_logits_rows_without_memory(model):
+    """fox_eval_all's block of logits rows refused: every row all the same."""
+    c = model.context(256, 32)
+    assert model.eval(c, np.arange(100))[0] == 0                         # (the pass's buffers)
+    model.set("fail_above", 64 * 600 * 4 - 1)
+    ids = np.arange(100) + 3
+    st, got = model.eval_all(c, ids)
+    assert st == 0 and np.array_equal(got, model.want(ids))
+    assert model.lib.fox_context_position(c) == 200
+    model.lib.fox_context_destroy(c)
