@@ -499,9 +499,31 @@ static fox_status batch_add(fox_context *c, const fox_gpu_tensor *w, const float
     return FOX_OK;
 }
 
+/* Attention of a batched pass of M tokens in calls of FOX_GPU_MAX_TOKENS: in
+ * split mode always, in exact mode where they are few for the positions they
+ * read.  The batched kernels run a token's sums one add at a time in one lane,
+ * 48 ns a position and a little more with more heads, whatever M (up to about
+ * 64); a call of the decode kernels spreads them over a workgroup and takes
+ * 7 ns a position and 1.1 more per 1024 query and per 1024 key columns (4
+ * more above 128 dimensions), beside 14 us of launches.  Measured per layer,
+ * batched / in calls of eight, us: 32 heads over 8 of 128: 9 tokens at 256
+ * positions 29 / 29, at 1024 69 / 45, at 8192 433 / 171; 24 tokens at 1024
+ * 69 / 87, at 8192 431 / 340; 40 at 8192 474 / 568; 8 heads over 8 of 64: 40
+ * at 8192 413 / 362, 64 there 418 / 581; 80 over 16 of 128: 16 at 4096 253 /
+ * 199, 24 there 256 / 300. */
+static int attention_in_eights(const fox_context *c, size_t M)
+{
+    const double p = (double)(c->pos + M), calls = (double)((M + FOX_GPU_MAX_TOKENS - 1) / FOX_GPU_MAX_TOKENS);
+    const double nq = (double)c->nq / 1024, nkv = (double)c->nkv / 1024;
+    if (c->attn_mode != FOX_GPU_ATTN_EXACT) return 1;
+    return calls * (14e3 + p * (6.5 + 1.1 * (nq + nkv) + (c->hd > 128 ? 4 : 0))) <
+           17e3 + p * (48 + 1.1 * nq);
+}
+
 /* forward_pass for M > FOX_GPU_MAX_TOKENS tokens in B.tok at position
- * B.pos[0]; the residual stream of every token ends in B.x */
-static fox_status batch_pass(fox_context *c, size_t M)
+ * B.pos[0] (eights: attention in calls of FOX_GPU_MAX_TOKENS, at B.pos[0 ..]);
+ * the residual stream of every token ends in B.x */
+static fox_status batch_pass(fox_context *c, size_t M, int eights)
 {
     const fox_model_info *mi = &c->m->info;
     pass_buffers *B = &c->B;
@@ -527,7 +549,7 @@ static fox_status batch_pass(fox_context *c, size_t M)
         GPU(fox_gpu_batch_rope_store(c->gpu, B->q, c->nq, B->k, c->nkv, B->v, c->nkv, mi->n_head,
                                      mi->n_head_kv, c->hd, M, c->rc, c->rs, B->pos, c->cfg.n_ctx,
                                      kc, vc), "forward: rope");
-        if (c->attn_mode == FOX_GPU_ATTN_EXACT) {
+        if (!eights) {
             GPU(fox_gpu_batch_attention(c->gpu, B->xb, c->wide, B->q, c->nq, kc, vc, mi->n_head,
                                         mi->n_head_kv, c->hd, M, B->pos, c->cfg.n_ctx),
                 "forward: attention");
@@ -619,15 +641,17 @@ static fox_status batch_eval(fox_context *c, const uint32_t *tokens, size_t M, i
 {
     uint32_t pos[FOX_GPU_BATCH_TOKENS / FOX_GPU_MAX_TOKENS + 1];
     const size_t np = (M + FOX_GPU_MAX_TOKENS - 1) / FOX_GPU_MAX_TOKENS;
+    const int eights = attention_in_eights(c, M);
+    const size_t stored = eights ? np : 1;
     size_t i, r;
     fox_status st;
     for (i = 0; i < np; i++) pos[i] = c->pos + (uint32_t)(i * FOX_GPU_MAX_TOKENS);
     GPU(fox_gpu_memcpy_h2d(c->gpu, c->B.tok, tokens, M * 4), "eval: tokens");
-    if (c->attn_mode == FOX_GPU_ATTN_EXACT)
-        GPU(fox_gpu_store_u32(c->gpu, c->B.pos, pos, 1), "eval: position");
+    if (stored <= 16)
+        GPU(fox_gpu_store_u32(c->gpu, c->B.pos, pos, stored), "eval: position");
     else
-        GPU(fox_gpu_memcpy_h2d(c->gpu, c->B.pos, pos, np * 4), "eval: position");
-    if ((st = batch_pass(c, M)) != FOX_OK) return st;
+        GPU(fox_gpu_memcpy_h2d(c->gpu, c->B.pos, pos, stored * 4), "eval: position");
+    if ((st = batch_pass(c, M, eights)) != FOX_OK) return st;
     if (!all) return last ? head(c, c->B.x + (M - 1) * c->d, c->B.xb, 1, c->dlogits) : FOX_OK;
     if (!c->blogits &&
         (st = dalloc(c, HEAD_ROWS * c->vocab * 4, (void **)&c->blogits)) != FOX_OK)

@@ -255,3 +255,27 @@ def test_a_refused_allocation_fails_no_later_call(gpu):
     assert e.value.status == 3
     gpu.batch_gemv([w], dx, 9, [out])
     assert np.isfinite(out.numpy()).all()
+
+
+def test_few_tokens_on_a_long_cache_equal_passes_of_eight(tmp_path):
+    """Batched passes whose attention runs in calls of eight tokens (few tokens
+    on a long cache), and one on the same cache that is long enough not to."""
+    s = synth.spec("8b", n_layer=2, n_vocab=512, n_embd=512, n_ff=768, n_head=8, n_head_kv=2, head_dim=64,
+                   n_ctx=1600)
+    path = str(tmp_path / "m.gguf")
+    synth.write_gguf(path, s)
+    rng = np.random.default_rng(7)
+    with rf.Model(path) as m:
+        a, b = m.context(1600), m.context(1600, n_batch=8)
+        for l in range(2):
+            k, v = (rng.standard_normal((1400, 128)).astype(np.float32) for _ in range(2))
+            a.set_kv(l, 0, k, v)
+            b.set_kv(l, 0, k, v)
+        for pos, n in ((1400, 9), (1391, 16), (1203, 23), (1000, 100)):
+            ids = synth.prompt_ids(n, s.n_vocab)
+            for c in (a, b):
+                c.set_position(pos)
+            x, y = a.eval_all(ids), b.eval_all(ids)
+            assert np.array_equal(bits(x), bits(y)), (pos, n)
+        a.close()
+        b.close()

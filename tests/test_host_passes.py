@@ -121,3 +121,20 @@ def test_logits_rows_without_memory(model):
     assert st == 0 and np.array_equal(got, model.want(ids))
     assert model.lib.fox_context_position(c) == 200
     model.lib.fox_context_destroy(c)
+
+
+def test_few_tokens_on_a_long_cache_attend_in_eights(model):
+    """The batched attention kernels run a token's sums in one lane: few tokens
+    on a long cache take the decode kernels' attention inside a batched pass."""
+    c = model.context(32768, 32)
+    for pos, n, eights in ((0, 9, 0), (0, 300, 0), (200, 12, 0), (1024, 9, 2), (8192, 24, 3),
+                           (8192, 64, 0), (30000, 32, 4), (30000, 300, 0)):
+        assert model.lib.fox_context_set_position(c, pos) == 0
+        model.set("small_attn", 0)
+        model.set("batches", 0)
+        ids = np.arange(n)
+        st, p = model.eval(c, ids)
+        assert st == 0 and np.array_equal(model.row(p), model.want(ids)[-1])
+        assert model.get("small_attn") == 2 * eights, (pos, n)          # (two layers)
+        assert model.get("batches") == 2
+    model.lib.fox_context_destroy(c)
