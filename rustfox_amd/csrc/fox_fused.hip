@@ -1694,24 +1694,35 @@ static fox_gpu_status fused_go(fox_gpu_ctx *ctx, const FusedArgs &a, int grid, u
     }
 }
 
-// (the K-quant kernels take f32 input and write outputs: int8 input with
-// per-block scales and the block-sum requests take the unfused path)
 // Ternary products of several tokens that batch_gemm (fox_batch.hip) runs
 // faster: where the operand and the terms leave room for one workgroup per
-// compute unit only (above 80 KB) and that one would take several rounds of
-// items.  (8 tokens, us here / there: gate/up 2 x 21504 x 5376 30.2 / 24.4,
-// 24000 x 8192 25.6 / 19.7; two workgroups per compute unit, 24000 x 5376 15.5 /
-// 15.9; one round, 2560 x 9728 9.5 / 10.5.)  Wider rows than five input
-// dwords per thread stay (19968 x 20000, 4 tokens: 34.6 / 37.0), and so does a
-// capped grid.
+// compute unit only (above 80 KB) and that one walks many row tiles, as rounds
+// of n_cu tiles.  A round costs the fused kernel 3 us (two slabs: 4),
+// batch_gemm 0.8 (1.6) after a start of 14 to 27 us (its preparation launch,
+// and the whole of K in each wave), so the line is a number of rounds: four,
+// six for one slab and more than 32 blocks, and three for two slabs where a
+// term row is a multiple of 32 words, which puts the fused kernel's rows on
+// one LDS bank.  (8 tokens, cold weights, us here / there.  One slab: K 8192,
+// 512 row tiles 12.4 / 15.4, 768 16.1 / 16.2, 800 19.0 / 16.3, 2048 31.1 /
+// 20.3; K 10240, 800 18.0 / 19.0, 1344 23.8 / 22.5.  Gate/up, K 5376: 512
+// 13.5 / 17.5, 768 18.1 / 18.6, 1344 30.1 / 25.3; K 8192: 512 21.6 / 22.7, 560
+// 27.7 / 23.2.  Two workgroups per compute unit, 24000 x 5376: 15.5 / 15.9.)
+// Wider rows than five input dwords per thread stay (19968 x 20000, 4 tokens:
+// 34.6 / 37.0), and so does a capped grid.
 static bool batch_better(const fox_gpu_ctx *ctx, int fmt, size_t K, size_t M, int nslab, size_t n_work)
 {
-    return fmt == FMT_TQ2 && M > 2 && ctx->max_wg == 0 && n_work >= 2 * (size_t)ctx->n_cu &&
-           K <= 5 * 4 * FWG && fused_lds(fmt, (int)K, (int)M, nslab).total > 80 * 1024;
+    if (fmt != FMT_TQ2 || M <= 2 || ctx->max_wg != 0 || K > 5 * 4 * FWG ||
+        fused_lds(fmt, (int)K, (int)M, nslab).total <= 80 * 1024)
+        return false;
+    const size_t rounds = (n_work + ctx->n_cu - 1) / ctx->n_cu;
+    if (nslab == 1) return rounds >= (K > 8192 ? 6 : 4);
+    return rounds >= (fused_ntp(fmt, (int)(K / 256)) % 32 == 0 ? 3 : 4);
 }
 
 // (fixed: the caller's scratch for fused_prep's output, or null for the
-// context's workspace)
+// context's workspace; the K-quant kernels take f32 input and write outputs:
+// int8 input with per-block scales and the block-sum requests take the
+// unfused path)
 template <int IN, int EPI>
 static fox_gpu_status fused_dispatch(fox_gpu_ctx *ctx, int fmt, const FusedArgs &a, int grid,
                                      uint8_t *fixed = nullptr)

@@ -227,6 +227,33 @@ def test_weights_past_32_bit_offsets(gpu):
         assert np.array_equal(bits(got[t]), bits(o.numpy())), f"token {t}"
 
 
+@pytest.mark.parametrize("kind,K,tiles,M", [
+    ("gemv", 8192, 768, 7), ("gemv", 8192, 769, 7), ("gemv", 9216, 1280, 6), ("gemv", 9216, 1281, 6),
+    ("gate_up", 5376, 768, 8), ("gate_up", 5376, 769, 8), ("gate_up", 7936, 512, 5),
+    ("gate_up", 7936, 513, 5),
+])
+def test_wide_ternary_products_on_either_side_of_the_rule(gpu, kind, K, tiles, M):
+    """Ternary products just below and above the row tiles from which they leave
+    the one-launch kernel: as with that kernel's grid capped (a cap that binds
+    nothing, but keeps it), which other tests compare with the oracle."""
+    rng = np.random.default_rng(K + tiles)
+    t, N = TYPES["TQ2_0"], 16 * tiles - 5
+    rows = weights(rng, t, 1 << 10, K).reshape(1 << 10, -1)
+    ws = [gpu.tensor(t, K, N, rows[rng.integers(0, 1 << 10, N)]) for _ in range(2 if kind == "gate_up" else 1)]
+    x, nw = gpu.array(rng.standard_normal((M, K)).astype(np.float32)), gpu.array(np.ones(K, np.float32))
+    got = []
+    for cap in (0, 1 << 20):
+        gpu.set_max_workgroups(cap)
+        o = gpu.empty(M * N, np.float32)
+        if kind == "gemv":
+            gpu.gemv(ws[0], x, M, o)
+        else:
+            gpu.gate_up_silu(ws[0], ws[1], x, M, nw, EPS, o)
+        got.append(bits(o.numpy()))
+    gpu.set_max_workgroups(0)
+    assert np.array_equal(got[0], got[1])
+
+
 def test_streamed_prompt_equals_resident(tmp_path):
     """A batched prompt over layers streamed through slots: the resident
     model's logits."""
