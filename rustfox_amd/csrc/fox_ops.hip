@@ -1478,7 +1478,7 @@ __global__ __launch_bounds__(256) void attn_avm(const float *__restrict__ att, s
 // up to two workgroups per compute unit, against attn_avm's 12 per round.
 // (27B-class heads, 8 tokens at 8200 positions, two rounds: 77.8 -> 61.3 us;
 // 80 heads over 16, whose five heads attn_avm pads to eight, 8 tokens at 6000
-// positions: attention 353 -> 126 us.  One round: 48 rows x 3 tokens at 7000
+// positions: attention 354 -> 134 us.  One round: 48 rows x 3 tokens at 7000
 // positions 35.8 there, 57.9 here.)
 template <int TPW>
 __global__ __launch_bounds__(128) void attn_avt(const float *__restrict__ att, size_t att_stride,
@@ -1745,13 +1745,16 @@ extern "C" fox_gpu_status fox_gpu_attention(fox_gpu_ctx *ctx, float *out, size_t
         // 32-bit byte offsets)
         const bool near_rows = 8 * n_head * att_stride * sizeof(float) <= (size_t)1 << 32;
         if (avm_wg > (size_t)ctx->n_cu && M > 1 && near_rows) {
-            // (eight tokens to a workgroup from five on, so that they share V;
-            // fewer leave a wave more columns)
-            const int tpw = M > 4 ? 4 : M > 2 ? 2 : 1, iM = (int)M;
+            // eight tokens to a workgroup from five on, so that they share V.
+            // Two tokens leave its second wave without sums, and yet a wave
+            // per token of 64 columns is slower, whose blocks are half as
+            // long: 40 heads over 8 of 128, positions 2000 40 us against 37
+            // here, 30000 403 / 337; 64 over 16 of 128 at 30000 417 / 351
+            // (attn_avm 390); at 30 positions 80 over 16 14.9 / 15.9
+            const int tpw = M > 4 ? 4 : 2, iM = (int)M;
             const size_t nu = n_kv_groups(n_head_kv, head_dim, 64 / tpw);
             const size_t nwg = (nu + 7) / 8 * 8 * gqa * ((M + 2 * tpw - 1) / (2 * tpw));
-            const void *av = tpw == 4 ? (const void *)attn_avt<4> : tpw == 2 ? (const void *)attn_avt<2>
-                                                                             : (const void *)attn_avt<1>;
+            const void *av = tpw == 4 ? (const void *)attn_avt<4> : (const void *)attn_avt<2>;
             const int in_head = (int)n_head;
             void *args[] = {(void *)&att, (void *)&att_stride, (void *)&v_cache, (void *)&in_head,
                             (void *)&ikv, (void *)&ihd, (void *)&pos, (void *)&ictx, (void *)&out,
