@@ -916,10 +916,11 @@ __global__ __launch_bounds__(KS * 64, FMT == FMT_Q4K ? 4 : 3) void few_gemm(Batc
 
 // batch_gemm's waves each walk the whole of K, so a matrix of few rows leaves
 // the chip part empty and every block waits for its loads (Q6_K 4096 x 14336,
-// 16 tokens: 59 us, here 26; Q4_K 4096 x 4096 19, here 10.5).  Here a workgroup is one row tile and one token tile, its
-// KS waves take units of U blocks in turn, operands straight from L2 to
-// registers, and pass the float terms through LDS to 256 lanes (token, row)
-// that add them in block order, as in few_gemm.
+// 16 tokens: 59 us, here 26; Q4_K 4096 x 4096 19, here 10.5).  Here a
+// workgroup is one row tile and one token tile, its KS waves take units of U
+// blocks in turn, operands straight from L2 to registers, and pass the float
+// terms through LDS to 256 lanes (token, row) that add them in block order, as
+// in few_gemm.
 template <int FMT>
 struct SplitTerms;                      // one lane's terms of a unit, per token k
 template <>
@@ -1127,7 +1128,8 @@ static fox_gpu_status batch_carve(fox_gpu_ctx *ctx, int fmt, size_t K, size_t M,
                                   BatchWs *w)
 {
     // (few_gemm's operand has room for eight tokens whatever M is)
-    const size_t nq = M <= FOX_GPU_MAX_TOKENS && fmt != FMT_TQ2 ? FOX_GPU_MAX_TOKENS * K : (M + 15) / 16 * 16 * K;
+    const size_t nq = M <= FOX_GPU_MAX_TOKENS && fmt != FMT_TQ2 ? FOX_GPU_MAX_TOKENS * K
+                                                                : (M + 15) / 16 * 16 * K;
     const size_t na = up256((M + 15) / 16 * (K / 256) * (size_t)aux_quads(fmt) * 16);
     const size_t ns = up256(M * 4);
     if (!fixed) {
@@ -1150,10 +1152,13 @@ static const void *prep_kernel(int r)
          : r <= 12 ? (const void *)batch_prep<FMT, NORM, 12> : (const void *)batch_prep<FMT, NORM, 16>;
 }
 
+// (the K-quants without a norm: blocks apart on grid y, one dword a thread)
 template <int FMT>
 static const void *prep_fmt(bool norm, int r)
 {
-    return norm ? prep_kernel<FMT, true>(r) : prep_kernel<FMT, false>(r);
+    if (norm) return prep_kernel<FMT, true>(r);
+    if constexpr (FMT == FMT_TQ2) return prep_kernel<FMT, false>(r);
+    else return (const void *)batch_prep<FMT, false, 1>;
 }
 
 template <int FMT, int R, int EPI>
@@ -1233,28 +1238,27 @@ static fox_gpu_status batch_run(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor
 {
     const int fmt = fmt_of(ws[0]->type);
     const size_t K = (size_t)ws[0]->ne0;
-    // (Q6_K gate/up pairs: two such tiles per wave do not fit its registers)
-    if (fmt < 0 || (fmt == FMT_Q6K && epi == BE_SILU && M > FOX_GPU_MAX_TOKENS &&
-                    !split_better(fmt, (int)ws[0]->n_tiles, (int)((M + 15) / 16), ctx->n_cu)) || K == 0 || K % 256 || K > 2048 * PREP_MAX_R || x_stride % 4 ||
+    if (fmt < 0 || K == 0 || K % 256 || K > 2048 * PREP_MAX_R || x_stride % 4 ||
         ((uintptr_t)x | (uintptr_t)norm_w) % 16)
+        return FOX_GPU_ERR_UNSUPPORTED;
+    // (Q6_K gate/up pairs: two such tiles per wave do not fit its registers)
+    if (fmt == FMT_Q6K && epi == BE_SILU && M > FOX_GPU_MAX_TOKENS &&
+        !split_better(fmt, (int)ws[0]->n_tiles, (int)((M + 15) / 16), ctx->n_cu))
         return FOX_GPU_ERR_UNSUPPORTED;
     BatchWs w;
     fox_gpu_status st = batch_carve(ctx, fmt, K, M, fixed, &w);
     if (st) return st;
     {
         const int r = (int)((K / 4 + 511) / 512);
-        const void *k = fmt == FMT_TQ2 ? prep_fmt<FMT_TQ2>(norm_w != nullptr, r)
-                      : fmt == FMT_Q4K ? prep_fmt<FMT_Q4K>(norm_w != nullptr, r)
-                                       : prep_fmt<FMT_Q6K>(norm_w != nullptr, r);
+        const bool norm = norm_w != nullptr;
+        const bool blocks = fmt != FMT_TQ2 && !norm;       // (grid y: 8 blocks each)
+        const void *k = fmt == FMT_TQ2 ? prep_fmt<FMT_TQ2>(norm, r)
+                      : fmt == FMT_Q4K ? prep_fmt<FMT_Q4K>(norm, r) : prep_fmt<FMT_Q6K>(norm, r);
         int iK = (int)K, iM = (int)M, few = fmt != FMT_TQ2 && M <= FOX_GPU_MAX_TOKENS;
-        void *args[] = {(void *)&x, (void *)&norm_w, (void *)&iK, (void *)&x_stride, (void *)&eps, (void *)&iM,
-                        (void *)&few,
-                        (void *)&w.q, (void *)&w.aux, (void *)&w.scale};
-        const bool split = fmt != FMT_TQ2 && !norm_w;      // (blocks apart on grid y, R = 1)
-        if (split) k = fmt == FMT_Q4K ? (const void *)batch_prep<FMT_Q4K, false, 1>
-                                      : (const void *)batch_prep<FMT_Q6K, false, 1>;
-        hipError_t e = hipLaunchKernel(k, dim3(few ? (unsigned)M : (unsigned)((M + 63) / 64 * 64), split ? (unsigned)r : 1u),
-                                       dim3(512), args, 0, ctx->stream);
+        void *args[] = {(void *)&x, (void *)&norm_w, (void *)&iK, (void *)&x_stride, (void *)&eps,
+                        (void *)&iM, (void *)&few, (void *)&w.q, (void *)&w.aux, (void *)&w.scale};
+        const dim3 grid(few ? (unsigned)M : (unsigned)((M + 63) / 64 * 64), blocks ? (unsigned)r : 1u);
+        hipError_t e = hipLaunchKernel(k, grid, dim3(512), args, 0, ctx->stream);
         if (e != hipSuccess) return fox_hip_fail(e, "batch: prepare");
         FOX_LAUNCHED("batch: prepare");
     }
@@ -1280,13 +1284,13 @@ static fox_gpu_status batch_run(fox_gpu_ctx *ctx, size_t n, const fox_gpu_tensor
     if (fmt != FMT_TQ2 && M <= FOX_GPU_MAX_TOKENS) {
         // K-quants, up to eight tokens: a workgroup per row tile
         const int nt = epi == BE_SILU ? a.tile_start[1] : tiles;
-        const void *k = few_kernel(fmt, nt < 512, epi);
+        const bool wide = nt < 2 * ctx->n_cu;
+        const void *k = few_kernel(fmt, wide, epi);
         void *args[] = {(void *)&a};
-        const size_t lds = K / 256 * (size_t)aux_quads(fmt) * 8;
-        if (lds > 64 * 1024) return FOX_GPU_ERR_UNSUPPORTED;
+        const size_t lds = K / 256 * (size_t)aux_quads(fmt) * 8;   // (at most 36 KB)
         hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e == hipSuccess)
-            e = hipLaunchKernel(k, dim3((unsigned)nt), dim3(nt < 512 ? 512 : 256), args, lds, ctx->stream);
+            e = hipLaunchKernel(k, dim3((unsigned)nt), dim3(wide ? 512 : 256), args, lds, ctx->stream);
         if (e != hipSuccess) return fox_hip_fail(e, "batch: product");
         FOX_LAUNCHED("batch: product");
         return FOX_GPU_OK;

@@ -368,10 +368,11 @@ extern "C" fox_gpu_status fox_gpu_batch_attention(fox_gpu_ctx *ctx, float *out, 
     if (((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 || q_stride % 4)
         return fox_fail(FOX_GPU_ERR_ARG, "attention: q and the caches must be 16-byte aligned and "
                         "the q stride a multiple of 4");
+    // (the decode kernels' limit, which keep a head's weights in LDS: a context
+    // that takes a prompt here goes on there)
     if (n_ctx > 32768)
-        return fox_fail(FOX_GPU_ERR_UNSUPPORTED,
-                        "attention: exact mode keeps a head's %zu weights in LDS; at most 32768 "
-                        "positions", n_ctx);
+        return fox_fail(FOX_GPU_ERR_UNSUPPORTED, "attention: %zu positions; exact mode takes at "
+                        "most 32768", n_ctx);
     const size_t att_stride = (n_ctx + 3) & ~(size_t)3;
     const int n_tiles = (int)((n_ctx + BQ_POS - 1) / BQ_POS);
     const size_t per_tok = n_head * (att_stride + (size_t)n_tiles) * sizeof(float);
