@@ -1478,7 +1478,7 @@ __global__ __launch_bounds__(256) void attn_avm(const float *__restrict__ att, s
 // up to two workgroups per compute unit, against attn_avm's 12 per round.
 // (27B-class heads, 8 tokens at 8200 positions, two rounds: 77.8 -> 61.3 us;
 // 80 heads over 16, whose five heads attn_avm pads to eight, 8 tokens at 6000
-// positions: attention 354 -> 134 us.  One round: 48 rows x 3 tokens at 7000
+// positions: attention 354 -> 145 us.  One round: 48 rows x 3 tokens at 7000
 // positions 35.8 there, 57.9 here.)
 template <int TPW>
 __global__ __launch_bounds__(128) void attn_avt(const float *__restrict__ att, size_t att_stride,

@@ -16,10 +16,10 @@ Shapes: the single-op microbenchmark (TQ1_0/TQ2_0 14336 x 4096, M = 1 and
 2048+, gate/up 2560 -> 9728, ffn_down 9728 -> 2560 and attn_output 4096 ->
 2560 with the residual add), the 8B-class layer's Q4_K/Q6_K matrices
 (14336 x 4096, 4096 x 14336) and the 27B-class layer's TQ1_0 ffn_down
-(21504 -> 5376: the fused path for one token and for 8, where one
-workgroup per compute unit has up to 160 KB of LDS; K = 24576 is past the
-fused kernel's input registers and takes the unfused path) and its 8-token
-pass at d_model 5376.
+(21504 -> 5376: the fused path for one token; 8 tokens' operand is more than
+a workgroup's 160 KB of LDS and K = 24576 past the fused kernel's input
+registers, and both take the batched product) and its 8-token pass at d_model
+5376.
 """
 import numpy as np
 import pytest
@@ -165,9 +165,10 @@ def test_4b_qkv_rope_bit_exact(capped, oracle, M, pos, cap):
                                         ("K past the fused limit", 1024, 24576, 8)])
 def test_residual_projections_bit_exact(capped, oracle, name, N, K, M, cap):
     """out += W x (the residual add fused into the GEMV, src/forward.c:374-377,
-    393-396).  K = 24576 is more than the fused kernel's input registers hold
-    (22528) and takes the unfused path (quantiser kernel over block slices,
-    then the block kernel)."""
+    393-396).  Eight tokens of K = 21504 are more than a workgroup's LDS holds
+    and K = 24576 is more than the fused kernel's input registers hold (22528):
+    both take the batched product (one quantiser launch, then the blocks split
+    over a workgroup's waves)."""
     print(f"case {name} N={N} K={K} M={M} cap={cap}", flush=True)
     rng = np.random.default_rng([N, K, M, 13])
     w = weights(rng, 34, N, K)
@@ -218,7 +219,8 @@ def test_8b_kquant_shapes_bit_exact(capped, oracle, tname, gtype, N, K, M, cap):
     4096 -> 1024), weights from the repository's quantiser
     (src/kernels.c:571-661 int8 dots, per-256 activation scales).  One token
     takes the fused kernel (also with its grid capped to 3 workgroups, each
-    then walking hundreds of tiles), 8 tokens the unfused path."""
+    then walking hundreds of tiles), 8 tokens few_gemm (a workgroup per row
+    tile)."""
     print(f"case gemv 8b {tname} {N}x{K} M={M} cap={cap}", flush=True)
     w, x, want = case_data(oracle, gtype, N, K, M, 8)
     capped.set_max_workgroups(cap)
