@@ -64,10 +64,12 @@ def test_passes_of_what_memory_there_is(model):
     for limit, largest in ((0, 500), (300 * per, 256), (100 * per, 64), (10 * per, 0)):
         c = model.context(512, 32)
         model.set("max_batch", 0)
+        model.set("mallocs", 0)
         model.set("fail_above", limit)
         st, p = model.eval(c, ids)
         assert st == 0 and np.array_equal(model.row(p), model.want(ids)[-1])
         assert model.get("max_batch") == largest
+        assert model.get("mallocs") == (largest > 0)        # (not tried again at every pass)
         model.set("fail_above", 0)
         model.lib.fox_context_destroy(c)
 
